@@ -3,8 +3,7 @@
 // counterpart in the reference.
 //
 // All three are implicit GEMMs.  On grids whose rows hold >= 32 voxels the
-// operands are staged in LDS (the input block with its halo for the forward,
-// a row chunk's 27 shifted tiles for the weight gradient); smaller grids
+// operands are staged in LDS (the input block with its halo for the forward); smaller grids
 // read their fragments straight from global memory (the 27-fold reuse of
 // every input voxel served by L1/L2):
 //   forward      M = voxels, N = cout, K = taps*cin      (A: 8 channels of one
@@ -13,9 +12,9 @@
 //                staged in LDS, 16 channels at a time (k_fwd_tile)
 //   bwd-data     the forward on the flipped, transposed weights
 //   bwd-weight   M = cout, N = cin, K = voxels (split over workgroups,
-//                FP32 partials, fixed-order reduction): all 27 taps of a
-//                chunk from one LDS staging when rows hold >= 32 voxels
-//                (k_bwd_w27), else one tap per workgroup (k_bwd_w)
+//                FP32 partials, fixed-order reduction): all 27 taps from one
+//                staging of each row (k_bwd_wy, 3^3 on rows of >= 4 voxels),
+//                else one tap per workgroup (k_bwd_w)
 // MFMA 16x16x32 bf16 operand layout: lane l holds row (A) / column (B) l%16
 // and the 8 K values of group l/16; D register r of lane l is row 4*(l/16)+r,
 // column l%16.
@@ -292,10 +291,12 @@ __global__ void __launch_bounds__(256)
     }
 }
 
-// Weight gradient of one tap for a (16*NM) x (16*NN) block of (co, ci).
+// Weight gradient of one tap for a (16*NM) x (16*NN) block of (co, ci): the
+// 1^3 kernel, and 3^3 on rows of 1 or 2 voxels.
 // grid.x = T * splits (tap fastest), grid.y = channel blocks.  Each wave
-// takes every 4th 32-voxel chunk of its split and writes its own partial:
-// part[(split*4 + wave)][tap][co][ci].
+// takes every 4th 32-voxel chunk of its split; the four waves' sums are
+// added in wave order: part[split][tap][co][ci], and part_b[split][co] (the
+// bias sums) from the middle tap's workgroups of the first ci block.
 // The GEMM's K index is the voxel, but channels are contiguous in memory:
 // each wave loads its chunk of dy (32 voxels x 16*NM channels) and of the
 // shifted input (32 voxels x 16*NN channels) with 16-byte loads and writes
@@ -305,7 +306,8 @@ __global__ void __launch_bounds__(256)
 template <int NM, int NN, int KS>
 __global__ void __launch_bounds__(256)
     k_bwd_w(const uint16_t* __restrict__ x, const uint16_t* __restrict__ dy,
-            float* __restrict__ part, Geo g, int cin, int cout, uint32_t chunks_per_split)
+            float* __restrict__ part, float* __restrict__ part_b, Geo g, int cin, int cout,
+            uint32_t chunks_per_split)
 {
     constexpr int T = KS * KS * KS;
     constexpr int CM = 16 * NM, CN = 16 * NN;       // channels of the two operands
@@ -329,6 +331,12 @@ __global__ void __launch_bounds__(256)
     for (int m = 0; m < NM; m++)
 #pragma unroll
         for (int n = 0; n < NN; n++) acc[m][n] = f32x4{0.f, 0.f, 0.f, 0.f};
+    const bool bias = part_b != nullptr && ci0 == 0 && tap == T / 2;
+    f32x4 accb[NM];
+#pragma unroll
+    for (int m = 0; m < NM; m++) accb[m] = f32x4{0.f, 0.f, 0.f, 0.f};
+    const u16x8 one8 = {0x3F80, 0x3F80, 0x3F80, 0x3F80, 0x3F80, 0x3F80, 0x3F80, 0x3F80};
+    const bf16x8 ones = __builtin_bit_cast(bf16x8, one8);
 
     // element e = lane + 64 k of a chunk: voxel quad e / (C/8) (4 consecutive
     // voxels), channel group e % (C/8) (8 channels): four 16-byte loads, then
@@ -406,6 +414,9 @@ __global__ void __launch_bounds__(256)
         for (int m = 0; m < NM; m++)
 #pragma unroll
             for (int n = 0; n < NN; n++) acc[m][n] = mfma(a[m], b[n], acc[m][n]);
+        if (bias)
+#pragma unroll
+            for (int m = 0; m < NM; m++) accb[m] = mfma(a[m], ones, accb[m]);
     };
 
     const uint32_t n_chunks = (g.V + 31u) / 32u;
@@ -430,232 +441,300 @@ __global__ void __launch_bounds__(256)
         }
     }
 
-    float* out = part + ((size_t)(split * 4u + (uint32_t)wave) * T + tap) * (size_t)cout * cin;
+    // the four waves' sums, one 16 x 16 block at a time
+    float* sum = reinterpret_cast<float*>(&lds[0][0]);
+    float* out = part + ((size_t)split * T + tap) * (size_t)cout * cin;
+    __syncthreads();
 #pragma unroll
     for (int m = 0; m < NM; m++)
 #pragma unroll
-        for (int n = 0; n < NN; n++)
+        for (int n = 0; n < NN; n++) {
 #pragma unroll
-            for (int r = 0; r < 4; r++)
-                out[(size_t)(co0 + m * 16 + 4 * grp + r) * cin + ci0 + n * 16 + r16] = acc[m][n][r];
+            for (int r = 0; r < 4; r++) sum[wave * 256 + (4 * grp + r) * 16 + r16] = acc[m][n][r];
+            __syncthreads();
+            const int t = threadIdx.x;
+            out[(size_t)(co0 + m * 16 + (t >> 4)) * cin + ci0 + n * 16 + (t & 15)] =
+                ((sum[t] + sum[256 + t]) + sum[512 + t]) + sum[768 + t];
+            __syncthreads();
+        }
+    if (bias) {
+        if (r16 == 0)
+#pragma unroll
+            for (int m = 0; m < NM; m++)
+#pragma unroll
+                for (int r = 0; r < 4; r++) sum[wave * CM + m * 16 + 4 * grp + r] = accb[m][r];
+        __syncthreads();
+        const int t = threadIdx.x;
+        if (t < CM) part_b[(size_t)split * cout + co0 + t] = ((sum[t] + sum[CM + t]) + sum[2 * CM + t]) + sum[3 * CM + t];
+    }
 }
 
-// Weight gradient of all 27 taps of a 3^3 convolution for a (16*NM) x 16
-// block of (co, ci), rows of at least 32 voxels (W >= 32).  grid.x = splits,
-// grid.y = channel blocks.  The workgroup walks 32-voxel chunks (one row
-// segment each): it stages the chunk's dy (32 voxels x 16*NM channels) and,
-// for every tap, the input the tap reads (the 9 neighbour row segments, each
-// in the 3 x shifts: 27 tiles of 16 channels x 32 voxels) transposed into
-// LDS [channel][voxel], so every MFMA fragment is one 16-byte LDS read and
-// each input element is fetched from memory once per chunk instead of once
-// per tap.  Wave w accumulates taps w, w+4, ..., w+24; one partial per split:
-// part[split][tap][co][ci].
-// With part_b, the workgroups of the first input-channel block also sum the
-// staged dy over their voxels (bias gradient): part_b[split][co].
-template <int NM>
-__global__ void __launch_bounds__(256)
-    k_bwd_w27(const uint16_t* __restrict__ x, const uint16_t* __restrict__ dy,
-              float* __restrict__ part, float* __restrict__ part_b, Geo g, int cin, int cout,
-              uint32_t chunks_per_split)
+// Weight gradient of all 27 taps of a 3^3 convolution for one 16 x 16 block
+// of (co, ci), rows of at least 4 voxels.  512 threads (8 wavefronts).
+// A wavefront takes K = 32 voxels of x at a time -- WS = min(W, 32) voxels
+// of NZ = 32 / WS consecutive z rows -- and marches along y.  Per row it
+// reads 3 fragments of x (the x shifts) and 3 of dy (the row just ahead, at
+// the three z shifts) from LDS and holds the dy fragments of the 3 x 3
+// neighbouring rows in registers, so 6 fragment reads feed 27 MFMAs: the
+// LDS would otherwise bound it (one fragment read per MFMA takes the LDS
+// twice the MFMA's time).  Both operands lie channels-last in LDS, 32 bytes
+// per voxel; ds_read_b64_tr_b16 hands each lane 4 voxels of one channel, so
+// a tap's shift is a row offset and nothing is transposed or staged twice.
+// Rows reach LDS through registers, two rows ahead of the row in use.
+// Bound: at 16 -> 16 channels the HBM reads and the MFMAs alike.
+// Measured (MI355X, 64^3, batch 8): 16 -> 16 50 us, 48 -> 16 123 us (before,
+// staging 27 shifted copies of x per row: 203 and 648 us); 16^3, 64 -> 64
+// 24 us (one tap per workgroup: 90 us).
+// Pairs of rows outside the grid are left out (a zero row would turn an
+// infinite partner into NaN).  Work: the columns (x segment, 8 NZ z rows,
+// sample) times H rows are one sequence of row steps, cut evenly into
+// `splits` runs; part[split][tap][co][ci], and from the workgroups of the
+// first ci block the bias sums part_b[split][co].
+typedef short s16x4 __attribute__((ext_vector_type(4)));
+
+__device__ __forceinline__ bf16x8 tr_frag(const uint16_t* lo, const uint16_t* hi)
 {
-    constexpr int CM = 16 * NM, CN = 16, T = 27, TW = 7;
-    constexpr int PITCH = 40;                            // halves per LDS row (32 voxels + pad)
-    constexpr int XITEMS = T * 8 * 2;                    // (tile, voxel quad, 8-channel group)
-    constexpr int DITEMS = 8 * (CM / 8);                 // (voxel quad, 8-channel group)
-    __shared__ __attribute__((aligned(16))) uint16_t lx[T * CN * PITCH];
-    __shared__ __attribute__((aligned(16))) uint16_t ld[CM * PITCH];
-    const int tid = threadIdx.x, lane = tid & 63, wave = tid >> 6;
+    typedef __attribute__((address_space(3))) s16x4 lds4;
+    const s16x4 a = __builtin_amdgcn_ds_read_tr16_b64_v4i16((lds4*)lo);
+    const s16x4 b = __builtin_amdgcn_ds_read_tr16_b64_v4i16((lds4*)hi);
+    typedef short s16x8 __attribute__((ext_vector_type(8)));
+    const s16x8 v = __builtin_shufflevector(a, b, 0, 1, 2, 3, 4, 5, 6, 7);
+    return __builtin_bit_cast(bf16x8, v);
+}
+
+template <int WS>
+__global__ void __launch_bounds__(512)
+    k_bwd_wy(const uint16_t* __restrict__ x, const uint16_t* __restrict__ dy, float* __restrict__ part,
+             float* __restrict__ part_b, Geo g, int cin, int cout, uint32_t rows, uint32_t rows_per_split,
+             uint32_t pairs)
+{
+    constexpr int NZ = 32 / WS, TZ = 8 * NZ, XV = WS + 2, T = 27;
+    constexpr int XP = TZ * XV * 2, DP = (TZ + 2) * WS * 2;   // 16-byte pieces of an x and a dy row set
+    constexpr int NJ = (XP + DP + 511) / 512;
+    constexpr int RT = 4;                                     // taps per round of the final sum
+    constexpr int BUF = (XP + DP) * 8;                        // halves per buffer
+    constexpr int SUMH = 8 * RT * 256 * 2;                    // halves of the final sum's floats
+    __shared__ __attribute__((aligned(16))) uint16_t lds[2 * BUF > SUMH ? 2 * BUF : SUMH];
+    const int tid = (int)threadIdx.x, lane = tid & 63;
+    const int wave = __builtin_amdgcn_readfirstlane(tid >> 6);
     const int r16 = lane & 15, grp = lane >> 4;
-    const int mblocks = cout / CM;
-    const int co0 = (int)(blockIdx.y % mblocks) * CM;
-    const int ci0 = (int)(blockIdx.y / mblocks) * CN;
+    // consecutive workgroups of one XCD: the channel blocks of one run (they
+    // share its lines), then the next run
+    const uint32_t id = xcd_remap(blockIdx.x, gridDim.x);
+    const uint32_t pair = id % pairs, split = id / pairs;
+    const int mblocks = cout / 16;
+    const int co0 = (int)(pair % (uint32_t)mblocks) * 16, ci0 = (int)(pair / (uint32_t)mblocks) * 16;
+    const bool bias = part_b != nullptr && ci0 == 0;
+    const int nxs = g.W / WS, nzb = (g.D + TZ - 1) / TZ;
 
-    f32x4 acc[TW][NM];
+    f32x4 acc[T], accb = f32x4{0.f, 0.f, 0.f, 0.f};
 #pragma unroll
-    for (int t = 0; t < TW; t++)
-#pragma unroll
-        for (int m = 0; m < NM; m++) acc[t][m] = f32x4{0.f, 0.f, 0.f, 0.f};
+    for (int t = 0; t < T; t++) acc[t] = f32x4{0.f, 0.f, 0.f, 0.f};
+    const s16x4 one4 = {0x3F80, 0x3F80, 0x3F80, 0x3F80};
+    const bf16x8 ones = __builtin_bit_cast(bf16x8, __builtin_shufflevector(one4, one4, 0, 1, 2, 3, 4, 5, 6, 7));
 
-    // this thread's staging items: x items tid, tid + 256 (< XITEMS), dy item tid (< DITEMS)
-    uint4 qx[2][4], qd[4];
-    auto fetch = [&](uint32_t c) {
-        const uint32_t v0 = c * 32u;
-        const int x0 = (int)(v0 & (uint32_t)(g.W - 1));
-        const int y0 = (int)((v0 >> g.lw) & (uint32_t)(g.H - 1));
-        const int z0 = (int)((v0 >> (g.lw + g.lh)) & (uint32_t)(g.D - 1));
+    // this lane's two 4-voxel groups of a fragment: voxels 4 grp + r16 / 4 and 16 more
+    const int k0 = 4 * grp + (r16 >> 2), k1 = k0 + 16, col = 4 * (r16 & 3);
+    const int xo0 = ((wave * NZ + k0 / WS) * XV + k0 % WS) * 16 + col;
+    const int xo1 = ((wave * NZ + k1 / WS) * XV + k1 % WS) * 16 + col;
+    const int do0 = XP * 8 + ((wave * NZ + k0 / WS) * WS + k0 % WS) * 16 + col;
+    const int do1 = XP * 8 + ((wave * NZ + k1 / WS) * WS + k1 % WS) * 16 + col;
+    // z of the voxel groups this lane's 8 K values belong to (K value order:
+    // voxels 4 grp .. 4 grp + 3, then the same 16 on)
+    const int zk0 = (4 * grp) / WS, zk1 = (16 + 4 * grp) / WS;
+
+    const uint32_t r1 = min(rows, (split + 1) * rows_per_split);
+    for (uint32_t r = split * rows_per_split; r < r1;) {
+        const uint32_t colm = r / (uint32_t)g.H;
+        const int ya = (int)(r % (uint32_t)g.H);
+        const int yb = min(g.H, ya + (int)(r1 - r));
+        r += (uint32_t)(yb - ya);
+        const int xs = (int)(colm % (uint32_t)nxs), zb = (int)((colm / (uint32_t)nxs) % (uint32_t)nzb);
+        const int x0 = xs * WS, z0 = zb * TZ;
+        const uint32_t smp = colm / (uint32_t)(nxs * nzb);
+
+        // this thread's pieces of a step: where from (the row y = 0) and whether inside
+        uint32_t off[NJ];
+        bool ok[NJ];
 #pragma unroll
-        for (int k = 0; k < 2; k++) {
-            const int it = tid + 256 * k;
-            const int tile = it >> 4, quad = (it >> 1) & 7, cg = it & 1;
-            int dz, dyo, dx;
-            tap_offset<3>(tile, dz, dyo, dx);
-            const bool row = it < XITEMS && (unsigned)(z0 + dz) < (unsigned)g.D &&
-                             (unsigned)(y0 + dyo) < (unsigned)g.H;
-            const int64_t base = (int64_t)v0 + (int64_t)(dz * g.H + dyo) * g.W + dx;
+        for (int j = 0; j < NJ; j++) {
+            const int p = tid + 512 * j;
+            const bool isx = p < XP;
+            const int hv = (isx ? p : p - XP) >> 1, zr = isx ? hv / XV : hv / WS;
+            const int gx = isx ? x0 - 1 + hv % XV : x0 + hv % WS, gz = isx ? z0 + zr : z0 - 1 + zr;
+            ok[j] = p < XP + DP && (unsigned)gx < (unsigned)g.W && (unsigned)gz < (unsigned)g.D;
+            const uint32_t v = ((smp * (uint32_t)g.D + (uint32_t)gz) * (uint32_t)g.H) * (uint32_t)g.W + (uint32_t)gx;
+            off[j] = v * (uint32_t)(isx ? cin : cout) + (uint32_t)((isx ? ci0 : co0) + 8 * (p & 1));
+        }
+        uint4 R[3][NJ];
+        // step s: the x rows y = s (from s = ya on) and the dy rows y = s + 1
+        auto fetch = [&](int s, uint4* q) {
 #pragma unroll
-            for (int t = 0; t < 4; t++) {
-                const int pos = 4 * quad + t;
-                const bool ok = row && (unsigned)(x0 + pos + dx) < (unsigned)g.W;
-                qx[k][t] = ok ? *reinterpret_cast<const uint4*>(x + (size_t)(base + pos) * cin + ci0 + 8 * cg)
-                              : uint4{0u, 0u, 0u, 0u};
+            for (int j = 0; j < NJ; j++) {
+                const bool isx = tid + 512 * j < XP;
+                const int yy = isx ? s : s + 1;
+                const bool in = ok[j] && s < yb && (isx ? s >= ya : (unsigned)yy < (unsigned)g.H);
+                const uint16_t* base = isx ? x : dy;
+                q[j] = in ? *reinterpret_cast<const uint4*>(base + off[j] + (uint32_t)(yy * g.W) * (uint32_t)(isx ? cin : cout))
+                          : uint4{0u, 0u, 0u, 0u};
+            }
+        };
+        auto put = [&](int buf, const uint4* q) {
+#pragma unroll
+            for (int j = 0; j < NJ; j++)
+                if (tid + 512 * j < XP + DP) *reinterpret_cast<uint4*>(lds + buf * BUF + (tid + 512 * j) * 8) = q[j];
+        };
+        const int zw = z0 + wave * NZ;                        // the wavefront's first z row
+        bf16x8 A[3][3];                                       // [y slot][dz + 1]
+        auto step = [&](auto phase, int s, int buf) {
+            constexpr int ph = decltype(phase)::value;
+            fetch(s + 3, R[ph]);
+            const uint16_t* L = lds + buf * BUF;
+            if (zw < g.D) {
+#pragma unroll
+                for (int dz = 0; dz < 3; dz++) A[ph][dz] = tr_frag(L + do0 + dz * WS * 16, L + do1 + dz * WS * 16);
+                if (s >= ya) {
+                    bf16x8 B[3];
+#pragma unroll
+                    for (int dx = 0; dx < 3; dx++) B[dx] = tr_frag(L + xo0 + dx * 16, L + xo1 + dx * 16);
+#pragma unroll
+                    for (int dz = 0; dz < 3; dz++) {          // dy row z + dz - 1
+                        if (NZ == 1 && (unsigned)(zw + dz - 1) >= (unsigned)g.D) continue;
+                        bf16x8 Bz[3];
+#pragma unroll
+                        for (int dx = 0; dx < 3; dx++) {
+                            Bz[dx] = B[dx];
+                            if (NZ > 1 && dz != 1) {
+                                // K values whose dy row lies outside the grid
+                                uint4 u = __builtin_bit_cast(uint4, B[dx]);
+                                if ((unsigned)(zw + zk0 + dz - 1) >= (unsigned)g.D) u.x = u.y = 0u;
+                                if ((unsigned)(zw + zk1 + dz - 1) >= (unsigned)g.D) u.z = u.w = 0u;
+                                Bz[dx] = __builtin_bit_cast(bf16x8, u);
+                            }
+                        }
+#pragma unroll
+                        for (int dyo = 0; dyo < 3; dyo++) {   // dy row s + dyo - 1
+                            if ((unsigned)(s + dyo - 1) >= (unsigned)g.H) continue;
+                            const bf16x8 a = A[dyo == 2 ? ph : dyo == 1 ? (ph + 2) % 3 : (ph + 1) % 3][dz];
+#pragma unroll
+                            for (int dx = 0; dx < 3; dx++) {
+                                const int tap = ((2 - dz) * 3 + (2 - dyo)) * 3 + dx;
+                                acc[tap] = mfma(a, Bz[dx], acc[tap]);
+                            }
+                            if (dz == 1 && dyo == 1 && bias) accb = mfma(a, ones, accb);
+                        }
+                    }
+                }
+            }
+            put(buf ^ 1, R[(ph + 1) % 3]);
+            __syncthreads();
+        };
+        const int s0 = ya - 2;
+        fetch(s0, R[0]);
+        fetch(s0 + 1, R[1]);
+        fetch(s0 + 2, R[2]);
+        put(0, R[0]);
+        __syncthreads();
+        int buf = 0;
+        for (int s = s0; s < yb;) {
+            step(std::integral_constant<int, 0>{}, s, buf);
+            buf ^= 1;
+            if (++s >= yb) break;
+            step(std::integral_constant<int, 1>{}, s, buf);
+            buf ^= 1;
+            if (++s >= yb) break;
+            step(std::integral_constant<int, 2>{}, s, buf);
+            buf ^= 1;
+            ++s;
+        }
+        __syncthreads();
+    }
+
+    // the 8 wavefronts' sums, RT taps at a time, in wavefront order
+    float* sum = reinterpret_cast<float*>(lds);
+    float* out = part + (size_t)split * T * cout * cin;
+#pragma unroll
+    for (int t0 = 0; t0 < T; t0 += RT) {
+#pragma unroll
+        for (int t = 0; t < RT; t++)
+            if (t0 + t < T) {
+#pragma unroll
+                for (int q = 0; q < 4; q++)
+                    sum[(wave * RT + t) * 256 + (4 * grp + q) * 16 + r16] = acc[t0 + t < T ? t0 + t : 0][q];
+            }
+        __syncthreads();
+        for (int e = tid; e < RT * 256; e += 512) {
+            const int t = t0 + e / 256, m = (e >> 4) & 15, n = e & 15;
+            if (t < T) {
+                float s = 0.f;
+#pragma unroll
+                for (int w = 0; w < 8; w++) s += sum[w * RT * 256 + e];
+                out[((size_t)t * cout + co0 + m) * cin + ci0 + n] = s;
             }
         }
-        {
-            const int quad = tid / (CM / 8), cg = tid % (CM / 8);
-#pragma unroll
-            for (int t = 0; t < 4; t++)
-                qd[t] = tid < DITEMS ? *reinterpret_cast<const uint4*>(dy + (size_t)(v0 + 4u * quad + t) * cout +
-                                                                      co0 + 8 * cg)
-                                     : uint4{0u, 0u, 0u, 0u};
-        }
-    };
-    // channel j of two voxels' 8-channel words -> one 32-bit word (voxel a low)
-    auto pair = [](const uint4& a, const uint4& b, int j) {
-        const uint32_t wa = (j >> 1) == 0 ? a.x : (j >> 1) == 1 ? a.y : (j >> 1) == 2 ? a.z : a.w;
-        const uint32_t wb = (j >> 1) == 0 ? b.x : (j >> 1) == 1 ? b.y : (j >> 1) == 2 ? b.z : b.w;
-        return (j & 1) ? ((wa >> 16) | (wb & 0xffff0000u)) : ((wa & 0xffffu) | (wb << 16));
-    };
-    // 4 voxels x 8 channels -> eight 8-byte LDS writes (4 voxels of one channel each)
-    auto put = [&](uint16_t* tile, int ch, int quad, const uint4* q4) {
-#pragma unroll
-        for (int j = 0; j < 8; j++) {
-            const uint32_t w2[2] = {pair(q4[0], q4[1], j), pair(q4[2], q4[3], j)};
-            __builtin_memcpy(__builtin_assume_aligned(tile + (ch + j) * PITCH + 4 * quad, 8), w2, 8);
-        }
-    };
-    auto stage = [&]() {
-#pragma unroll
-        for (int k = 0; k < 2; k++) {
-            const int it = tid + 256 * k;
-            if (it < XITEMS) put(lx + (it >> 4) * CN * PITCH, 8 * (it & 1), (it >> 1) & 7, qx[k]);
-        }
-        if (tid < DITEMS) put(ld, 8 * (tid % (CM / 8)), tid / (CM / 8), qd);
-    };
-    auto frag = [&](const uint16_t* row) {
-        uint4 t;
-        __builtin_memcpy(&t, __builtin_assume_aligned(row, 16), 16);
-        return __builtin_bit_cast(bf16x8, t);
-    };
-
-    const uint32_t n_chunks = g.V / 32u;
-    const uint32_t c0 = blockIdx.x * chunks_per_split;
-    const uint32_t c1 = min(n_chunks, c0 + chunks_per_split);
-    const bool bias = part_b != nullptr && ci0 == 0 && tid < CM;
-    float sb = 0.f;
-    if (c0 < c1) fetch(c0);
-    for (uint32_t c = c0; c < c1; c++) {
-        stage();
-        __syncthreads();
-        if (c + 1 < c1) fetch(c + 1);
-        if (bias)
-            for (int v = 0; v < 32; v++) sb += __builtin_bit_cast(float, (uint32_t)ld[tid * PITCH + v] << 16);
-        bf16x8 a[NM];
-#pragma unroll
-        for (int m = 0; m < NM; m++) a[m] = frag(ld + (m * 16 + r16) * PITCH + 8 * grp);
-#pragma unroll
-        for (int t = 0; t < TW; t++) {
-            const int tap = wave + 4 * t;
-            if (tap < T) {
-                const bf16x8 b = frag(lx + (tap * CN + r16) * PITCH + 8 * grp);
-#pragma unroll
-                for (int m = 0; m < NM; m++) acc[t][m] = mfma(a[m], b, acc[t][m]);
-            }
-        }
         __syncthreads();
     }
-
-    if (bias) part_b[(size_t)blockIdx.x * cout + co0 + tid] = sb;
+    if (bias) {
+        if (r16 == 0)
 #pragma unroll
-    for (int t = 0; t < TW; t++) {
-        const int tap = wave + 4 * t;
-        if (tap >= T) continue;
-        float* out = part + ((size_t)blockIdx.x * T + tap) * (size_t)cout * cin;
+            for (int q = 0; q < 4; q++) sum[wave * 16 + 4 * grp + q] = accb[q];
+        __syncthreads();
+        if (tid < 16) {
+            float s = 0.f;
 #pragma unroll
-        for (int m = 0; m < NM; m++)
-#pragma unroll
-            for (int r = 0; r < 4; r++)
-                out[(size_t)(co0 + m * 16 + 4 * grp + r) * cin + ci0 + r16] = acc[t][m][r];
+            for (int w = 0; w < 8; w++) s += sum[w * 16 + tid];
+            part_b[(size_t)split * cout + co0 + tid] = s;
+        }
     }
 }
 
-// dw[co][tap][ci] = sum_p part[p][tap][co][ci] in two fixed-order levels
-// (deterministic, coalesced over the outputs, 64 outputs per workgroup with
-// 4 threads per output adding every 4th partial, the four sums combined in
-// a fixed order):
-//   level 1 (grid.y = G slices of S partials): the sum of slice y replaces
-//            its first partial, part[y*S] (only this workgroup touches it)
-//   level 2: dw = sum over y of part[y*S]
+// dw[co][tap][ci] = sum_p part[p][tap][co][ci] (and db[co] = sum_p
+// part_b[p][co], the last workgroups), in a fixed order: 16 groups of
+// threads each add every 16th partial, then the 16 sums are added in order.
+// A thread holds 4 consecutive ci (one 16-byte load per partial).
 __global__ void __launch_bounds__(256)
-    k_reduce_w(float* __restrict__ part, int P, int S, int T, int cin, int cout, float* __restrict__ dw,
-               int level)
+    k_reduce_w(const float* __restrict__ part, const float* __restrict__ part_b, int P, int T, int cin, int cout,
+               float* __restrict__ dw, float* __restrict__ db)
 {
-    __shared__ float lds[4][64];
-    const size_t n = (size_t)cout * T * cin;
-    const int e = threadIdx.x & 63, k0 = threadIdx.x >> 6;
-    const size_t i = (size_t)blockIdx.x * 64 + e;
-    const size_t stride = (size_t)T * cout * cin;
-    size_t at = 0;
-    float s = 0.f;
-    if (i < n) {
-        const int ci = (int)(i % cin);
-        const int tap = (int)((i / cin) % T);
-        const int co = (int)(i / ((size_t)cin * T));
-        at = ((size_t)tap * cout + co) * cin + ci;
-        if (level == 1) {
-            const int k1 = min(P, (int)(blockIdx.y + 1) * S);
-            for (int k = (int)blockIdx.y * S + k0; k < k1; k += 4) s += part[(size_t)k * stride + at];
-        } else {
-            for (int y = k0; y * S < P; y += 4) s += part[(size_t)y * S * stride + at];
+    __shared__ float4 lds[256];
+    const int e = threadIdx.x & 15, k0 = threadIdx.x >> 4;
+    const size_t n = (size_t)cout * T * cin, nq = n / 4;
+    const size_t i = (size_t)blockIdx.x * 16 + e;
+    const bool isb = i >= nq;                          // the bias rows follow the weights
+    const size_t ib = i - nq;
+    const bool ok = !isb || (db != nullptr && ib < (size_t)cout / 4);
+    const float* src = isb ? part_b + 4 * ib : part + 4 * i;
+    const size_t stride = isb ? (size_t)cout : n;
+    float4 s = float4{0.f, 0.f, 0.f, 0.f};
+    if (ok)
+        for (int k = k0; k < P; k += 16) {
+            const float4 v = *reinterpret_cast<const float4*>(src + (size_t)k * stride);
+            s.x += v.x;
+            s.y += v.y;
+            s.z += v.z;
+            s.w += v.w;
         }
-    }
-    lds[k0][e] = s;
-    __syncthreads();
-    if (k0 == 0 && i < n) {
-        const float t = ((lds[0][e] + lds[1][e]) + lds[2][e]) + lds[3][e];
-        if (level == 1)
-            part[(size_t)blockIdx.y * S * stride + at] = t;
-        else
-            dw[i] = t;
-    }
-}
-
-// Per-channel sums of dy over voxel ranges: part[blockIdx.x][c].
-__global__ void __launch_bounds__(256)
-    k_colsum(const uint16_t* __restrict__ dy, uint32_t V, int C, uint32_t per_block,
-             float* __restrict__ part)
-{
-    __shared__ float lds[256];
-    const int rows = 256 / C;  // C <= 256; threads past rows*C idle
-    const int c = threadIdx.x % C, j = threadIdx.x / C;
-    const uint32_t v0 = blockIdx.x * per_block, v1 = min(V, v0 + per_block);
-    float s = 0.f;
-    if (j < rows)
-        for (uint32_t v = v0 + (uint32_t)j; v < v1; v += (uint32_t)rows)
-            s += __builtin_bit_cast(float, (uint32_t)dy[(size_t)v * C + c] << 16);
     lds[threadIdx.x] = s;
     __syncthreads();
-    if (threadIdx.x < C) {
-        float t = 0.f;
-        for (int k = 0; k < rows; k++) t += lds[k * C + threadIdx.x];
-        part[(size_t)blockIdx.x * C + threadIdx.x] = t;
+    if (k0 != 0 || !ok) return;
+    float4 t = lds[e];
+    for (int k = 1; k < 16; k++) {
+        const float4 v = lds[16 * k + e];
+        t.x += v.x;
+        t.y += v.y;
+        t.z += v.z;
+        t.w += v.w;
     }
-}
-
-// out[c] = sum_k part[k][c]: one workgroup per channel, fixed-order tree
-__global__ void __launch_bounds__(256)
-    k_reduce_cols(const float* __restrict__ part, int P, int C, float* __restrict__ out)
-{
-    __shared__ float lds[256];
-    const int c = (int)blockIdx.x;
-    float s = 0.f;
-    for (int k = threadIdx.x; k < P; k += 256) s += part[(size_t)k * C + c];
-    lds[threadIdx.x] = s;
-    __syncthreads();
-    for (int w = 128; w > 0; w >>= 1) {
-        if ((int)threadIdx.x < w) lds[threadIdx.x] += lds[threadIdx.x + w];
-        __syncthreads();
+    if (isb) {
+        float* o = db + 4 * ib;                        // (the caller's arrays: 4-byte aligned)
+        o[0] = t.x, o[1] = t.y, o[2] = t.z, o[3] = t.w;
+    } else {
+        // part order [tap][co][ci] -> dw order [co][tap][ci]
+        const int c4 = cin / 4;
+        const int ci = (int)(i % c4) * 4, co = (int)((i / c4) % cout), tap = (int)(i / ((size_t)c4 * cout));
+        float* o = dw + ((size_t)co * T + tap) * cin + ci;
+        o[0] = t.x, o[1] = t.y, o[2] = t.z, o[3] = t.w;
     }
-    if (threadIdx.x == 0) out[c] = lds[0];
 }
 
 __global__ void __launch_bounds__(256)
@@ -743,53 +822,41 @@ int launch_fwd(const Shape& s, const uint16_t* x, const uint16_t* w, const float
     });
 }
 
+// How a weight gradient is cut up.  k_bwd_wy (3^3, rows of >= 4 voxels: its
+// LDS row sets fit two buffers down to 4-voxel rows) takes one workgroup per
+// CU and 16 x 16 channel block; fewer, longer runs would leave CUs idle, more
+// would only add partials.  part_splits bounds the splits of every smaller
+// batch too (the workspace is sized once for the largest).
 struct WPlan {
-    int nm, nn, T;
-    bool all_taps;  // k_bwd_w27: 3^3 kernel, rows of >= 32 voxels
-    uint32_t splits, chunks_per_split;
-    size_t part_floats;
-    int partials;   // partials per output element (reduced by k_reduce_w)
+    int T;
+    bool rows_kernel;
+    int nm, nn;                     // k_bwd_w
+    uint32_t pairs, rows, per;      // k_bwd_wy: channel blocks, row steps, row steps per split
+    uint32_t splits, part_splits;
 };
 
 WPlan plan_w(const Shape& s)
 {
-    WPlan p;
+    WPlan p{};
     p.T = s.ks * s.ks * s.ks;
-    p.all_taps = s.ks == 3 && s.w >= 32;
-    if (p.all_taps) {
+    p.rows_kernel = s.ks == 3 && s.w >= 4;
+    uint32_t units;
+    if (p.rows_kernel) {
+        const int ws = std::min(s.w, 32), tz = 8 * (32 / ws);
+        p.pairs = (uint32_t)((s.cout / 16) * (s.cin / 16));
+        units = p.rows = (uint32_t)((s.w / ws) * ((s.d + tz - 1) / tz)) * (uint32_t)s.n * (uint32_t)s.h;
+        p.part_splits = std::max(1u, std::min(256u / p.pairs, units));
+    } else {
         p.nm = tiles_of(s.cout / 16, 4);
-        p.nn = 1;
-        const uint64_t V = (uint64_t)s.n * s.d * s.h * s.w;
-        const uint32_t n_chunks = (uint32_t)(V / 32);
-        const uint32_t blocks = (uint32_t)((s.cout / (16 * p.nm)) * (s.cin / 16));
-        // about three workgroups per CU (the kernel's register use allows
-        // three), each walking a contiguous run of chunks
-        uint32_t splits = (768u + blocks - 1) / blocks;
-        // at most 16 M partial floats (64 MB of workspace)
-        const uint32_t cap = (uint32_t)std::max<uint64_t>(1, (16ull << 20) / ((uint64_t)27 * s.cout * s.cin));
-        splits = std::max(1u, std::min({splits, cap, n_chunks}));
-        p.chunks_per_split = (n_chunks + splits - 1) / splits;
-        p.splits = (n_chunks + p.chunks_per_split - 1) / p.chunks_per_split;
-        p.part_floats = (size_t)p.splits * 27 * s.cout * s.cin;
-        p.partials = (int)p.splits;
-        return p;
+        p.nn = tiles_of(s.cin / 16, 4);
+        units = (uint32_t)(((uint64_t)s.n * s.d * s.h * s.w + 31) / 32);
+        const uint32_t blocks = (uint32_t)(p.T * (s.cout / (16 * p.nm)) * (s.cin / (16 * p.nn)));
+        p.part_splits = std::max(1u, std::min({(2048u + blocks - 1) / blocks, 512u, (units + 3u) / 4u}));
     }
-    p.nm = tiles_of(s.cout / 16, 4);
-    p.nn = tiles_of(s.cin / 16, 4);
-    const uint64_t V = (uint64_t)s.n * s.d * s.h * s.w;
-    const uint32_t n_chunks = (uint32_t)((V + 31) / 32);
-    const uint32_t blocks = (uint32_t)(p.T * (s.cout / (16 * p.nm)) * (s.cin / (16 * p.nn)));
-    uint32_t splits = (2048u + blocks - 1) / blocks;
-    splits = std::max(1u, std::min({splits, 512u, (n_chunks + 3u) / 4u}));
-    p.chunks_per_split = (n_chunks + splits - 1) / splits;
-    p.splits = (n_chunks + p.chunks_per_split - 1) / p.chunks_per_split;
-    if (p.splits == 0) p.splits = 1;
-    p.part_floats = (size_t)p.splits * 4 * p.T * s.cout * s.cin;
-    p.partials = (int)(p.splits * 4);
+    p.per = (units + p.part_splits - 1) / p.part_splits;
+    p.splits = (units + p.per - 1) / p.per;
     return p;
 }
-
-constexpr uint32_t kColBlocks = 512;
 
 }  // namespace
 
@@ -834,13 +901,11 @@ int bwd_data(const Shape& s, const uint16_t* dy, const uint16_t* wt, void* dx, i
     return NX_OK;
 }
 
+// weight partials, then bias partials
 size_t bwd_weight_ws(const Shape& s)
 {
     const WPlan p = plan_w(s);
-    const size_t cols = (size_t)kColBlocks * s.cout;
-    // all-taps plan: weight partials, then the bias partials (splits x cout)
-    if (p.all_taps) return (p.part_floats + (size_t)p.splits * s.cout) * sizeof(float);
-    return (std::max(p.part_floats, cols)) * sizeof(float);
+    return (size_t)p.part_splits * ((size_t)p.T * s.cout * s.cin + s.cout) * sizeof(float);
 }
 
 int bwd_weight(const Shape& s, const uint16_t* x, const uint16_t* dy, float* dw, float* db, void* ws,
@@ -848,67 +913,50 @@ int bwd_weight(const Shape& s, const uint16_t* x, const uint16_t* dy, float* dw,
 {
     const Geo g = geo_of(s);
     const WPlan p = plan_w(s);
-    float* part = static_cast<float*>(ws);
-    const dim3 grid(p.all_taps ? p.splits : p.T * p.splits,
-                    (unsigned)((s.cout / (16 * p.nm)) * (s.cin / (16 * p.nn))));
-    if (p.all_taps) {
-        auto go27 = [&](auto NM) {
-            hipLaunchKernelGGL((k_bwd_w27<decltype(NM)::value>), grid, dim3(256), 0, st, x, dy, part,
-                               db ? part + p.part_floats : nullptr, g, s.cin, s.cout, p.chunks_per_split);
-        };
-        switch (p.nm) {
-            case 4: go27(std::integral_constant<int, 4>{}); break;
-            case 3: go27(std::integral_constant<int, 3>{}); break;
-            case 2: go27(std::integral_constant<int, 2>{}); break;
-            default: go27(std::integral_constant<int, 1>{}); break;
-        }
-        NX_CHECK_LAUNCH("k_bwd_w27");
-    }
-    int err = p.all_taps ? 0 : by_ks(s.ks, [&](auto KS) {
-        auto go = [&](auto NM, auto NN) {
-            hipLaunchKernelGGL((k_bwd_w<decltype(NM)::value, decltype(NN)::value, KS>), grid,
-                               dim3(256), 0, st, x, dy, part, g, s.cin, s.cout, p.chunks_per_split);
-        };
-        auto by_nn = [&](auto NM) {
-            switch (p.nn) {
-                case 4: go(NM, std::integral_constant<int, 4>{}); break;
-                case 3: go(NM, std::integral_constant<int, 3>{}); break;
-                case 2: go(NM, std::integral_constant<int, 2>{}); break;
-                default: go(NM, std::integral_constant<int, 1>{}); break;
-            }
-        };
-        switch (p.nm) {
-            case 4: by_nn(std::integral_constant<int, 4>{}); break;
-            case 3: by_nn(std::integral_constant<int, 3>{}); break;
-            case 2: by_nn(std::integral_constant<int, 2>{}); break;
-            default: by_nn(std::integral_constant<int, 1>{}); break;
-        }
-    });
-    if (err) return err;
-    NX_CHECK_LAUNCH("k_bwd_w");
     const size_t nw = (size_t)s.cout * p.T * s.cin;
-    // level 1 in slices of S partials, then the G slice sums
-    const int G = std::max(1, std::min(64, p.partials / 32));
-    const int S = (p.partials + G - 1) / G;
-    const unsigned gx = (unsigned)((nw + 63) / 64);
-    hipLaunchKernelGGL(k_reduce_w, dim3(gx, (unsigned)((p.partials + S - 1) / S)), dim3(256), 0, st, part,
-                       p.partials, S, p.T, s.cin, s.cout, dw, 1);
-    hipLaunchKernelGGL(k_reduce_w, dim3(gx), dim3(256), 0, st, part, p.partials, S, p.T, s.cin, s.cout,
-                       dw, 2);
-    NX_CHECK_LAUNCH("k_reduce_w");
-    if (db && p.all_taps) {
-        hipLaunchKernelGGL(k_reduce_cols, dim3(s.cout), dim3(256), 0, st, part + p.part_floats,
-                           (int)p.splits, s.cout, db);
-        NX_CHECK_LAUNCH("k_reduce_cols");
-    } else if (db) {
-        // the column partials reuse the workspace after the weight reduction
-        const uint32_t per = (g.V + kColBlocks - 1) / kColBlocks;
-        hipLaunchKernelGGL(k_colsum, dim3(kColBlocks), dim3(256), 0, st, dy, g.V, s.cout, per, part);
-        NX_CHECK_LAUNCH("k_colsum");
-        hipLaunchKernelGGL(k_reduce_cols, dim3(s.cout), dim3(256), 0, st, part, (int)kColBlocks,
-                           s.cout, db);
-        NX_CHECK_LAUNCH("k_reduce_cols");
+    float* part = static_cast<float*>(ws);
+    float* part_b = db ? part + (size_t)p.splits * nw : nullptr;
+    if (p.rows_kernel) {
+        auto go = [&](auto WS) {
+            hipLaunchKernelGGL((k_bwd_wy<decltype(WS)::value>), dim3(p.splits * p.pairs), dim3(512), 0, st, x, dy,
+                               part, part_b, g, s.cin, s.cout, p.rows, p.per, p.pairs);
+        };
+        switch (std::min(s.w, 32)) {
+            case 32: go(std::integral_constant<int, 32>{}); break;
+            case 16: go(std::integral_constant<int, 16>{}); break;
+            case 8: go(std::integral_constant<int, 8>{}); break;
+            default: go(std::integral_constant<int, 4>{}); break;
+        }
+        NX_CHECK_LAUNCH("k_bwd_wy");
+    } else {
+        const dim3 grid(p.T * p.splits, (unsigned)((s.cout / (16 * p.nm)) * (s.cin / (16 * p.nn))));
+        const int err = by_ks(s.ks, [&](auto KS) {
+            auto go = [&](auto NM, auto NN) {
+                hipLaunchKernelGGL((k_bwd_w<decltype(NM)::value, decltype(NN)::value, KS>), grid, dim3(256), 0, st,
+                                   x, dy, part, part_b, g, s.cin, s.cout, p.per);
+            };
+            auto by_nn = [&](auto NM) {
+                switch (p.nn) {
+                    case 4: go(NM, std::integral_constant<int, 4>{}); break;
+                    case 3: go(NM, std::integral_constant<int, 3>{}); break;
+                    case 2: go(NM, std::integral_constant<int, 2>{}); break;
+                    default: go(NM, std::integral_constant<int, 1>{}); break;
+                }
+            };
+            switch (p.nm) {
+                case 4: by_nn(std::integral_constant<int, 4>{}); break;
+                case 3: by_nn(std::integral_constant<int, 3>{}); break;
+                case 2: by_nn(std::integral_constant<int, 2>{}); break;
+                default: by_nn(std::integral_constant<int, 1>{}); break;
+            }
+        });
+        if (err) return err;
+        NX_CHECK_LAUNCH("k_bwd_w");
     }
+    const size_t quads = nw / 4 + (db ? (size_t)s.cout / 4 : 0);
+    hipLaunchKernelGGL(k_reduce_w, dim3((unsigned)((quads + 15) / 16)), dim3(256), 0, st, part, part_b, (int)p.splits,
+                       p.T, s.cin, s.cout, dw, db);
+    NX_CHECK_LAUNCH("k_reduce_w");
     return NX_OK;
 }
 
