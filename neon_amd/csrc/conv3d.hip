@@ -27,6 +27,7 @@ namespace nx::conv {
 namespace {
 
 typedef __bf16 bf16x8 __attribute__((ext_vector_type(8)));
+typedef __bf16 bf16x4 __attribute__((ext_vector_type(4)));
 typedef unsigned short u16x8 __attribute__((ext_vector_type(8)));
 typedef float f32x4 __attribute__((ext_vector_type(4)));
 
@@ -52,6 +53,27 @@ __device__ __forceinline__ bf16x8 ld8(const uint16_t* p)
 __device__ __forceinline__ f32x4 mfma(bf16x8 a, bf16x8 b, f32x4 c)
 {
     return __builtin_amdgcn_mfma_f32_16x16x32_bf16(a, b, c, 0, 0, 0);
+}
+
+// Four consecutive channels of a voxel at element i + o of y (i the same for
+// the whole wavefront); mask as in k_fwd_blk.
+__device__ __forceinline__ void put4(void* y, const uint16_t* mask, size_t i, uint32_t o, f32x4 v, bool f32out)
+{
+    if (f32out) {
+        float* p = static_cast<float*>(y) + i + o;
+#pragma unroll
+        for (int r = 0; r < 4; r++) p[r] = v[r];
+        return;
+    }
+    typedef unsigned short u16x4 __attribute__((ext_vector_type(4)));
+    u16x4 h = __builtin_bit_cast(u16x4, __builtin_convertvector(v, bf16x4));
+    if (mask) {
+        const u16x4 m = *reinterpret_cast<const u16x4*>(mask + i + o);
+#pragma unroll
+        for (int r = 0; r < 4; r++)
+            if ((m[r] & 0x8000u) != 0 || (m[r] & 0x7fffu) == 0) h[r] = 0;
+    }
+    __builtin_memcpy(static_cast<uint16_t*>(y) + i + o, &h, 8);
 }
 
 template <int KS>
@@ -170,124 +192,430 @@ __global__ void __launch_bounds__(256)
     }
 }
 
-// 3^3 forward (and backward-data) with the input tile in LDS, for rows of
-// >= 32 voxels.  A workgroup computes a 32 x 4 x 4 block of output voxels
-// (x, y, z).  For each slice of 16 input channels it stages the block's input
-// with its one-voxel halo, 34 x 6 x 6 voxels x 16 channels (39 KB), in
-// channels-last order (one 16-byte LDS write per load); each wave then
-// takes 4 rows of 32 voxels, reads every A fragment (8 channels of one tap
-// for one voxel) with one ds_read_b128, and uses each weight fragment for
-// all of its rows.  Each input voxel is read from memory ~2x instead of 27x.
-// CINC = 16 fixes the channel count (one slice, fewer registers); 0 reads it
-// from the argument.
-template <int NT, int CINC>
-__global__ void __launch_bounds__(256)
-    k_fwd_tile(const uint16_t* __restrict__ x, const uint16_t* __restrict__ w,
-               const float* __restrict__ bias, void* __restrict__ y, Geo g, int cin_arg, int cout, int flags)
+// 3^3 forward (and backward-data) with the input block in LDS, for rows of at
+// least 4 voxels.  M = output channels (A: weights, one 16-byte load per
+// lane), N = 16 voxels (B: 8 channels of a voxel, one ds_read_b128), K = 32
+// channels of one tap, or for the last 16 channels of an odd count the taps
+// (dx = -1, dx = 0) of a voxel pair, then dx = 1 alone.  A tile is 16 voxels:
+// WX along x times YT = 16 / WX rows.  A wavefront computes RY x RZ tiles in y
+// and z for NCO blocks of 16 output channels; NXW x NYW x NZW wavefronts share
+// one staged block with its halo, CM channels (32, or 16 where the input has
+// no more) at a time.  A B fragment serves every output row of the wavefront
+// that a tap reaches from it and all NCO channel blocks (3 or 9 NCO MFMAs):
+// with one LDS read per MFMA the LDS takes twice the MFMA's time.  A
+// workgroup takes a run of blocks; the next slice of channels, or of the next
+// block, is loaded into registers while the matrix cores work on this one,
+// and the next weights likewise.  A lane ends with 4 consecutive channels of
+// a voxel: 8- or 16-byte stores.
+// Measured (MI355X): 64^3 x 8, 48 -> 16 157 us (225 us with one LDS read per
+// MFMA, 16 channels at a time); 32^3 x 8, 96 -> 32 55 us (101); 32^3 x 16,
+// 64 -> 64 165 us (250); 16^3 x 8, 64 -> 64 22 us (43, fragments from memory).
+// mask: null, or the activations whose ReLU the result passes back through
+// (0 where the activation is not positive).
+template <int WX, int NXW, int NYW, int NZW, int RY, int RZ, int NCO, bool AHEAD>
+__global__ void __launch_bounds__(256, 2)
+    k_fwd_blk(const uint16_t* __restrict__ x, const uint16_t* __restrict__ w, const float* __restrict__ bias,
+              const uint16_t* __restrict__ mask, void* __restrict__ y, Geo g, int cin, int cout, int flags,
+              uint32_t blocks, uint32_t per_wg)
 {
-    const int cin = CINC ? CINC : cin_arg;           // CINC: channel count fixed at compile time
-    constexpr int TX = 32, TY = 4, TZ = 4, HX = TX + 2, HY = TY + 2, HZ = TZ + 2, CS = 16;
-    constexpr int RW = TY * TZ / 4;                  // rows per wave
-    constexpr int KS_ = 27 * CS, KC = (KS_ + 31) / 32;
-    constexpr int ITEMS = HX * HY * HZ * (CS / 8);   // 16-byte pieces of one slice's halo tile
-    __shared__ __attribute__((aligned(16))) uint16_t tile[HX * HY * HZ * CS];
-    const int tid = threadIdx.x, lane = tid & 63, wave = tid >> 6;
+    static_assert(NXW * NYW * NZW == 4, "four wavefronts");
+    constexpr int CM = 32;                                       // channels of a full slice
+    constexpr int YT = 16 / WX, SY = (RY - 1) * YT + 3;          // SY: source row offsets of a wavefront
+    constexpr int BX = NXW * WX, BY = NYW * YT * RY, BZ = NZW * RZ;
+    constexpr int HX = BX + 2, HY = BY + 2, HZ = BZ + 2, HV = HX * HY * HZ;
+    constexpr int ROWS = HY * HZ;
+    // 16-byte pieces of a slice per thread: own voxels, halo columns
+    constexpr int NM = (ROWS * BX * (CM / 8) + 255) / 256, NH = (ROWS * 2 * (CM / 8) + 255) / 256;
+    constexpr int ZG = NCO == 1 || (!AHEAD && NCO == 2) ? 1 : 3; // weight groups per K step: all dz, or one each
+    constexpr int NDZ = 3 / ZG;
+    __shared__ __attribute__((aligned(16))) uint16_t tile[HV * CM];
+    const int tid = (int)threadIdx.x, lane = tid & 63;
+    const int wave = __builtin_amdgcn_readfirstlane(tid >> 6);
     const int r16 = lane & 15, grp = lane >> 4;
-    const int co0 = (int)blockIdx.y * NT * 16;
-    const int K = 27 * cin;
-    // tile origin: blocks x fastest, then y, then z (z spans batch * depth)
-    const int nbx = g.W / TX, nby = g.H / TY, nbz = g.D / TZ;
-    const int bx = (int)(blockIdx.x % (uint32_t)nbx);
-    const int by = (int)((blockIdx.x / (uint32_t)nbx) % (uint32_t)nby);
-    const int bzall = (int)(blockIdx.x / (uint32_t)(nbx * nby));   // (sample, z block)
-    const int sample = bzall / nbz, z0 = (bzall % nbz) * TZ, y0 = by * TY, x0 = bx * TX;
-    const size_t sample_base = (size_t)sample * g.D * g.H * g.W;
+    const uint32_t ncb = (uint32_t)(cout / (16 * NCO));
+    const uint32_t nbx = (uint32_t)(g.W / BX), nby = (uint32_t)((g.H + BY - 1) / BY), nbz = (uint32_t)((g.D + BZ - 1) / BZ);
+    const int wx = wave % NXW, wy = (wave / NXW) % NYW, wz = wave / (NXW * NYW);
+    const int lx = r16 % WX, ly = r16 / WX;
+    // halo-block voxel of this lane at offset (-1, -1, -1) of its first tile
+    const int hv0 = (wz * RZ * HY + wy * YT * RY + ly) * HX + wx * WX + lx;
 
-    const uint16_t* wrow[NT];
-#pragma unroll
-    for (int n = 0; n < NT; n++) wrow[n] = w + (size_t)(co0 + n * 16 + r16) * K;
-    f32x4 acc[RW][2][NT];
-#pragma unroll
-    for (int j = 0; j < RW; j++)
-#pragma unroll
-        for (int t = 0; t < 2; t++)
-#pragma unroll
-            for (int n = 0; n < NT; n++) acc[j][t][n] = f32x4{0.f, 0.f, 0.f, 0.f};
-
-    for (int c0 = 0; c0 < cin; c0 += CS) {
-        if (c0) __syncthreads();                     // the previous slice's reads are done
-        for (int it = tid; it < ITEMS; it += 256) {
-            const int piece = it & 1, hv = it >> 1;
-            const int hx = hv % HX, hy = (hv / HX) % HY, hz = hv / (HX * HY);
-            const int gx = x0 - 1 + hx, gy = y0 - 1 + hy, gz = z0 - 1 + hz;
-            uint4 v = uint4{0u, 0u, 0u, 0u};
-            if ((unsigned)gx < (unsigned)g.W && (unsigned)gy < (unsigned)g.H && (unsigned)gz < (unsigned)g.D)
-                v = *reinterpret_cast<const uint4*>(
-                    x + (sample_base + ((size_t)gz * g.H + gy) * g.W + gx) * cin + c0 + 8 * piece);
-            *reinterpret_cast<uint4*>(tile + (size_t)hv * CS + 8 * piece) = v;
+    // blocks of one XCD in order: channel blocks of a position, then x, y, z, sample
+    struct Block {
+        int co0, x0, y0, z0;
+        uint32_t smp;
+    };
+    auto block_of = [&](uint32_t id) {
+        Block b;
+        b.co0 = (int)(id % ncb) * 16 * NCO;
+        id /= ncb;
+        b.x0 = (int)(id % nbx) * BX;
+        id /= nbx;
+        b.y0 = (int)(id % nby) * BY;
+        id /= nby;
+        b.z0 = (int)(id % nbz) * BZ;
+        b.smp = id / nbz;
+        return b;
+    };
+    // Staging: the block's own voxels by whole rows (BX x PV pieces, a power of
+    // two; where a row fills a wavefront's load its address and its test are
+    // scalar), then the two halo columns.  A slice is 32 channels (PV = 4
+    // 16-byte pieces a voxel) or the last 16 (PV = 2).
+    uint4 pre[NM], pre_h[NH];
+    auto row_of = [&](auto pvc, int k, int& row, int& q) {
+        constexpr int RP = BX * decltype(pvc)::value;
+        const int at = (k * 4 + wave) * 64;
+        if constexpr (RP >= 64) {
+            row = at / RP;
+            q = at % RP + lane;
+        } else {
+            row = at / RP + lane / RP;
+            q = lane % RP;
         }
-        __syncthreads();
-
-        // K step kc of the slice: lane group grp holds tap (32 kc + 8 grp) / 16,
-        // channels c0 + (8 grp) % 16 ..+7; past the last tap it contributes
-        // zeros -- the MFMAs run for every lane (a lane left out of one would
-        // not receive its accumulator rows)
-        auto fetch_b = [&](int kc, bf16x8* b) {
-            const int kk = kc * 32 + 8 * grp;
-            const int tap = kk / CS, ci = kk % CS;
+    };
+    auto row_base = [&](const Block& b, int row, bool& in) {
+        const int gy = b.y0 - 1 + row % HY, gz = b.z0 - 1 + row / HY;
+        in = row < ROWS && (unsigned)gy < (unsigned)g.H && (unsigned)gz < (unsigned)g.D;
+        return (uint32_t)((gz * g.H + gy) * g.W + b.x0);
+    };
+    auto fetch_pv = [&](auto pvc, const Block& b, int c0) __attribute__((always_inline)) {
+        constexpr int PV = decltype(pvc)::value;
+        const uint16_t* xs = x + (size_t)b.smp * (uint32_t)(g.D * g.H * g.W) * (uint32_t)cin + c0;
 #pragma unroll
-            for (int n = 0; n < NT; n++)
-                b[n] = kk < KS_ ? ld8(wrow[n] + tap * cin + c0 + ci) : bf16x8{};
-        };
-        bf16x8 b0[NT], b1[NT];
-        fetch_b(0, b0);
-        for (int kc = 0; kc < KC; kc++) {
-            if (kc + 1 < KC) fetch_b(kc + 1, b1);
-            const int kk = kc * 32 + 8 * grp;
-            const bool kok = kk < KS_;
-            const int tap = kok ? kk / CS : 26, ci = kok ? kk % CS : 0;
-            int dz, dyo, dx;
-            tap_offset<3>(tap, dz, dyo, dx);
+        for (int k = 0; k < (ROWS * BX * PV + 255) / 256; k++) {
+            int row, q;
+            row_of(pvc, k, row, q);
+            bool in;
+            const uint16_t* p = xs + (size_t)(row_base(b, row, in) * (uint32_t)cin);
+            pre[k] = in ? *reinterpret_cast<const uint4*>(p + (uint32_t)((q / PV) * cin + 8 * (q % PV))) : uint4{0u, 0u, 0u, 0u};
+        }
 #pragma unroll
-            for (int j = 0; j < RW; j++) {
-                const int row = wave * RW + j;
-                const int ly = row % TY, lz = row / TY;
+        for (int k = 0; k < (ROWS * 2 * PV + 255) / 256; k++) {
+            const int it = tid + 256 * k, row = it / (2 * PV), side = (it / PV) & 1, pc = it % PV;
+            bool in;
+            const uint32_t v = row_base(b, row, in) + (side ? (uint32_t)BX : ~0u);
+            in = in && (side ? b.x0 + BX < g.W : b.x0 > 0);
+            pre_h[k] = in ? *reinterpret_cast<const uint4*>(xs + (uint32_t)(v * (uint32_t)cin + 8 * pc)) : uint4{0u, 0u, 0u, 0u};
+        }
+    };
+    auto fetch = [&](const Block& b, int c0) __attribute__((always_inline)) {
+        if (cin - c0 >= 32) fetch_pv(std::integral_constant<int, CM / 8>{}, b, c0);
+        else fetch_pv(std::integral_constant<int, 2>{}, b, c0);
+    };
+    // the same without registers held: a batch of loads, then their LDS writes
+    auto stage = [&](auto pvc, const Block& b, int c0) __attribute__((always_inline)) {
+        constexpr int PV = decltype(pvc)::value, KM = (ROWS * BX * PV + 255) / 256, NB = 9;
+        const uint16_t* xs = x + (size_t)b.smp * (uint32_t)(g.D * g.H * g.W) * (uint32_t)cin + c0;
+        uint4 h[NH];
 #pragma unroll
-                for (int t = 0; t < 2; t++) {
-                    const int hv = ((lz + dz + 1) * HY + (ly + dyo + 1)) * HX + (16 * t + r16 + dx + 1);
-                    const bf16x8 a = kok ? ld8(tile + (size_t)hv * CS + ci) : bf16x8{};
+        for (int k = 0; k < (ROWS * 2 * PV + 255) / 256; k++) {
+            const int it = tid + 256 * k, row = it / (2 * PV), side = (it / PV) & 1, pc = it % PV;
+            bool in;
+            const uint32_t v = row_base(b, row, in) + (side ? (uint32_t)BX : ~0u);
+            in = in && (side ? b.x0 + BX < g.W : b.x0 > 0);
+            h[k] = in ? *reinterpret_cast<const uint4*>(xs + (uint32_t)(v * (uint32_t)cin + 8 * pc)) : uint4{0u, 0u, 0u, 0u};
+        }
+#pragma unroll 1
+        for (int k0 = 0; k0 < KM; k0 += NB) {
+            uint4 v[NB];
 #pragma unroll
-                    for (int n = 0; n < NT; n++) acc[j][t][n] = mfma(a, b0[n], acc[j][t][n]);
-                }
+            for (int k = 0; k < NB; k++) {
+                int row, q;
+                row_of(pvc, k0 + k, row, q);
+                bool in;
+                const uint16_t* p = xs + (size_t)(row_base(b, row, in) * (uint32_t)cin);
+                v[k] = in ? *reinterpret_cast<const uint4*>(p + (uint32_t)((q / PV) * cin + 8 * (q % PV))) : uint4{0u, 0u, 0u, 0u};
             }
 #pragma unroll
-            for (int n = 0; n < NT; n++) b0[n] = b1[n];
+            for (int k = 0; k < NB; k++) {
+                int row, q;
+                row_of(pvc, k0 + k, row, q);
+                if (row < ROWS) *reinterpret_cast<uint4*>(tile + (row * HX + 1) * PV * 8 + q * 8) = v[k];
+            }
         }
-    }
+#pragma unroll
+        for (int k = 0; k < (ROWS * 2 * PV + 255) / 256; k++) {
+            const int it = tid + 256 * k, row = it / (2 * PV), side = (it / PV) & 1, pc = it % PV;
+            if (row < ROWS) *reinterpret_cast<uint4*>(tile + ((row * HX + (side ? HX - 1 : 0)) * PV + pc) * 8) = h[k];
+        }
+    };
+    auto put = [&](auto pvc) {
+        constexpr int PV = decltype(pvc)::value;
+#pragma unroll
+        for (int k = 0; k < (ROWS * BX * PV + 255) / 256; k++) {
+            int row, q;
+            row_of(pvc, k, row, q);
+            if (row < ROWS) *reinterpret_cast<uint4*>(tile + (row * HX + 1) * PV * 8 + q * 8) = pre[k];
+        }
+#pragma unroll
+        for (int k = 0; k < (ROWS * 2 * PV + 255) / 256; k++) {
+            const int it = tid + 256 * k, row = it / (2 * PV), side = (it / PV) & 1, pc = it % PV;
+            if (row < ROWS) *reinterpret_cast<uint4*>(tile + ((row * HX + (side ? HX - 1 : 0)) * PV + pc) * 8) = pre_h[k];
+        }
+    };
 
-    const bool relu = flags & kRelu, f32out = flags & kOutF32;
+    const uint32_t first = xcd_remap(blockIdx.x, gridDim.x) * per_wg, last = min(blocks, first + per_wg);
+    if (first >= last) return;
+    f32x4 acc[RZ][RY][NCO];
+    auto slice = [&](auto csc, const Block& b, int c0, const Block& nb, int nc0, bool more) __attribute__((always_inline)) {
+        constexpr int CS = decltype(csc)::value, PV = CS / 8;
+        constexpr int NK = CS == 32 ? 3 : 2;                     // K steps per (dz, dy): dx, or dx pairs
+        const bool half = CS == 16 && grp >= 2;                  // the second tap of a pair
+        const uint16_t* wb = w + (size_t)b.co0 * 27 * cin + c0;
+        const uint32_t wo = (uint32_t)(r16 * 27 * cin + (CS == 32 ? 8 * grp : 8 * (grp & 1) + (grp >> 1) * cin));
+        const uint16_t* tl = tile + hv0 * CS + 8 * grp;          // CS = 16: groups 2, 3 read the next voxel
+        bf16x8 a[AHEAD ? 2 : 1][NDZ][3][NCO];
+        // weight group wg = (K step, last first) * ZG + dz group; past dx = 1 a
+        // pair has no second tap
+        auto load_w = [&](int wg, bf16x8 (*d)[3][NCO]) {
+            const int kx = NK - 1 - wg / ZG;
+            const bool none = CS == 16 && kx == 1 && half;
 #pragma unroll
-    for (int j = 0; j < RW; j++) {
-        const int row = wave * RW + j;
-        const int ly = row % TY, lz = row / TY;
-        const size_t vrow = sample_base + ((size_t)(z0 + lz) * g.H + (y0 + ly)) * g.W + x0;
+            for (int i = 0; i < NDZ; i++)
 #pragma unroll
-        for (int n = 0; n < NT; n++) {
-            const int co = co0 + n * 16 + r16;
-            const float bv = bias ? bias[co] : 0.f;
+                for (int dyo = 0; dyo < 3; dyo++)
 #pragma unroll
-            for (int t = 0; t < 2; t++)
+                    for (int n = 0; n < NCO; n++) {
+                        const int tap = ((wg % ZG + i) * 3 + dyo) * 3 + (CS == 32 ? kx : 2 * kx);
+                        d[i][dyo][n] = none ? bf16x8{} : ld8(wb + (size_t)((n * 16 * 27 + tap) * cin) + wo);
+                    }
+        };
+        auto load_x = [&](int kx, int zr, int s) {
+            bf16x8 v = ld8(tl + ((zr * HY + s) * HX + (CS == 32 ? kx : 2 * kx)) * CS);
+            if (CS == 16 && kx == 1 && half) v = bf16x8{};
+            return v;
+        };
+        // Loads return in order, so a wait for weights would also wait for
+        // the next slice if that was asked for first: it goes after the last
+        // weights, which are never far ahead.
+        constexpr int NG = NK * ZG;
+        load_w(0, a[0]);
+        if (AHEAD && NG == 2) load_w(1, a[1]);
+        __syncthreads();                                         // the previous slice's reads are done
+        if (AHEAD) put(std::integral_constant<int, PV>{});
+        else stage(std::integral_constant<int, PV>{}, b, c0);
+        __syncthreads();
+        if (AHEAD && NG == 2 && more) fetch(nb, nc0);
+        // steps of one source plane; its fragments are read while the matrix
+        // cores work on the plane before where the registers allow it (NCO = 1)
+        constexpr int NZR = RZ + NDZ - 1;
+        constexpr bool PIPE = NCO == 1 && !AHEAD;
+        bf16x8 v[PIPE ? 2 : 1][SY];
+        auto plane = [&](int st) {
 #pragma unroll
-                for (int r = 0; r < 4; r++) {
-                    const size_t v = vrow + 16 * t + 4 * grp + r;
-                    float sv = acc[j][t][n][r] + bv;
-                    if (relu) sv = sv > 0.f ? sv : 0.f;
-                    if (f32out)
-                        static_cast<float*>(y)[v * cout + co] = sv;
-                    else
-                        static_cast<uint16_t*>(y)[v * cout + co] = f2bf(sv);
+            for (int s = 0; s < SY; s++) v[PIPE ? st & 1 : 0][s] = load_x(NK - 1 - st / NZR / ZG, st % NZR + st / NZR % ZG, s);
+        };
+        if (PIPE) plane(0);
+#pragma unroll
+        for (int st = 0; st < NG * NZR; st++) {
+            const int wg = st / NZR, zr = st % NZR;
+            if (zr == 0) {
+                if (AHEAD && NG > 2 && wg + 1 < NG) {
+                    load_w(wg + 1, a[(wg + 1) & 1]);
+                    if (wg + 2 == NG && more) fetch(nb, nc0);
                 }
+                if (!AHEAD && wg > 0) load_w(wg, a[0]);
+            }
+            if (PIPE && st + 1 < NG * NZR) plane(st + 1);
+            if (PIPE || zr == 0) __builtin_amdgcn_sched_barrier(0);
+            if (!PIPE) plane(st);
+#pragma unroll
+            for (int s = 0; s < SY; s++)
+#pragma unroll
+                for (int i = 0; i < NDZ; i++)
+#pragma unroll
+                    for (int dyo = 0; dyo < 3; dyo++) {
+                        const int jz = zr - i, jt = s - dyo;
+                        if (jz < 0 || jz >= RZ || jt < 0 || jt % YT || jt / YT >= RY) continue;
+#pragma unroll
+                        for (int n = 0; n < NCO; n++)
+                            acc[jz][jt / YT][n] = mfma(a[AHEAD ? wg & 1 : 0][i][dyo][n], v[PIPE ? st & 1 : 0][s], acc[jz][jt / YT][n]);
+                    }
         }
+    };
+
+    Block b = block_of(first);
+    if (AHEAD) fetch(b, 0);
+    for (uint32_t id = first; id < last; id++) {
+#pragma unroll
+        for (int i = 0; i < RZ; i++)
+#pragma unroll
+            for (int j = 0; j < RY; j++)
+#pragma unroll
+                for (int n = 0; n < NCO; n++) acc[i][j][n] = f32x4{0.f, 0.f, 0.f, 0.f};
+        const Block next = block_of(min(id + 1, last - 1));
+        f32x4 bv[NCO];
+#pragma unroll
+        for (int n = 0; n < NCO; n++) {
+            bv[n] = f32x4{0.f, 0.f, 0.f, 0.f};
+            if (bias)
+#pragma unroll
+                for (int r = 0; r < 4; r++) bv[n][r] = bias[b.co0 + n * 16 + 4 * grp + r];
+        }
+        for (int c0 = 0; c0 < cin;) {
+            const int cn = c0 + (cin - c0 >= 32 ? 32 : 16);
+            const bool end = cn >= cin, more = !end || id + 1 < last;
+            if (cn - c0 == 32)
+                slice(std::integral_constant<int, CM>{}, b, c0, end ? next : b, end ? 0 : cn, more);
+            else
+                slice(std::integral_constant<int, 16>{}, b, c0, end ? next : b, end ? 0 : cn, more);
+            c0 = cn;
+        }
+        const bool relu = flags & kRelu, f32out = flags & kOutF32;
+#pragma unroll
+        for (int jz = 0; jz < RZ; jz++)
+#pragma unroll
+            for (int jy = 0; jy < RY; jy++) {
+                const int gz = b.z0 + wz * RZ + jz, gy = b.y0 + (wy * RY + jy) * YT;
+                if (gz >= g.D || gy + ly >= g.H) continue;
+                const size_t v = (((size_t)b.smp * g.D + gz) * g.H + gy) * g.W + b.x0 + wx * WX;
+#pragma unroll
+                for (int n = 0; n < NCO; n++) {
+                    f32x4 o = acc[jz][jy][n];
+                    if (bias) o += bv[n];
+                    if (relu)
+#pragma unroll
+                        for (int r = 0; r < 4; r++) o[r] = o[r] > 0.f ? o[r] : 0.f;
+                    put4(y, mask, v * cout + b.co0 + n * 16, (uint32_t)((ly * g.W + lx) * cout + 4 * grp), o, f32out);
+                }
+            }
+        b = next;
+    }
+}
+
+// 3^3 forward (and backward-data) of a 16-channel input, rows of >= 32 voxels:
+// the multiply-adds per voxel are too few there to hide a block's staging, so
+// 8 wavefronts march along y over 8 z rows of 32 voxels instead.  The weights
+// of a 16-channel output block stay in registers (18 K steps: per (dz, dy)
+// the taps dx = -1, 0 of a voxel pair, then dx = 1), each x row is staged
+// once, two rows ahead, and adds to the three output rows it reaches, whose
+// accumulators turn with it.  The columns (x segment, 8 z rows, sample) times
+// H rows are cut evenly into `splits` runs, one workgroup a CU.
+// Bound: HBM (16 -> 16 reads and writes each voxel once) and the stores.
+// Measured (MI355X, 64^3, batch 8): 16 -> 16 52 us, 16 -> 48 134 us (before,
+// block by block: 67 and 227 us; k_fwd_blk's form: 75 and 172 us).
+__global__ void __launch_bounds__(512)
+    k_fwd_y16(const uint16_t* __restrict__ x, const uint16_t* __restrict__ w, const float* __restrict__ bias,
+              const uint16_t* __restrict__ mask, void* __restrict__ y, Geo g, int cout, int flags, uint32_t rows,
+              uint32_t rows_per_split)
+{
+    constexpr int TZ = 8, XV = 34, PIECES = (TZ + 2) * XV * 2, NJ = (PIECES + 511) / 512, BUF = PIECES * 8 + 16;
+    __shared__ __attribute__((aligned(16))) uint16_t lds[2 * BUF];
+    const int tid = (int)threadIdx.x, lane = tid & 63;
+    const int wave = __builtin_amdgcn_readfirstlane(tid >> 6);
+    const int r16 = lane & 15, grp = lane >> 4;
+    // the channel blocks of one run side by side on one XCD
+    const uint32_t id = xcd_remap(blockIdx.x, gridDim.x), ncb = (uint32_t)cout / 16u;
+    const int co0 = (int)(id % ncb) * 16;
+    const uint32_t split = id / ncb;
+    const int nxs = g.W / 32, nzb = (g.D + TZ - 1) / TZ;
+    const bool relu = flags & kRelu, f32out = flags & kOutF32, half = grp >= 2;
+    bf16x8 a[3][3][2];
+    f32x4 bv = f32x4{0.f, 0.f, 0.f, 0.f};
+#pragma unroll
+    for (int dz = 0; dz < 3; dz++)
+#pragma unroll
+        for (int dyo = 0; dyo < 3; dyo++)
+#pragma unroll
+            for (int kx = 0; kx < 2; kx++)
+                a[dz][dyo][kx] = kx == 1 && half ? bf16x8{}
+                                                 : ld8(w + (size_t)(co0 * 27 + (dz * 3 + dyo) * 3 + 2 * kx) * 16 +
+                                                       (uint32_t)(r16 * 27 * 16 + 8 * grp));
+    if (bias)
+#pragma unroll
+        for (int r = 0; r < 4; r++) bv[r] = bias[co0 + 4 * grp + r];
+
+    const uint32_t r1 = min(rows, (split + 1) * rows_per_split);
+    for (uint32_t r = split * rows_per_split; r < r1;) {
+        const uint32_t colm = r / (uint32_t)g.H;
+        const int ya = (int)(r % (uint32_t)g.H);
+        const int yb = min(g.H, ya + (int)(r1 - r));
+        r += (uint32_t)(yb - ya);
+        const int x0 = (int)(colm % (uint32_t)nxs) * 32, z0 = (int)((colm / (uint32_t)nxs) % (uint32_t)nzb) * TZ;
+        const uint32_t smp = colm / (uint32_t)(nxs * nzb);
+        const uint32_t sv = smp * (uint32_t)g.D;
+        uint32_t off[NJ];
+        bool ok[NJ];
+#pragma unroll
+        for (int j = 0; j < NJ; j++) {
+            const int p = tid + 512 * j, hv = p >> 1, gx = x0 - 1 + hv % XV, gz = z0 - 1 + hv / XV;
+            ok[j] = p < PIECES && (unsigned)gx < (unsigned)g.W && (unsigned)gz < (unsigned)g.D;
+            off[j] = ((sv + (uint32_t)gz) * (uint32_t)(g.H * g.W) + (uint32_t)gx) * 16u + 8u * (uint32_t)(p & 1);
+        }
+        uint4 R[3][NJ];
+        auto fetch = [&](int s, uint4* q) __attribute__((always_inline)) {
+            const bool in = s <= yb && (unsigned)s < (unsigned)g.H;
+#pragma unroll
+            for (int j = 0; j < NJ; j++)
+                q[j] = in && ok[j] ? *reinterpret_cast<const uint4*>(x + (size_t)(s * g.W * 16) + off[j])
+                                   : uint4{0u, 0u, 0u, 0u};
+        };
+        auto put = [&](int buf, const uint4* q) __attribute__((always_inline)) {
+#pragma unroll
+            for (int j = 0; j < NJ; j++)
+                if (tid + 512 * j < PIECES) *reinterpret_cast<uint4*>(lds + buf * BUF + (tid + 512 * j) * 8) = q[j];
+        };
+        const int zw = z0 + wave;
+        f32x4 acc[3][2];                                      // [output row slot][x tile]
+#pragma unroll
+        for (int k = 0; k < 3; k++) acc[k][0] = acc[k][1] = f32x4{0.f, 0.f, 0.f, 0.f};
+        // x row s; slots: output row s + 1 in ph, s in ph + 2, s - 1 in ph + 1 (mod 3)
+        auto step = [&](auto phase, int s, int buf) __attribute__((always_inline)) {
+            constexpr int ph = decltype(phase)::value;
+            fetch(s + 3, R[ph]);
+            acc[ph][0] = acc[ph][1] = f32x4{0.f, 0.f, 0.f, 0.f};
+            if (zw < g.D) {
+                if ((unsigned)s < (unsigned)g.H) {
+                    const uint16_t* L = lds + buf * BUF + (wave * XV + r16) * 16 + 8 * grp;
+#pragma unroll
+                    for (int dz = 2; dz >= 0; dz--)
+#pragma unroll
+                        for (int xt = 0; xt < 2; xt++)
+#pragma unroll
+                            for (int kx = 0; kx < 2; kx++) {
+                                bf16x8 v = ld8(L + (dz * XV + xt * 16 + 2 * kx) * 16);
+                                if (kx == 1 && half) v = bf16x8{};
+#pragma unroll
+                                for (int dyo = 0; dyo < 3; dyo++) {
+                                    f32x4& c = acc[dyo == 0 ? ph : dyo == 1 ? (ph + 2) % 3 : (ph + 1) % 3][xt];
+                                    c = mfma(a[dz][dyo][kx], v, c);
+                                }
+                            }
+                }
+                if (s > ya) {                                 // output row s - 1 is complete
+                    const size_t v = ((size_t)(sv + (uint32_t)zw) * g.H + (s - 1)) * g.W + x0;
+#pragma unroll
+                    for (int xt = 0; xt < 2; xt++) {
+                        f32x4 o = acc[(ph + 1) % 3][xt];
+                        if (bias) o += bv;
+                        if (relu)
+#pragma unroll
+                            for (int q = 0; q < 4; q++) o[q] = o[q] > 0.f ? o[q] : 0.f;
+                        put4(y, mask, (v + 16 * xt) * cout + co0, (uint32_t)(r16 * cout + 4 * grp), o, f32out);
+                    }
+                }
+            }
+            put(buf ^ 1, R[(ph + 1) % 3]);
+            __syncthreads();
+        };
+        const int s0 = ya - 1;
+        fetch(s0, R[0]);
+        fetch(s0 + 1, R[1]);
+        fetch(s0 + 2, R[2]);
+        put(0, R[0]);
+        __syncthreads();
+        int buf = 0;
+        for (int s = s0; s <= yb;) {
+            step(std::integral_constant<int, 0>{}, s, buf);
+            buf ^= 1;
+            if (++s > yb) break;
+            step(std::integral_constant<int, 1>{}, s, buf);
+            buf ^= 1;
+            if (++s > yb) break;
+            step(std::integral_constant<int, 2>{}, s, buf);
+            buf ^= 1;
+            ++s;
+        }
+        __syncthreads();
     }
 }
 
@@ -781,30 +1109,57 @@ int tiles_of(int c16, int cap)
     return 1;
 }
 
-int launch_fwd(const Shape& s, const uint16_t* x, const uint16_t* w, const float* bias, void* y,
-               int flags, hipStream_t st)
+int launch_fwd(const Shape& s, const uint16_t* x, const uint16_t* w, const float* bias, const uint16_t* mask,
+               void* y, int flags, hipStream_t st)
 {
     const Geo g = geo_of(s);
     if (g.V == 0) return NX_OK;
-    // LDS-tiled kernel: 3^3, rows of >= 32 voxels, blocks of 32 x 4 x 4
-    if (s.ks == 3 && s.w >= 32 && s.h >= 4 && s.d >= 4) {
-        const int nt = tiles_of(s.cout / 16, 4);
-        const dim3 grid((unsigned)((size_t)s.n * (s.d / 4) * (s.h / 4) * (s.w / 32)),
-                        (unsigned)(s.cout / (16 * nt)));
-        auto go = [&](auto NTc) {
-            constexpr int NT = decltype(NTc)::value;
-            if (s.cin == 16)
-                hipLaunchKernelGGL((k_fwd_tile<NT, 16>), grid, dim3(256), 0, st, x, w, bias, y, g, s.cin, s.cout,
-                                   flags);
-            else
-                hipLaunchKernelGGL((k_fwd_tile<NT, 0>), grid, dim3(256), 0, st, x, w, bias, y, g, s.cin, s.cout,
-                                   flags);
+    if (s.ks == 3 && s.w >= 32 && s.cin == 16) {
+        const uint32_t cb = (uint32_t)s.cout / 16u;
+        const uint32_t rows = (uint32_t)((s.w / 32) * ((s.d + 7) / 8)) * (uint32_t)s.n * (uint32_t)s.h;
+        const uint32_t splits = std::max(1u, std::min(256u / cb, rows)), per = (rows + splits - 1) / splits;
+        hipLaunchKernelGGL(k_fwd_y16, dim3((rows + per - 1) / per * cb), dim3(512), 0, st, x, w, bias, mask, y, g,
+                           s.cout, flags, rows, per);
+        return NX_OK;
+    }
+    // rows of >= 4 voxels: the block kernel.  Its block follows the row's
+    // length, smaller per wavefront on small grids (which would leave CUs
+    // idle); two channel blocks a wavefront where cout allows it (three or
+    // four leave no registers for the loads).  Blocks of small grids load the
+    // next slice ahead; the large block's slice would not fit the registers,
+    // there the second workgroup of the CU hides the staging.
+    if (s.ks == 3 && s.w >= 4) {
+        auto go = [&](auto WX, auto NXW, auto NYW, auto NZW, auto RY, auto RZ, auto NCO, auto AHEAD) {
+            constexpr int wx = decltype(WX)::value, nx_ = decltype(NXW)::value, ny = decltype(NYW)::value,
+                          nz = decltype(NZW)::value, ry = decltype(RY)::value, rz = decltype(RZ)::value,
+                          nc = decltype(NCO)::value;
+            constexpr bool ahead = decltype(AHEAD)::value;
+            constexpr int bx = nx_ * wx, by = ny * (16 / wx) * ry, bz = nz * rz;
+            const unsigned n = (unsigned)(s.n * (s.w / bx) * ((s.h + by - 1) / by) * ((s.d + bz - 1) / bz)) *
+                               (unsigned)(s.cout / (16 * nc));
+            const unsigned per = (n + 511u) / 512u;  // two workgroups per CU
+            hipLaunchKernelGGL((k_fwd_blk<wx, nx_, ny, nz, ry, rz, nc, ahead>), dim3((n + per - 1) / per), dim3(256), 0,
+                               st, x, w, bias, mask, y, g, s.cin, s.cout, flags, n, per);
         };
-        switch (nt) {
-            case 4: go(std::integral_constant<int, 4>{}); break;
-            case 3: go(std::integral_constant<int, 3>{}); break;
-            case 2: go(std::integral_constant<int, 2>{}); break;
-            default: go(std::integral_constant<int, 1>{}); break;
+        using std::integral_constant;
+        const integral_constant<int, 1> i1{};
+        const integral_constant<int, 2> i2{};
+        const integral_constant<int, 4> i4{};
+        const integral_constant<int, 8> i8{};
+        const integral_constant<int, 16> i16{};
+        const std::true_type yes{};
+        const std::false_type no{};
+        const bool even = s.cout % 32 == 0;
+        if (s.w >= 32) {
+            if (even) go(i16, i2, i1, i2, i4, i2, i2, no);
+            else go(i16, i2, i1, i2, i4, i2, i1, no);
+        } else if (s.w == 16) {
+            if (even) go(i16, i1, i2, i2, i2, i2, i2, yes);
+            else go(i16, i1, i2, i2, i2, i2, i1, yes);
+        } else if (s.w == 8) {
+            go(i8, i1, i2, i2, i1, i2, i1, yes);
+        } else {
+            go(i4, i1, i1, i4, i1, i1, i1, yes);
         }
         return NX_OK;
     }
@@ -875,7 +1230,7 @@ int check(const Shape& s)
 int fwd(const Shape& s, const uint16_t* x, const uint16_t* w, const float* bias, void* y, int flags,
         hipStream_t st)
 {
-    if (int e = launch_fwd(s, x, w, bias, y, flags, st)) return e;
+    if (int e = launch_fwd(s, x, w, bias, nullptr, y, flags, st)) return e;
     NX_CHECK_LAUNCH("k_fwd");
     return NX_OK;
 }
@@ -896,7 +1251,7 @@ int bwd_data(const Shape& s, const uint16_t* dy, const uint16_t* wt, void* dx, i
     Shape t = s;
     t.cin = s.cout;
     t.cout = s.cin;
-    if (int e = launch_fwd(t, dy, wt, nullptr, dx, flags & kOutF32, st)) return e;
+    if (int e = launch_fwd(t, dy, wt, nullptr, nullptr, dx, flags & kOutF32, st)) return e;
     NX_CHECK_LAUNCH("k_fwd (bwd-data)");
     return NX_OK;
 }
