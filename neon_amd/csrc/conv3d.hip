@@ -55,6 +55,9 @@ __device__ __forceinline__ f32x4 mfma(bf16x8 a, bf16x8 b, f32x4 c)
     return __builtin_amdgcn_mfma_f32_16x16x32_bf16(a, b, c, 0, 0, 0);
 }
 
+// a bf16 value > 0 (or NaN without sign): ReLU passes its gradient
+__device__ __forceinline__ bool positive(uint16_t h) { return (h & 0x8000u) == 0 && (h & 0x7fffu) != 0; }
+
 // Four consecutive channels of a voxel at element i + o of y (i the same for
 // the whole wavefront); mask as in k_fwd_blk.
 __device__ __forceinline__ void put4(void* y, const uint16_t* mask, size_t i, uint32_t o, f32x4 v, bool f32out)
@@ -71,7 +74,7 @@ __device__ __forceinline__ void put4(void* y, const uint16_t* mask, size_t i, ui
         const u16x4 m = *reinterpret_cast<const u16x4*>(mask + i + o);
 #pragma unroll
         for (int r = 0; r < 4; r++)
-            if ((m[r] & 0x8000u) != 0 || (m[r] & 0x7fffu) == 0) h[r] = 0;
+            if (!positive(m[r])) h[r] = 0;
     }
     __builtin_memcpy(static_cast<uint16_t*>(y) + i + o, &h, 8);
 }
@@ -88,14 +91,80 @@ __device__ __forceinline__ void tap_offset(int tap, int& dz, int& dy, int& dx)
     }
 }
 
-// One wave: 32 voxels x (16*NT) output channels; 4 waves per workgroup.
-// grid.y selects the block of 16*NT output channels.
-template <int NT, int KS>
+// 1^3 convolution: out[v][co] = sum_ci x[v][ci] w[co][ci] (and backward-data on
+// the flipped weights).  A wavefront takes 64 voxels x 16 NCO output channels;
+// M = channels (A: weights), N = voxels (B: 16 bytes of a voxel straight from
+// memory), so a lane ends with 4 consecutive channels of a voxel.  Bound by
+// HBM.  Stores the first `keep` channels, `keep` apart, where that is not cout.
+// Measured (MI355X, 64^3, batch 8, 16 -> 16): 23 us (float, 4 of 16 channels
+// kept), 32 us backward (before, one 2- or 4-byte store per channel and all 16
+// floats of a voxel: 36 and 36 us).
+template <int NCO>
 __global__ void __launch_bounds__(256)
-    k_fwd(const uint16_t* __restrict__ x, const uint16_t* __restrict__ w,
-          const float* __restrict__ bias, void* __restrict__ y, Geo g, int cin, int cout, int flags)
+    k_pw(const uint16_t* __restrict__ x, const uint16_t* __restrict__ w, const float* __restrict__ bias,
+         const uint16_t* __restrict__ mask, void* __restrict__ y, uint32_t V, int cin, int cout, int flags, int keep)
 {
-    constexpr int T = KS * KS * KS;
+    const int lane = threadIdx.x & 63, wave = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
+    const int r16 = lane & 15, grp = lane >> 4;
+    const uint32_t v0 = (blockIdx.x * 4u + (uint32_t)wave) * 64u;
+    if (v0 >= V) return;  // whole wave
+    const int co0 = (int)blockIdx.y * 16 * NCO;
+    f32x4 acc[4][NCO];
+#pragma unroll
+    for (int t = 0; t < 4; t++)
+#pragma unroll
+        for (int n = 0; n < NCO; n++) acc[t][n] = f32x4{0.f, 0.f, 0.f, 0.f};
+    for (int c0 = 0; c0 < cin; c0 += 32) {
+        const bool in = c0 + 8 * grp < cin;
+        bf16x8 a[NCO], b[4];
+#pragma unroll
+        for (int t = 0; t < 4; t++)
+            b[t] = in && v0 + 16 * t + r16 < V ? ld8(x + (size_t)v0 * cin + (uint32_t)((16 * t + r16) * cin + c0 + 8 * grp))
+                                               : bf16x8{};
+#pragma unroll
+        for (int n = 0; n < NCO; n++)
+            a[n] = in ? ld8(w + (size_t)(co0 + 16 * n) * cin + (uint32_t)(r16 * cin + c0 + 8 * grp)) : bf16x8{};
+#pragma unroll
+        for (int t = 0; t < 4; t++)
+#pragma unroll
+            for (int n = 0; n < NCO; n++) acc[t][n] = mfma(a[n], b[t], acc[t][n]);
+    }
+    const bool relu = flags & kRelu, f32out = flags & kOutF32;
+#pragma unroll
+    for (int n = 0; n < NCO; n++) {
+        const int co = co0 + 16 * n + 4 * grp;
+        f32x4 bv = f32x4{0.f, 0.f, 0.f, 0.f};
+        if (bias)
+#pragma unroll
+            for (int r = 0; r < 4; r++) bv[r] = bias[co + r];
+#pragma unroll
+        for (int t = 0; t < 4; t++) {
+            if (v0 + 16 * t + r16 >= V) continue;
+            f32x4 o = acc[t][n];
+            if (bias) o += bv;
+            if (relu)
+#pragma unroll
+                for (int r = 0; r < 4; r++) o[r] = o[r] > 0.f ? o[r] : 0.f;
+            if (keep == cout) {
+                put4(y, mask, (size_t)v0 * cout + co0 + 16 * n, (uint32_t)((16 * t + r16) * cout + 4 * grp), o, f32out);
+            } else if (co < keep) {
+                float* p = static_cast<float*>(y) + (size_t)(v0 + 16 * t + r16) * keep + co;
+#pragma unroll
+                for (int r = 0; r < 4; r++)
+                    if (co + r < keep) p[r] = o[r];
+            }
+        }
+    }
+}
+
+// 3^3 on rows of 1 or 2 voxels.  One wave: 32 voxels x (16*NT) output
+// channels; 4 waves per workgroup.  grid.y selects the block of 16*NT output channels.
+template <int NT>
+__global__ void __launch_bounds__(256)
+    k_fwd(const uint16_t* __restrict__ x, const uint16_t* __restrict__ w, const float* __restrict__ bias,
+          const uint16_t* __restrict__ mask, void* __restrict__ y, Geo g, int cin, int cout, int flags)
+{
+    constexpr int T = 27;
     const int K = T * cin, KC = (K + 31) / 32;
     const int lane = threadIdx.x & 63, wave = threadIdx.x >> 6;
     const int r16 = lane & 15, grp = lane >> 4;
@@ -134,7 +203,7 @@ __global__ void __launch_bounds__(256)
         const int kk = kc * 32 + 8 * grp;
         if (kk < K) {
             int dz, dy, dx;
-            tap_offset<KS>(tap, dz, dy, dx);
+            tap_offset<3>(tap, dz, dy, dx);
             const int off = (dz * g.H + dy) * g.W + dx;
 #pragma unroll
             for (int t = 0; t < 2; t++) {
@@ -187,7 +256,8 @@ __global__ void __launch_bounds__(256)
                 if (f32out)
                     static_cast<float*>(y)[(size_t)v * cout + co] = s;
                 else
-                    static_cast<uint16_t*>(y)[(size_t)v * cout + co] = f2bf(s);
+                    static_cast<uint16_t*>(y)[(size_t)v * cout + co] =
+                        mask && !positive(mask[(size_t)v * cout + co]) ? (uint16_t)0 : f2bf(s);
             }
     }
 }
@@ -1065,16 +1135,20 @@ __global__ void __launch_bounds__(256)
     }
 }
 
+// grid.y selects the convolution of the table
 __global__ void __launch_bounds__(256)
-    k_flip(const uint16_t* __restrict__ w, uint16_t* __restrict__ wt, int T, int cin, int cout)
+    k_flip(const uint16_t* __restrict__ w_all, uint16_t* __restrict__ wt_all, FlipTable tab)
 {
-    const size_t n = (size_t)cout * T * cin;
-    for (size_t i = (size_t)blockIdx.x * 256 + threadIdx.x; i < n; i += (size_t)gridDim.x * 256) {
+    const FlipEntry f = tab.e[blockIdx.y];
+    const uint16_t* w = w_all + f.off;
+    uint16_t* wt = wt_all + f.off;
+    const uint32_t n = (uint32_t)(f.cout * f.taps * f.cin);
+    for (uint32_t i = blockIdx.x * 256 + threadIdx.x; i < n; i += gridDim.x * 256) {
         // i indexes wt[ci][tap][co]
-        const int co = (int)(i % cout);
-        const int tap = (int)((i / cout) % T);
-        const int ci = (int)(i / ((size_t)cout * T));
-        wt[i] = w[((size_t)co * T + (T - 1 - tap)) * cin + ci];
+        const int co = (int)(i % (uint32_t)f.cout);
+        const int tap = (int)((i / (uint32_t)f.cout) % (uint32_t)f.taps);
+        const int ci = (int)(i / (uint32_t)(f.cout * f.taps));
+        wt[i] = w[((uint32_t)co * f.taps + (f.taps - 1 - tap)) * f.cin + ci];
     }
 }
 
@@ -1110,11 +1184,26 @@ int tiles_of(int c16, int cap)
 }
 
 int launch_fwd(const Shape& s, const uint16_t* x, const uint16_t* w, const float* bias, const uint16_t* mask,
-               void* y, int flags, hipStream_t st)
+               void* y, int flags, int keep, hipStream_t st)
 {
     const Geo g = geo_of(s);
     if (g.V == 0) return NX_OK;
-    if (s.ks == 3 && s.w >= 32 && s.cin == 16) {
+    if (s.ks == 1) {
+        const int nco = tiles_of(s.cout / 16, 4);
+        const dim3 grid((g.V + 255u) / 256u, (unsigned)(s.cout / (16 * nco)));
+        auto go = [&](auto NCO) {
+            hipLaunchKernelGGL((k_pw<decltype(NCO)::value>), grid, dim3(256), 0, st, x, w, bias, mask, y, g.V, s.cin,
+                               s.cout, flags, keep);
+        };
+        switch (nco) {
+            case 4: go(std::integral_constant<int, 4>{}); break;
+            case 3: go(std::integral_constant<int, 3>{}); break;
+            case 2: go(std::integral_constant<int, 2>{}); break;
+            default: go(std::integral_constant<int, 1>{}); break;
+        }
+        return NX_OK;
+    }
+    if (s.w >= 32 && s.cin == 16) {
         const uint32_t cb = (uint32_t)s.cout / 16u;
         const uint32_t rows = (uint32_t)((s.w / 32) * ((s.d + 7) / 8)) * (uint32_t)s.n * (uint32_t)s.h;
         const uint32_t splits = std::max(1u, std::min(256u / cb, rows)), per = (rows + splits - 1) / splits;
@@ -1128,7 +1217,7 @@ int launch_fwd(const Shape& s, const uint16_t* x, const uint16_t* w, const float
     // four leave no registers for the loads).  Blocks of small grids load the
     // next slice ahead; the large block's slice would not fit the registers,
     // there the second workgroup of the CU hides the staging.
-    if (s.ks == 3 && s.w >= 4) {
+    if (s.w >= 4) {
         auto go = [&](auto WX, auto NXW, auto NYW, auto NZW, auto RY, auto RZ, auto NCO, auto AHEAD) {
             constexpr int wx = decltype(WX)::value, nx_ = decltype(NXW)::value, ny = decltype(NYW)::value,
                           nz = decltype(NZW)::value, ry = decltype(RY)::value, rz = decltype(RZ)::value,
@@ -1165,16 +1254,19 @@ int launch_fwd(const Shape& s, const uint16_t* x, const uint16_t* w, const float
     }
     const int nt = tiles_of(s.cout / 16, 8);
     const dim3 grid((g.V + 127u) / 128u, (unsigned)(s.cout / (16 * nt)));
-    return by_ks(s.ks, [&](auto KS) {
-        switch (nt) {
-            case 8: hipLaunchKernelGGL((k_fwd<8, KS>), grid, dim3(256), 0, st, x, w, bias, y, g, s.cin, s.cout, flags); break;
-            case 6: hipLaunchKernelGGL((k_fwd<6, KS>), grid, dim3(256), 0, st, x, w, bias, y, g, s.cin, s.cout, flags); break;
-            case 4: hipLaunchKernelGGL((k_fwd<4, KS>), grid, dim3(256), 0, st, x, w, bias, y, g, s.cin, s.cout, flags); break;
-            case 3: hipLaunchKernelGGL((k_fwd<3, KS>), grid, dim3(256), 0, st, x, w, bias, y, g, s.cin, s.cout, flags); break;
-            case 2: hipLaunchKernelGGL((k_fwd<2, KS>), grid, dim3(256), 0, st, x, w, bias, y, g, s.cin, s.cout, flags); break;
-            default: hipLaunchKernelGGL((k_fwd<1, KS>), grid, dim3(256), 0, st, x, w, bias, y, g, s.cin, s.cout, flags); break;
-        }
-    });
+    auto go = [&](auto NT) {
+        hipLaunchKernelGGL((k_fwd<decltype(NT)::value>), grid, dim3(256), 0, st, x, w, bias, mask, y, g, s.cin, s.cout,
+                           flags);
+    };
+    switch (nt) {
+        case 8: go(std::integral_constant<int, 8>{}); break;
+        case 6: go(std::integral_constant<int, 6>{}); break;
+        case 4: go(std::integral_constant<int, 4>{}); break;
+        case 3: go(std::integral_constant<int, 3>{}); break;
+        case 2: go(std::integral_constant<int, 2>{}); break;
+        default: go(std::integral_constant<int, 1>{}); break;
+    }
+    return NX_OK;
 }
 
 // How a weight gradient is cut up.  k_bwd_wy (3^3, rows of >= 4 voxels: its
@@ -1228,30 +1320,30 @@ int check(const Shape& s)
 }
 
 int fwd(const Shape& s, const uint16_t* x, const uint16_t* w, const float* bias, void* y, int flags,
-        hipStream_t st)
+        hipStream_t st, int keep)
 {
-    if (int e = launch_fwd(s, x, w, bias, nullptr, y, flags, st)) return e;
+    if (int e = launch_fwd(s, x, w, bias, nullptr, y, flags, keep ? keep : s.cout, st)) return e;
     NX_CHECK_LAUNCH("k_fwd");
     return NX_OK;
 }
 
-int flip(const Shape& s, const uint16_t* w, uint16_t* wt, hipStream_t st)
+int flip(const FlipTable& tab, const uint16_t* w, uint16_t* wt, hipStream_t st)
 {
-    const int T = s.ks * s.ks * s.ks;
-    const size_t n = (size_t)s.cout * T * s.cin;
-    hipLaunchKernelGGL(k_flip, dim3((unsigned)std::min<size_t>((n + 255) / 256, 4096)), dim3(256), 0,
-                       st, w, wt, T, s.cin, s.cout);
+    uint32_t most = 1;
+    for (int k = 0; k < tab.n; k++)
+        most = std::max(most, (uint32_t)(tab.e[k].cout * tab.e[k].taps * tab.e[k].cin));
+    hipLaunchKernelGGL(k_flip, dim3(std::min((most + 255u) / 256u, 4096u), (unsigned)tab.n), dim3(256), 0, st, w, wt, tab);
     NX_CHECK_LAUNCH("k_flip");
     return NX_OK;
 }
 
-int bwd_data(const Shape& s, const uint16_t* dy, const uint16_t* wt, void* dx, int flags,
+int bwd_data(const Shape& s, const uint16_t* dy, const uint16_t* wt, const uint16_t* mask, void* dx, int flags,
              hipStream_t st)
 {
     Shape t = s;
     t.cin = s.cout;
     t.cout = s.cin;
-    if (int e = launch_fwd(t, dy, wt, nullptr, nullptr, dx, flags & kOutF32, st)) return e;
+    if (int e = launch_fwd(t, dy, wt, nullptr, mask, dx, flags & kOutF32, s.cin, st)) return e;
     NX_CHECK_LAUNCH("k_fwd (bwd-data)");
     return NX_OK;
 }
@@ -1356,8 +1448,9 @@ int nx_conv3d_bwd_data_bf16(const uint16_t* dy, const uint16_t* w, void* dx, con
     void* ws = nullptr;
     const size_t nw = (size_t)cout * ksize * ksize * ksize * cin;
     if (int e = scratch(nw * sizeof(uint16_t), &ws)) return e;
-    if (int e = conv::flip(sh, w, static_cast<uint16_t*>(ws), (hipStream_t)s)) return e;
-    return conv::bwd_data(sh, dy, static_cast<uint16_t*>(ws), dx, flags & conv::kOutF32, (hipStream_t)s);
+    const conv::FlipTable tab{1, {{0, cin, cout, ksize * ksize * ksize}}};
+    if (int e = conv::flip(tab, w, static_cast<uint16_t*>(ws), (hipStream_t)s)) return e;
+    return conv::bwd_data(sh, dy, static_cast<uint16_t*>(ws), nullptr, dx, flags & conv::kOutF32, (hipStream_t)s);
 }
 
 int nx_conv3d_bwd_weight_bf16(const uint16_t* x, const uint16_t* dy, float* dw, float* db,

@@ -22,14 +22,26 @@ struct Shape {
 enum : int { kRelu = 1, kOutF32 = 2 };
 
 // y = conv(x, w) + bias (bias may be null), ReLU if flags & kRelu; y is bf16
-// or, with kOutF32, float.
+// or, with kOutF32, float.  keep (ks = 1 and float y only): store the first
+// `keep` channels, packed; 0: all.
 int fwd(const Shape& s, const uint16_t* x, const uint16_t* w, const float* bias, void* y, int flags,
-        hipStream_t st);
-// w (bf16 [cout][T][cin]) -> wt (bf16 [cin][T][cout], taps reversed): the
-// weights of the transposed convolution.
-int flip(const Shape& s, const uint16_t* w, uint16_t* wt, hipStream_t st);
+        hipStream_t st, int keep = 0);
+// w (bf16 [cout][T][cin]) -> wt (bf16 [cin][T][cout], taps reversed), the
+// weights of the transposed convolution, of every convolution of a table (one
+// launch); off: element offset in both arrays.
+struct FlipEntry {
+    uint32_t off;
+    int cin, cout, taps;
+};
+struct FlipTable {
+    int n;
+    FlipEntry e[16];
+};
+int flip(const FlipTable& tab, const uint16_t* w, uint16_t* wt, hipStream_t st);
 // dx = conv^T(dy, w) given the flipped weights wt; dx bf16 or float (kOutF32).
-int bwd_data(const Shape& s, const uint16_t* dy, const uint16_t* wt, void* dx, int flags,
+// mask (bf16 dx only): null, or activations of dx's shape; dx is 0 where they
+// are not positive (the ReLU below).
+int bwd_data(const Shape& s, const uint16_t* dy, const uint16_t* wt, const uint16_t* mask, void* dx, int flags,
              hipStream_t st);
 // dw[co][tap][ci] = sum_v dy[v][co] x[v + off(tap)][ci], db[co] = sum_v dy[v][co]
 // (db may be null).  ws: workspace of bwd_weight_ws(s) bytes.

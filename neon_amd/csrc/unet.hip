@@ -38,122 +38,145 @@ __device__ __forceinline__ float bf2f(uint16_t h) { return __builtin_bit_cast(fl
 #define GRID_STRIDE(i, n) \
     for (size_t i = (size_t)blockIdx.x * 256 + threadIdx.x; i < (n); i += (size_t)gridDim.x * 256)
 
+// The kernels between the convolutions move 8 channels (16 bytes) of a voxel
+// per thread (every channel count is a multiple of 16); all are bound by HBM.
+// With one channel a thread they were bound by their index divisions and
+// 2-byte accesses (64^3, batch 8, per training step: upcat 236 -> 70 us, the
+// loss 114 -> 37, skip gradients and up_bwd 145 -> 129 with the 337 us of
+// separate ReLU passes now inside them and the convolutions).
+// Element counts / 8 fit 32 bits (max_batch * size^3 * 256 < 2^31), which
+// keeps the index divisions short.
+typedef unsigned short u16x8 __attribute__((ext_vector_type(8)));
+
+__device__ __forceinline__ u16x8 ld8(const uint16_t* p) { return *reinterpret_cast<const u16x8*>(p); }
+__device__ __forceinline__ void st8(uint16_t* p, u16x8 v) { *reinterpret_cast<u16x8*>(p) = v; }
+__device__ __forceinline__ bool positive(uint16_t h) { return (h & 0x8000u) == 0 && (h & 0x7fffu) != 0; }
+
+// gradients that pass a ReLU: 0 where the activation is not positive
+__device__ __forceinline__ u16x8 relu_grad(u16x8 g, u16x8 act)
+{
+#pragma unroll
+    for (int k = 0; k < 8; k++)
+        if (!positive(act[k])) g[k] = 0;
+    return g;
+}
+
 __global__ void __launch_bounds__(256)
     k_pack_input(const float* __restrict__ x, uint16_t* __restrict__ out, size_t V, int in_ch)
 {
-    GRID_STRIDE(i, V * kC0)
+    GRID_STRIDE(v, V)
     {
-        const size_t v = i / kC0;
-        const int c = (int)(i % kC0);
-        out[i] = c < in_ch ? f2bf(x[v * in_ch + c]) : (uint16_t)0;
+        u16x8 o[2];
+#pragma unroll
+        for (int c = 0; c < kC0; c++) o[c >> 3][c & 7] = c < in_ch ? f2bf(x[v * in_ch + c]) : (uint16_t)0;
+        st8(out + v * kC0, o[0]);
+        st8(out + v * kC0 + 8, o[1]);
     }
 }
 
 // voxel index of (b, z, y, x) on a side-s cube and its parent on side s/2
-__device__ __forceinline__ size_t parent_of(size_t v, int ls)
+__device__ __forceinline__ uint32_t parent_of(uint32_t v, int ls)
 {
-    const size_t s = (size_t)1 << ls, h = s >> 1;
-    const size_t x = v & (s - 1), y = (v >> ls) & (s - 1), z = (v >> (2 * ls)) & (s - 1);
-    const size_t b = v >> (3 * ls);
+    const uint32_t s = 1u << ls, h = s >> 1;
+    const uint32_t x = v & (s - 1), y = (v >> ls) & (s - 1), z = (v >> (2 * ls)) & (s - 1), b = v >> (3 * ls);
     return ((b * h + (z >> 1)) * h + (y >> 1)) * h + (x >> 1);
+}
+
+// child k (bits z y x) of voxel vh of the side-2^(ls-1) cube
+__device__ __forceinline__ uint32_t child_of(uint32_t vh, int ls, int k)
+{
+    const uint32_t s = 1u << ls, lh = (uint32_t)ls - 1u, h = s >> 1;
+    const uint32_t x = vh & (h - 1), y = (vh >> lh) & (h - 1), z = (vh >> (2 * lh)) & (h - 1), b = vh >> (3 * lh);
+    return ((b * s + 2 * z + (k >> 2)) * s + 2 * y + ((k >> 1) & 1)) * s + 2 * x + (k & 1);
 }
 
 // out[b][z][y][x][c] = mean of the 2x2x2 children on the side-2h cube (ls = log2 of 2h)
 __global__ void __launch_bounds__(256)
-    k_pool(const uint16_t* __restrict__ in, uint16_t* __restrict__ out, size_t Vh, int ls, int C)
+    k_pool(const uint16_t* __restrict__ in, uint16_t* __restrict__ out, uint32_t Vh, int ls, uint32_t C8)
 {
-    const size_t s = (size_t)1 << ls, h = s >> 1;
-    GRID_STRIDE(i, Vh * C)
+    GRID_STRIDE(i, Vh * C8)
     {
-        const size_t vh = i / C;
-        const int c = (int)(i % C);
-        const size_t x = vh % h, y = (vh / h) % h, z = (vh / (h * h)) % h, b = vh / (h * h * h);
-        float acc = 0.f;
-        for (int k = 0; k < 8; k++) {
-            const size_t v = ((b * s + 2 * z + (k >> 2)) * s + 2 * y + ((k >> 1) & 1)) * s + 2 * x + (k & 1);
-            acc += bf2f(in[v * C + c]);
+        const uint32_t vh = (uint32_t)i / C8, c = (uint32_t)i % C8;
+        u16x8 q[8], o;
+#pragma unroll
+        for (int k = 0; k < 8; k++) q[k] = ld8(in + ((size_t)child_of(vh, ls, k) * C8 + c) * 8);
+#pragma unroll
+        for (int e = 0; e < 8; e++) {
+            float acc = 0.f;
+#pragma unroll
+            for (int k = 0; k < 8; k++) acc += bf2f(q[k][e]);
+            o[e] = f2bf(acc * 0.125f);
         }
-        out[i] = f2bf(acc * 0.125f);
+        st8(out + i * 8, o);
     }
 }
 
 // out[v] = [low[parent(v)] (Cu channels), skip[v] (Cs channels)]
 __global__ void __launch_bounds__(256)
     k_upcat(const uint16_t* __restrict__ low, const uint16_t* __restrict__ skip,
-            uint16_t* __restrict__ out, size_t V, int ls, int Cu, int Cs)
+            uint16_t* __restrict__ out, uint32_t V, int ls, uint32_t Cu8, uint32_t Cs8)
 {
-    const int Cc = Cu + Cs;
-    GRID_STRIDE(i, V * Cc)
+    const uint32_t Cc8 = Cu8 + Cs8;
+    GRID_STRIDE(i, V * Cc8)
     {
-        const size_t v = i / Cc;
-        const int c = (int)(i % Cc);
-        out[i] = c < Cu ? low[parent_of(v, ls) * Cu + c] : skip[v * Cs + (c - Cu)];
+        const uint32_t v = (uint32_t)i / Cc8, c = (uint32_t)i % Cc8;
+        st8(out + i * 8, ld8(c < Cu8 ? low + ((size_t)parent_of(v, ls) * Cu8 + c) * 8
+                                     : skip + ((size_t)v * Cs8 + (c - Cu8)) * 8));
     }
 }
 
-// gradient through upsampling: out[vh][c] = sum over the 8 children of g[child][c], c < Cu
+// gradient through upsampling and the ReLU of the layer below: out[vh][c] =
+// sum over the 8 children of g[child][c], c < Cu, where act[vh][c] > 0
 __global__ void __launch_bounds__(256)
-    k_up_bwd(const uint16_t* __restrict__ g, uint16_t* __restrict__ out, size_t Vh, int ls, int Cc,
-             int Cu)
+    k_up_bwd(const uint16_t* __restrict__ g, const uint16_t* __restrict__ act, uint16_t* __restrict__ out, uint32_t Vh,
+             int ls, uint32_t Cc8, uint32_t Cu8)
 {
-    const size_t s = (size_t)1 << ls, h = s >> 1;
-    GRID_STRIDE(i, Vh * Cu)
+    GRID_STRIDE(i, Vh * Cu8)
     {
-        const size_t vh = i / Cu;
-        const int c = (int)(i % Cu);
-        const size_t x = vh % h, y = (vh / h) % h, z = (vh / (h * h)) % h, b = vh / (h * h * h);
-        float acc = 0.f;
-        for (int k = 0; k < 8; k++) {
-            const size_t v = ((b * s + 2 * z + (k >> 2)) * s + 2 * y + ((k >> 1) & 1)) * s + 2 * x + (k & 1);
-            acc += bf2f(g[v * Cc + c]);
+        const uint32_t vh = (uint32_t)i / Cu8, c = (uint32_t)i % Cu8;
+        u16x8 q[8], o;
+#pragma unroll
+        for (int k = 0; k < 8; k++) q[k] = ld8(g + ((size_t)child_of(vh, ls, k) * Cc8 + c) * 8);
+#pragma unroll
+        for (int e = 0; e < 8; e++) {
+            float acc = 0.f;
+#pragma unroll
+            for (int k = 0; k < 8; k++) acc += bf2f(q[k][e]);
+            o[e] = f2bf(acc);
         }
-        out[i] = f2bf(acc);
+        st8(out + i * 8, relu_grad(o, ld8(act + i * 8)));
     }
 }
 
-// gradient of a skip tensor e_l: its slice of the concatenation gradient plus
-// the pooling gradient gin_next[parent]/8
+// gradient of a skip tensor e_l through its ReLU: its slice (from channel
+// 8 off8) of the concatenation gradient plus the pooling gradient
+// gin_next[parent]/8, where act = e_l > 0
 __global__ void __launch_bounds__(256)
-    k_skip_grad(const uint16_t* __restrict__ gcat, int Cc, int off, const uint16_t* __restrict__ gnext,
-                uint16_t* __restrict__ out, size_t V, int ls, int C)
+    k_skip_grad(const uint16_t* __restrict__ gcat, uint32_t Cc8, uint32_t off8, const uint16_t* __restrict__ gnext,
+                const uint16_t* __restrict__ act, uint16_t* __restrict__ out, uint32_t V, int ls, uint32_t C8)
 {
-    GRID_STRIDE(i, V * C)
+    GRID_STRIDE(i, V * C8)
     {
-        const size_t v = i / C;
-        const int c = (int)(i % C);
-        const float a = bf2f(gcat[v * Cc + off + c]);
-        const float b = bf2f(gnext[parent_of(v, ls) * C + c]);
-        out[i] = f2bf(a + b * 0.125f);
-    }
-}
-
-__global__ void __launch_bounds__(256)
-    k_relu_bwd(const uint16_t* __restrict__ y, const uint16_t* __restrict__ g, uint16_t* __restrict__ out,
-               size_t n)
-{
-    GRID_STRIDE(i, n)
-    {
-        const uint16_t h = y[i];
-        out[i] = ((h & 0x8000u) == 0 && (h & 0x7fffu) != 0) ? g[i] : (uint16_t)0;
-    }
-}
-
-__global__ void __launch_bounds__(256)
-    k_unpack_output(const float* __restrict__ o, float* __restrict__ y, size_t V, int oc)
-{
-    GRID_STRIDE(i, V * oc)
-    {
-        y[i] = o[(i / oc) * kC0 + i % oc];
+        const uint32_t v = (uint32_t)i / C8, c = (uint32_t)i % C8;
+        const u16x8 a = ld8(gcat + ((size_t)v * Cc8 + off8 + c) * 8);
+        const u16x8 b = ld8(gnext + ((size_t)parent_of(v, ls) * C8 + c) * 8);
+        u16x8 o;
+#pragma unroll
+        for (int e = 0; e < 8; e++) o[e] = f2bf(bf2f(a[e]) + bf2f(b[e]) * 0.125f);
+        st8(out + i * 8, relu_grad(o, ld8(act + i * 8)));
     }
 }
 
 __global__ void __launch_bounds__(256)
     k_pack_grad(const float* __restrict__ dy, uint16_t* __restrict__ g, size_t V, int oc)
 {
-    GRID_STRIDE(i, V * kC0)
+    GRID_STRIDE(v, V)
     {
-        const int c = (int)(i % kC0);
-        g[i] = c < oc ? f2bf(dy[(i / kC0) * oc + c]) : (uint16_t)0;
+        u16x8 o[2];
+#pragma unroll
+        for (int c = 0; c < kC0; c++) o[c >> 3][c & 7] = c < oc ? f2bf(dy[v * oc + c]) : (uint16_t)0;
+        st8(g + v * kC0, o[0]);
+        st8(g + v * kC0 + 8, o[1]);
     }
 }
 
@@ -166,15 +189,18 @@ __global__ void __launch_bounds__(256)
     double acc[1] = {0.0};
     for (size_t v = (size_t)blockIdx.x * 256 + threadIdx.x; v < V; v += (size_t)gridDim.x * 256) {
         const float w = wgt[v];
+        u16x8 gv[2];
+#pragma unroll
         for (int c = 0; c < kC0; c++) {
-            float gv = 0.f;
+            gv[c >> 3][c & 7] = 0;
             if (c < oc) {
-                const float d = o[v * kC0 + c] - t[v * oc + c];
+                const float d = o[v * oc + c] - t[v * oc + c];
                 acc[0] += (double)w * (double)d * (double)d;
-                gv = 2.f * w * d;
+                gv[c >> 3][c & 7] = f2bf(2.f * w * d);
             }
-            g[v * kC0 + c] = f2bf(gv);
         }
+        st8(g + v * kC0, gv[0]);
+        st8(g + v * kC0 + 8, gv[1]);
     }
     block_sum_f64<1>(acc, lds);
     if (threadIdx.x == 0) part[blockIdx.x] = acc[0];
@@ -282,58 +308,51 @@ struct Rng {
     }
 };
 
-int conv_fwd(nx_unet_s* u, int ci, int b, const uint16_t* x, void* y, int flags, hipStream_t st)
+int conv_fwd(nx_unet_s* u, int ci, int b, const uint16_t* x, void* y, int flags, hipStream_t st, int keep = 0)
 {
     const ConvSpec& c = u->convs[ci];
-    return conv::fwd(u->shape(ci, b), x, u->wbf + c.w_off, u->w32 + c.b_off, y, flags, st);
+    return conv::fwd(u->shape(ci, b), x, u->wbf + c.w_off, u->w32 + c.b_off, y, flags, st, keep);
 }
 
-int conv_bwd(nx_unet_s* u, int ci, int b, const uint16_t* x, const uint16_t* gy, uint16_t* gx,
+// act: null, or the activations below gx whose ReLU the gradient passes
+int conv_bwd(nx_unet_s* u, int ci, int b, const uint16_t* x, const uint16_t* gy, const uint16_t* act, uint16_t* gx,
              hipStream_t st)
 {
     const ConvSpec& c = u->convs[ci];
     const conv::Shape s = u->shape(ci, b);
     if (int e = conv::bwd_weight(s, x, gy, u->g32 + c.w_off, u->g32 + c.b_off, u->ws, st)) return e;
-    if (gx) return conv::bwd_data(s, gy, u->wt + c.w_off, gx, 0, st);
+    if (gx) return conv::bwd_data(s, gy, u->wt + c.w_off, act, gx, 0, st);
     return NX_OK;
 }
 
-int relu_bwd(const uint16_t* y, const uint16_t* g, uint16_t* out, size_t n, hipStream_t st)
-{
-    hipLaunchKernelGGL(k_relu_bwd, dim3(blocks_for(n)), dim3(256), 0, st, y, g, out, n);
-    NX_CHECK_LAUNCH("k_relu_bwd");
-    return NX_OK;
-}
-
-int forward(nx_unet_s* u, const float* x, int b, hipStream_t st)
+// the network's output, out_ch floats a voxel, to y
+int forward(nx_unet_s* u, const float* x, int b, float* y, hipStream_t st)
 {
     const int L = u->L;
     const size_t V0 = u->vox(0, b);
-    hipLaunchKernelGGL(k_pack_input, dim3(blocks_for(V0 * kC0)), dim3(256), 0, st, x, u->in[0], V0,
-                       u->d.in_ch);
+    hipLaunchKernelGGL(k_pack_input, dim3(blocks_for(V0)), dim3(256), 0, st, x, u->in[0], V0, u->d.in_ch);
     NX_CHECK_LAUNCH("k_pack_input");
     for (int l = 0; l < L; l++) {
         if (int e = conv_fwd(u, u->enc(l, 0), b, u->in[l], u->a[l], conv::kRelu, st)) return e;
         if (int e = conv_fwd(u, u->enc(l, 1), b, u->a[l], u->e[l], conv::kRelu, st)) return e;
         if (l < L - 1) {
-            const size_t Vh = u->vox(l + 1, b);
-            hipLaunchKernelGGL(k_pool, dim3(blocks_for(Vh * u->wd[l])), dim3(256), 0, st, u->e[l],
-                               u->in[l + 1], Vh, u->ls0 - l, u->wd[l]);
+            const uint32_t Vh = (uint32_t)u->vox(l + 1, b), C8 = (uint32_t)u->wd[l] / 8;
+            hipLaunchKernelGGL(k_pool, dim3(blocks_for((size_t)Vh * C8)), dim3(256), 0, st, u->e[l], u->in[l + 1], Vh,
+                               u->ls0 - l, C8);
             NX_CHECK_LAUNCH("k_pool");
         }
     }
     const uint16_t* low = u->e[L - 1];
     for (int l = L - 2; l >= 0; l--) {
-        const size_t V = u->vox(l, b);
-        const int Cu = u->wd[l + 1], Cs = u->wd[l];
-        hipLaunchKernelGGL(k_upcat, dim3(blocks_for(V * (Cu + Cs))), dim3(256), 0, st, low, u->e[l],
-                           u->cat[l], V, u->ls0 - l, Cu, Cs);
+        const uint32_t V = (uint32_t)u->vox(l, b), Cu8 = (uint32_t)u->wd[l + 1] / 8, Cs8 = (uint32_t)u->wd[l] / 8;
+        hipLaunchKernelGGL(k_upcat, dim3(blocks_for((size_t)V * (Cu8 + Cs8))), dim3(256), 0, st, low, u->e[l], u->cat[l],
+                           V, u->ls0 - l, Cu8, Cs8);
         NX_CHECK_LAUNCH("k_upcat");
         if (int e = conv_fwd(u, u->dec(l, 0), b, u->cat[l], u->bb[l], conv::kRelu, st)) return e;
         if (int e = conv_fwd(u, u->dec(l, 1), b, u->bb[l], u->dd[l], conv::kRelu, st)) return e;
         low = u->dd[l];
     }
-    if (int e = conv_fwd(u, u->outc(), b, low, u->out32, conv::kOutF32, st)) return e;
+    if (int e = conv_fwd(u, u->outc(), b, low, y, conv::kOutF32, st, u->d.out_ch)) return e;
     u->fwd_batch = b;
     return NX_OK;
 }
@@ -342,38 +361,33 @@ int forward(nx_unet_s* u, const float* x, int b, hipStream_t st)
 int backward(nx_unet_s* u, int b, hipStream_t st)
 {
     const int L = u->L;
-    for (int ci = 0; ci < (int)u->convs.size(); ci++)
-        if (int e = conv::flip(u->shape(ci, b), u->wbf + u->convs[ci].w_off, u->wt + u->convs[ci].w_off, st))
-            return e;
-    const uint16_t* top = L > 1 ? u->dd[0] : u->e[0];
-    if (int e = conv_bwd(u, u->outc(), b, top, u->gout, u->g1[0], st)) return e;
+    conv::FlipTable tab{(int)u->convs.size(), {}};
+    for (int ci = 0; ci < tab.n; ci++) {
+        const ConvSpec& c = u->convs[ci];
+        tab.e[ci] = {(uint32_t)c.w_off, c.cin, c.cout, c.ks * c.ks * c.ks};
+    }
+    if (int e = conv::flip(tab, u->wbf, u->wt, st)) return e;
+    // g2[l]: the gradient before the ReLU of the level's second convolution
+    // (decoder, then encoder), g1[l] of its first
+    if (int e = conv_bwd(u, u->outc(), b, u->dd[0], u->gout, u->dd[0], u->g2[0], st)) return e;
     for (int l = 0; l < L - 1; l++) {
-        const size_t V = u->vox(l, b);
-        const size_t n = V * u->wd[l];
-        if (int e = relu_bwd(u->dd[l], u->g1[l], u->g2[l], n, st)) return e;
-        if (int e = conv_bwd(u, u->dec(l, 1), b, u->bb[l], u->g2[l], u->g1[l], st)) return e;
-        if (int e = relu_bwd(u->bb[l], u->g1[l], u->g2[l], n, st)) return e;
-        if (int e = conv_bwd(u, u->dec(l, 0), b, u->cat[l], u->g2[l], u->gcat[l], st)) return e;
-        const size_t Vh = u->vox(l + 1, b);
-        const int Cu = u->wd[l + 1], Cc = u->wd[l + 1] + u->wd[l];
-        hipLaunchKernelGGL(k_up_bwd, dim3(blocks_for(Vh * Cu)), dim3(256), 0, st, u->gcat[l], u->g1[l + 1],
-                           Vh, u->ls0 - l, Cc, Cu);
+        if (int e = conv_bwd(u, u->dec(l, 1), b, u->bb[l], u->g2[l], u->bb[l], u->g1[l], st)) return e;
+        if (int e = conv_bwd(u, u->dec(l, 0), b, u->cat[l], u->g1[l], nullptr, u->gcat[l], st)) return e;
+        const uint32_t Vh = (uint32_t)u->vox(l + 1, b), Cu8 = (uint32_t)u->wd[l + 1] / 8;
+        hipLaunchKernelGGL(k_up_bwd, dim3(blocks_for((size_t)Vh * Cu8)), dim3(256), 0, st, u->gcat[l],
+                           l + 1 == L - 1 ? u->e[l + 1] : u->dd[l + 1], u->g2[l + 1], Vh, u->ls0 - l,
+                           Cu8 + (uint32_t)u->wd[l] / 8, Cu8);
         NX_CHECK_LAUNCH("k_up_bwd");
     }
     for (int l = L - 1; l >= 0; l--) {
-        const size_t V = u->vox(l, b);
-        const size_t n = V * u->wd[l];
         if (l < L - 1) {
-            hipLaunchKernelGGL(k_skip_grad, dim3(blocks_for(n)), dim3(256), 0, st, u->gcat[l],
-                               u->wd[l + 1] + u->wd[l], u->wd[l + 1], u->gin[l + 1], u->g1[l], V,
-                               u->ls0 - l, u->wd[l]);
+            const uint32_t V = (uint32_t)u->vox(l, b), C8 = (uint32_t)u->wd[l] / 8, Cu8 = (uint32_t)u->wd[l + 1] / 8;
+            hipLaunchKernelGGL(k_skip_grad, dim3(blocks_for((size_t)V * C8)), dim3(256), 0, st, u->gcat[l], Cu8 + C8, Cu8,
+                               u->gin[l + 1], u->e[l], u->g2[l], V, u->ls0 - l, C8);
             NX_CHECK_LAUNCH("k_skip_grad");
         }
-        if (int e = relu_bwd(u->e[l], u->g1[l], u->g2[l], n, st)) return e;
-        if (int e = conv_bwd(u, u->enc(l, 1), b, u->a[l], u->g2[l], u->g1[l], st)) return e;
-        if (int e = relu_bwd(u->a[l], u->g1[l], u->g2[l], n, st)) return e;
-        if (int e = conv_bwd(u, u->enc(l, 0), b, u->in[l], u->g2[l], l > 0 ? u->gin[l] : nullptr, st))
-            return e;
+        if (int e = conv_bwd(u, u->enc(l, 1), b, u->a[l], u->g2[l], u->a[l], u->g1[l], st)) return e;
+        if (int e = conv_bwd(u, u->enc(l, 0), b, u->in[l], u->g1[l], nullptr, l > 0 ? u->gin[l] : nullptr, st)) return e;
     }
     return NX_OK;
 }
@@ -458,7 +472,7 @@ int nx_unet_create(const nx_unet_desc* d, nx_unet* out)
     const size_t V0 = u->vox(0, u->B);
     size_t ws = 0;
     for (int ci = 0; ci < (int)u->convs.size(); ci++) ws = std::max(ws, conv::bwd_weight_ws(u->shape(ci, u->B)));
-    if ((e = dalloc_t(u, V0 * kC0, &u->out32)) || (e = dalloc_t(u, V0 * kC0, &u->gout)) ||
+    if ((e = dalloc_t(u, V0 * d->out_ch, &u->out32)) || (e = dalloc_t(u, V0 * kC0, &u->gout)) ||
         (e = dalloc(u, ws, &u->ws)) || (e = dalloc_t(u, 8192, &u->loss_part)) ||
         (e = dalloc_t(u, 4, &u->loss_dev)))
         return fail(e);
@@ -532,12 +546,7 @@ int nx_unet_forward(nx_unet u, const float* x, int32_t batch, float* y, nx_strea
     if (int e = check_batch(u, batch)) return e;
     if (!x || !y) return set_error(NX_ERR_INVALID, "nx_unet_forward: null pointer");
     const hipStream_t st = (hipStream_t)s;
-    if (int e = forward(u, x, batch, st)) return e;
-    const size_t V0 = u->vox(0, batch);
-    hipLaunchKernelGGL(k_unpack_output, dim3(blocks_for(V0 * u->d.out_ch)), dim3(256), 0, st, u->out32, y,
-                       V0, u->d.out_ch);
-    NX_CHECK_LAUNCH("k_unpack_output");
-    return NX_OK;
+    return forward(u, x, batch, y, st);
 }
 
 int nx_unet_backward(nx_unet u, const float* dy, int32_t batch, nx_stream s)
@@ -548,7 +557,7 @@ int nx_unet_backward(nx_unet u, const float* dy, int32_t batch, nx_stream s)
         return set_error(NX_ERR_INVALID, "nx_unet_backward: batch differs from the last forward");
     const hipStream_t st = (hipStream_t)s;
     const size_t V0 = u->vox(0, batch);
-    hipLaunchKernelGGL(k_pack_grad, dim3(blocks_for(V0 * kC0)), dim3(256), 0, st, dy, u->gout, V0,
+    hipLaunchKernelGGL(k_pack_grad, dim3(blocks_for(V0)), dim3(256), 0, st, dy, u->gout, V0,
                        u->d.out_ch);
     NX_CHECK_LAUNCH("k_pack_grad");
     return backward(u, batch, st);
@@ -560,7 +569,7 @@ int nx_unet_train_step(nx_unet u, const float* x, const float* target, const flo
     if (int e = check_batch(u, batch)) return e;
     if (!x || !target || !weight) return set_error(NX_ERR_INVALID, "nx_unet_train_step: null pointer");
     const hipStream_t st = (hipStream_t)s;
-    if (int e = forward(u, x, batch, st)) return e;
+    if (int e = forward(u, x, batch, u->out32, st)) return e;
     const size_t V0 = u->vox(0, batch);
     const unsigned nb = std::min<unsigned>(blocks_for(V0), 8192u);
     hipLaunchKernelGGL(k_mse, dim3(nb), dim3(256), 0, st, u->out32, target, weight, u->gout, u->loss_part,
