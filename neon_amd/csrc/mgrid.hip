@@ -88,96 +88,184 @@ __host__ __device__ constexpr double w27(int q)
 // promotions: the density and velocity sums over q in order (util.h:47-62),
 // the double literals of the equilibrium, the shear split and gamma
 // evaluated in binary64 and stored in T, tiny = 1e-7 in gamma's denominator.
-// Two forms with the same results: kbc27_kept keeps the equilibrium,
-// fneq and the shear part of every population in arrays; kbc27_recomputed
-// recomputes them in each of the collision's three passes -- moment flux,
-// e0 / e1, output -- from copies of rho, u and usqr that the compiler may
-// not look through, so only the 27 populations stay live (occupancy).  The
-// same expressions give the same values.
+// Two forms with the same results: kbc27_kept keeps the equilibrium and fneq
+// of every population in arrays; kbc27_recomputed recomputes them in each of
+// the collision's three passes -- moment flux, e0 / e1, output -- from copies
+// of rho, u and usqr that the compiler may not look through, so only the 27
+// populations stay live (occupancy).
+//
+// The pass is bound by vector instructions, so what cannot change a result is
+// left out: terms times a zero velocity component or a zero shear part (0 x
+// is +-0, and these sums are never -0; a non-finite x makes every output NaN
+// either way), and the second half of each +-c pair's polynomial (c.u of the
+// opposite is exactly -c.u).
+constexpr int nonzero27(int q) { return (K27X[q] != 0) + (K27Y[q] != 0) + (K27Z[q] != 0); }
+
+// c.v with c of population q: the reference's sum over x, y, z without its
+// zero terms
+template <typename T>
+__device__ __forceinline__ T dot27(int q, T v0, T v1, T v2)
+{
+    T cu = 0;
+    bool first = true;
+    if (K27X[q]) cu = K27X[q] > 0 ? v0 : -v0, first = false;
+    if (K27Y[q]) cu = first ? (K27Y[q] > 0 ? v1 : -v1) : (K27Y[q] > 0 ? cu + v1 : cu - v1), first = false;
+    if (K27Z[q]) cu = first ? (K27Z[q] > 0 ? v2 : -v2) : (K27Z[q] > 0 ? cu + v2 : cu - v2);
+    return cu;
+}
+
 template <typename T>
 __device__ __forceinline__ T kbc27_feq(int q, T rho, T v0, T v1, T v2, T usqr)
 {
-    T cu = 0;
-    cu += (T)K27X[q] * v0;
-    cu += (T)K27Y[q] * v1;
-    cu += (T)K27Z[q] * v2;
-    cu = (T)((double)cu * 3.0);
+    const T cu = (T)((double)dot27<T>(q, v0, v1, v2) * 3.0);
     return (T)((double)rho * w27(q) * (1. + (double)cu + 0.5 * (double)cu * (double)cu - (double)usqr));
 }
 
+// Six moments Pi: xx, xy, xz, yy, yz, zz
 template <typename T>
-__device__ __forceinline__ void kbc27_kept(const T f[27], T om, T out[27])
+__device__ __forceinline__ void kbc27_flux(int q, T fneq, T p[6])
 {
-    const T beta = (T)((double)om * 0.5);
-    const T invBeta = (T)(1.0 / (double)beta);
-    const T tiny = (T)1e-7;
-    T rho = 0;
-#pragma unroll
-    for (int q = 0; q < 27; q++) rho += f[q];
-    T v0 = 0, v1 = 0, v2 = 0;
-#pragma unroll
-    for (int q = 0; q < 27; q++) {
-        v0 += f[q] * (T)K27X[q];
-        v1 += f[q] * (T)K27Y[q];
-        v2 += f[q] * (T)K27Z[q];
-    }
-    v0 /= rho;
-    v1 /= rho;
-    v2 /= rho;
-    const T usqr = (T)((3.0 / 2.0) * (double)(v0 * v0 + v1 * v1 + v2 * v2));
-    T feq[27], fneq[27];
-    T p0 = 0, p1 = 0, p2 = 0, p3 = 0, p4 = 0, p5 = 0;  // Pi: xx, xy, xz, yy, yz, zz
-#pragma unroll
-    for (int q = 0; q < 27; q++) {
-        T cu = 0;
-        cu += (T)K27X[q] * v0;
-        cu += (T)K27Y[q] * v1;
-        cu += (T)K27Z[q] * v2;
-        cu = (T)((double)cu * 3.0);
-        feq[q] = (T)((double)rho * w27(q) * (1. + (double)cu + 0.5 * (double)cu * (double)cu - (double)usqr));
-        fneq[q] = f[q] - feq[q];
-    }
-#pragma unroll
-    for (int q = 0; q < 27; q++) {
-        p0 += fneq[q] * (T)(K27X[q] * K27X[q]);
-        p1 += fneq[q] * (T)(K27X[q] * K27Y[q]);
-        p2 += fneq[q] * (T)(K27X[q] * K27Z[q]);
-        p3 += fneq[q] * (T)(K27Y[q] * K27Y[q]);
-        p4 += fneq[q] * (T)(K27Y[q] * K27Z[q]);
-        p5 += fneq[q] * (T)(K27Z[q] * K27Z[q]);
-    }
-    const T Nxz = p0 - p5, Nyz = p3 - p5;
-    const T shx = (T)((2.0 * (double)Nxz - (double)Nyz) / 6.0);
-    const T shy = (T)((-(double)Nxz + 2.0 * (double)Nyz) / 6.0);
-    const T shz = (T)((double)(-Nxz - Nyz) / 6.0);
-    const T sxy = (T)((double)p1 / 4.0), sxz = (T)((double)p2 / 4.0), syz = (T)((double)p4 / 4.0);
-    T dS[27];
-    T e0 = 0, e1 = 0;
-#pragma unroll
-    for (int q = 0; q < 27; q++) {
-        const int cx = K27X[q], cy = K27Y[q], cz = K27Z[q];
-        const int nz = (cx != 0) + (cy != 0) + (cz != 0);
-        T sh = (T)0;
-        if (nz == 1) sh = cx ? shx : (cy ? shy : shz);
-        if (nz == 2) sh = !cz ? (cx * cy > 0 ? sxy : -sxy) : (!cy ? (cx * cz > 0 ? sxz : -sxz) : (cy * cz > 0 ? syz : -syz));
-        dS[q] = rho * sh;
-        const T dH = fneq[q] - dS[q];
-        e0 += (dS[q] * dH / feq[q]);
-        e1 += (dH * dH / feq[q]);
-    }
-    const T gamma = (T)((double)invBeta - (2.0 - (double)invBeta) * (double)e0 / (double)(tiny + e1));
-#pragma unroll
-    for (int q = 0; q < 27; q++) {
-        const T dH = fneq[q] - dS[q];
-        out[q] = (T)((double)f[q] - (double)beta * (2.0 * (double)dS[q] + (double)(gamma * dH)));
-    }
+    const int c[3] = {K27X[q], K27Y[q], K27Z[q]};
+    int k = 0;
+    for (int a = 0; a < 3; a++)
+        for (int b = a; b < 3; b++, k++)
+            if (c[a] * c[b] != 0) p[k] = c[a] * c[b] > 0 ? p[k] + fneq : p[k] - fneq;
 }
 
 template <typename T>
-__device__ __forceinline__ void kbc27_recomputed(const T f[27], T om, T out[27])
+struct Shear27 {
+    T face[3], xy, xz, yz;  // rho times the shear part of (x, 0, 0) .. and of (+, +)
+    __device__ __forceinline__ Shear27(T rho, const T p[6])
+    {
+        const T Nxz = p[0] - p[5], Nyz = p[3] - p[5];
+        face[0] = rho * (T)((2.0 * (double)Nxz - (double)Nyz) / 6.0);
+        face[1] = rho * (T)((-(double)Nxz + 2.0 * (double)Nyz) / 6.0);
+        face[2] = rho * (T)((double)(-Nxz - Nyz) / 6.0);
+        xy = rho * (T)((double)p[1] / 4.0);
+        xz = rho * (T)((double)p[2] / 4.0);
+        yz = rho * (T)((double)p[4] / 4.0);
+    }
+    // populations with 1 or 2 non-zero components; the others have none
+    __device__ __forceinline__ T at(int q) const
+    {
+        const int cx = K27X[q], cy = K27Y[q], cz = K27Z[q];
+        if (nonzero27(q) == 1) return cx ? face[0] : (cy ? face[1] : face[2]);
+        if (nonzero27(q) == 2)
+            return !cz ? (cx * cy > 0 ? xy : -xy) : (!cy ? (cx * cz > 0 ? xz : -xz) : (cy * cz > 0 ? yz : -yz));
+        return T(0);
+    }
+};
+
+// Quotients by one binary32 divisor, correctly rounded, through a binary64
+// reciprocal (v_rcp_f32 and one cubic step: within 2^-52) shared by them.  a /
+// b of 24-bit values is never closer than 2^-49 to a rounding boundary, so
+// rounding the binary64 product to binary32 is rounding the quotient; a
+// division by itself is about twice the instructions.  |b| in [2^-100, 2^100];
+// a quotient below the normal range may round to its neighbour.
+struct Recip32 {
+    double r;
+    __device__ __forceinline__ explicit Recip32(float b)
+    {
+        const double d = (double)b, r0 = (double)__builtin_amdgcn_rcpf(b);
+        const double e = __builtin_fma(-d, r0, 1.0);
+        r = __builtin_fma(r0, __builtin_fma(e, e, e), r0);
+    }
+    __device__ __forceinline__ float operator()(float a) const { return (float)((double)a * r); }
+};
+__device__ __forceinline__ bool recip32_ok(float lo, float hi) { return lo >= 0x1p-100f && hi <= 0x1p100f; }
+
+struct Relax {  // one level's relaxation: beta = omega / 2 in T, 1 / beta
+    double omega, beta, inv_beta;
+};
+
+// binary32.  Measured (MI355X, 128^3 lid, coarse step): 457 us, with the
+// divisions, zero terms and both halves of each pair evaluated 493 us.
+__device__ __forceinline__ void kbc27_kept(const float f[27], const Relax& om, float out[27])
 {
-    const T beta = (T)((double)om * 0.5);
-    const T invBeta = (T)(1.0 / (double)beta);
+    using T = float;
+    const double beta = om.beta, invBeta = om.inv_beta;
+    const T tiny = (T)1e-7;
+    T rho = 0;
+#pragma unroll
+    for (int q = 0; q < 27; q++) rho += f[q];
+    T j0 = 0, j1 = 0, j2 = 0;
+#pragma unroll
+    for (int q = 0; q < 27; q++) {
+        if (K27X[q]) j0 = K27X[q] > 0 ? j0 + f[q] : j0 - f[q];
+        if (K27Y[q]) j1 = K27Y[q] > 0 ? j1 + f[q] : j1 - f[q];
+        if (K27Z[q]) j2 = K27Z[q] > 0 ? j2 + f[q] : j2 - f[q];
+    }
+    T v0, v1, v2;
+    if (recip32_ok(__builtin_fabsf(rho), __builtin_fabsf(rho))) {
+        const Recip32 by(rho);
+        v0 = by(j0), v1 = by(j1), v2 = by(j2);
+    } else {
+        v0 = j0 / rho, v1 = j1 / rho, v2 = j2 / rho;
+    }
+    const T usqr = (T)((3.0 / 2.0) * (double)(v0 * v0 + v1 * v1 + v2 * v2));
+    const double us = (double)usqr;
+    T feq[27], fneq[27];
+    T p[6] = {0, 0, 0, 0, 0, 0};
+    T lo, hi;
+#pragma unroll
+    for (int q = 0; q < 27; q++) {
+        const int o = K27OPP[q];
+        if (o < q) continue;
+        const double rw = (double)rho * w27(q);
+        if (o == q) {
+            feq[q] = (T)(rw * (1. - us));
+            lo = hi = __builtin_fabsf(feq[q]);
+            continue;
+        }
+        const double cu = (double)(T)((double)dot27<T>(q, v0, v1, v2) * 3.0);
+        const double sq = 0.5 * cu * cu;
+        feq[q] = (T)(rw * (1. + cu + sq - us));
+        feq[o] = (T)(rw * (1. - cu + sq - us));
+        lo = __builtin_fminf(__builtin_fminf(lo, __builtin_fabsf(feq[q])), __builtin_fabsf(feq[o]));
+        hi = __builtin_fmaxf(__builtin_fmaxf(hi, __builtin_fabsf(feq[q])), __builtin_fabsf(feq[o]));
+    }
+#pragma unroll
+    for (int q = 0; q < 27; q++) {
+        fneq[q] = f[q] - feq[q];
+        kbc27_flux<T>(q, fneq[q], p);
+    }
+    const Shear27<T> sh(rho, p);
+    T e0 = 0, e1 = 0;
+    auto sums = [&](auto&& divisor) __attribute__((always_inline)) {
+#pragma unroll
+        for (int q = 0; q < 27; q++) {
+            const auto by = divisor(feq[q]);
+            const T dS = sh.at(q);
+            const bool sheared = nonzero27(q) == 1 || nonzero27(q) == 2;
+            const T dH = sheared ? fneq[q] - dS : fneq[q];
+            if (sheared) e0 += by(dS * dH);
+            e1 += by(dH * dH);
+        }
+    };
+    if (recip32_ok(lo, hi)) {
+        sums([](T b) { return Recip32(b); });
+    } else {
+        struct Div {
+            T b;
+            __device__ __forceinline__ T operator()(T a) const { return a / b; }
+        };
+        sums([](T b) { return Div{b}; });
+    }
+    const T gamma = (T)(invBeta - (2.0 - invBeta) * (double)e0 / (double)(tiny + e1));
+#pragma unroll
+    for (int q = 0; q < 27; q++) {
+        const bool sheared = nonzero27(q) == 1 || nonzero27(q) == 2;
+        const T dS = sh.at(q);
+        const T dH = sheared ? fneq[q] - dS : fneq[q];
+        const double g = (double)(gamma * dH);
+        out[q] = (T)((double)f[q] - beta * (sheared ? 2.0 * (double)dS + g : g));
+    }
+}
+
+__device__ __forceinline__ void kbc27_recomputed(const double f[27], const Relax& om, double out[27])
+{
+    using T = double;
+    const T beta = om.beta, invBeta = om.inv_beta;
     const T tiny = (T)1e-7;
     T rho = 0;
 #pragma unroll
@@ -185,38 +273,18 @@ __device__ __forceinline__ void kbc27_recomputed(const T f[27], T om, T out[27])
     T v0 = 0, v1 = 0, v2 = 0;
 #pragma unroll
     for (int q = 0; q < 27; q++) {
-        v0 += f[q] * (T)K27X[q];
-        v1 += f[q] * (T)K27Y[q];
-        v2 += f[q] * (T)K27Z[q];
+        if (K27X[q]) v0 = K27X[q] > 0 ? v0 + f[q] : v0 - f[q];
+        if (K27Y[q]) v1 = K27Y[q] > 0 ? v1 + f[q] : v1 - f[q];
+        if (K27Z[q]) v2 = K27Z[q] > 0 ? v2 + f[q] : v2 - f[q];
     }
     v0 /= rho;
     v1 /= rho;
     v2 /= rho;
-    const T usqr = (T)((3.0 / 2.0) * (double)(v0 * v0 + v1 * v1 + v2 * v2));
-    T p0 = 0, p1 = 0, p2 = 0, p3 = 0, p4 = 0, p5 = 0;  // Pi: xx, xy, xz, yy, yz, zz
+    const T usqr = (3.0 / 2.0) * (v0 * v0 + v1 * v1 + v2 * v2);
+    T p[6] = {0, 0, 0, 0, 0, 0};
 #pragma unroll
-    for (int q = 0; q < 27; q++) {
-        const T fneq = f[q] - kbc27_feq<T>(q, rho, v0, v1, v2, usqr);
-        p0 += fneq * (T)(K27X[q] * K27X[q]);
-        p1 += fneq * (T)(K27X[q] * K27Y[q]);
-        p2 += fneq * (T)(K27X[q] * K27Z[q]);
-        p3 += fneq * (T)(K27Y[q] * K27Y[q]);
-        p4 += fneq * (T)(K27Y[q] * K27Z[q]);
-        p5 += fneq * (T)(K27Z[q] * K27Z[q]);
-    }
-    const T Nxz = p0 - p5, Nyz = p3 - p5;
-    const T shx = (T)((2.0 * (double)Nxz - (double)Nyz) / 6.0);
-    const T shy = (T)((-(double)Nxz + 2.0 * (double)Nyz) / 6.0);
-    const T shz = (T)((double)(-Nxz - Nyz) / 6.0);
-    const T sxy = (T)((double)p1 / 4.0), sxz = (T)((double)p2 / 4.0), syz = (T)((double)p4 / 4.0);
-    auto shear = [&](int q) -> T {
-        const int cx = K27X[q], cy = K27Y[q], cz = K27Z[q];
-        const int nz = (cx != 0) + (cy != 0) + (cz != 0);
-        if (nz == 1) return cx ? shx : (cy ? shy : shz);
-        if (nz == 2)
-            return !cz ? (cx * cy > 0 ? sxy : -sxy) : (!cy ? (cx * cz > 0 ? sxz : -sxz) : (cy * cz > 0 ? syz : -syz));
-        return (T)0;
-    };
+    for (int q = 0; q < 27; q++) kbc27_flux<T>(q, f[q] - kbc27_feq<T>(q, rho, v0, v1, v2, usqr), p);
+    const Shear27<T> sh(rho, p);
     T e0 = 0, e1 = 0;
     {
         T r = rho, a = v0, b = v1, c = v2, us = usqr;
@@ -228,13 +296,14 @@ __device__ __forceinline__ void kbc27_recomputed(const T f[27], T om, T out[27])
 #pragma unroll
         for (int q = 0; q < 27; q++) {
             const T feq = kbc27_feq<T>(q, r, a, b, c, us);
-            const T dS = rho * shear(q);
-            const T dH = (f[q] - feq) - dS;
-            e0 += (dS * dH / feq);
+            const bool sheared = nonzero27(q) == 1 || nonzero27(q) == 2;
+            const T dS = sh.at(q);
+            const T dH = sheared ? (f[q] - feq) - dS : f[q] - feq;
+            if (sheared) e0 += (dS * dH / feq);
             e1 += (dH * dH / feq);
         }
     }
-    const T gamma = (T)((double)invBeta - (2.0 - (double)invBeta) * (double)e0 / (double)(tiny + e1));
+    const T gamma = invBeta - (2.0 - invBeta) * e0 / (tiny + e1);
     T r = rho, a = v0, b = v1, c = v2, us = usqr;
     nx_pin(r);
     nx_pin(a);
@@ -244,23 +313,17 @@ __device__ __forceinline__ void kbc27_recomputed(const T f[27], T om, T out[27])
 #pragma unroll
     for (int q = 0; q < 27; q++) {
         const T feq = kbc27_feq<T>(q, r, a, b, c, us);
-        const T dS = rho * shear(q);
-        const T dH = (f[q] - feq) - dS;
-        out[q] = (T)((double)f[q] - (double)beta * (2.0 * (double)dS + (double)(gamma * dH)));
+        const bool sheared = nonzero27(q) == 1 || nonzero27(q) == 2;
+        const T dS = sh.at(q);
+        const T dH = sheared ? (f[q] - feq) - dS : f[q] - feq;
+        out[q] = f[q] - beta * (sheared ? 2.0 * dS + gamma * dH : gamma * dH);
     }
 }
 
 // binary64: the recomputing form (127 instead of 221 VGPRs, 16% faster on
-// the 240^3 grid); binary32: the form that keeps the 3 x 27 values (75
-// against 121 VGPRs did not pay for the recomputation there)
-template <typename T>
-__device__ __forceinline__ void kbc27(const T f[27], T om, T out[27])
-{
-    if constexpr (sizeof(T) == 8)
-        kbc27_recomputed<T>(f, om, out);
-    else
-        kbc27_kept<T>(f, om, out);
-}
+// the 240^3 grid); binary32: the form that keeps the values
+__device__ __forceinline__ void kbc27(const double f[27], const Relax& om, double out[27]) { kbc27_recomputed(f, om, out); }
+__device__ __forceinline__ void kbc27(const float f[27], const Relax& om, float out[27]) { kbc27_kept(f, om, out); }
 
 // lattice traits: populations, velocity table, rest population, collision
 struct L19 {
@@ -271,9 +334,9 @@ struct L19 {
     static constexpr __host__ __device__ int opp(int q) { return OPP[q]; }
     static constexpr __host__ __device__ double w(int q) { return wq(q); }
     template <typename T>
-    static __device__ __forceinline__ void collide(const T f[19], T om, T out[19])
+    static __device__ __forceinline__ void collide(const T f[19], const Relax& om, T out[19])
     {
-        bgk<T>(f, om, out);
+        bgk<T>(f, (T)om.omega, out);
     }
 };
 struct L27 {
@@ -284,9 +347,9 @@ struct L27 {
     static constexpr __host__ __device__ int opp(int q) { return K27OPP[q]; }
     static constexpr __host__ __device__ double w(int q) { return w27(q); }
     template <typename T>
-    static __device__ __forceinline__ void collide(const T f[27], T om, T out[27])
+    static __device__ __forceinline__ void collide(const T f[27], const Relax& om, T out[27])
     {
-        kbc27<T>(f, om, out);
+        kbc27(f, om, out);
     }
 };
 
@@ -301,7 +364,7 @@ constexpr int kLinksPerWord = 21;
 template <int S, class LT>
 __global__ void __launch_bounds__(kBV)
     k_mr_collide(const typename MS<S>::T* __restrict__ fin, typename MS<S>::T* __restrict__ fout,
-                 const uint32_t* __restrict__ state, double omega)
+                 const uint32_t* __restrict__ state, Relax om)
 {
     using T = typename MS<S>::T;
     constexpr int NQ = LT::Q;
@@ -317,7 +380,7 @@ __global__ void __launch_bounds__(kBV)
     T f[NQ], o[NQ];
 #pragma unroll
     for (int q = 0; q < NQ; q++) f[q] = fin[own + (uint64_t)q * kBV];
-    LT::template collide<T>(f, (T)omega, o);
+    LT::template collide<T>(f, om, o);
 #pragma unroll
     for (int q = 0; q < NQ; q++) __builtin_nontemporal_store(o[q], &fout[own + (uint64_t)q * kBV]);
 }
@@ -365,7 +428,7 @@ __global__ void __launch_bounds__(kBV)
     k_mr_stream(const typename MS<S>::T* __restrict__ fout, typename MS<S>::T* __restrict__ out,
                 const uint32_t* __restrict__ state, const uint64_t* __restrict__ links, uint64_t n_slots,
                 const uint32_t* __restrict__ conn, const int32_t* __restrict__ origins,
-                const float* __restrict__ ss, UpLevel up, double omega)
+                const float* __restrict__ ss, UpLevel up, Relax om)
 {
     using T = typename MS<S>::T;
     constexpr int NQ = LT::Q;
@@ -445,7 +508,7 @@ __global__ void __launch_bounds__(kBV)
     }
     if constexpr (COLLIDE) {
         T o[NQ];
-        LT::template collide<T>(f, (T)omega, o);
+        LT::template collide<T>(f, om, o);
 #pragma unroll
         for (int q = 0; q < NQ; q++) __builtin_nontemporal_store(o[q], &out[own + (uint64_t)q * kBV]);
     } else if constexpr (KEEP) {
@@ -1091,6 +1154,12 @@ struct Stepper {
         const int il = g.depth - l - 1;
         return 2 * omega0 / (std::scalbln(1.0, il + 1) + (1. - std::scalbln(1.0, il)) * omega0);
     }
+    // beta and 1 / beta in T, as the reference's collision evaluates them
+    Relax relax(int l) const
+    {
+        const T om = (T)omega(l), beta = (T)((double)om * 0.5);
+        return Relax{(double)om, (double)beta, (double)(T)(1.0 / (double)beta)};
+    }
     UpLevel up(int l) const
     {
         if (l + 1 >= g.depth) return UpLevel{nullptr, nullptr, {0, 0, 0}};
@@ -1102,7 +1171,7 @@ struct Stepper {
         const Level& lv = g.L[l];
         if (lv.n_blocks)
             hipLaunchKernelGGL((k_mr_collide<S, LT>), dim3(lv.n_blocks), dim3(kBV), 0, st, (const T*)lv.fin,
-                               (T*)lv.fout, lv.d_state, omega(l));
+                               (T*)lv.fout, lv.d_state, relax(l));
     }
     void store(int l) const
     {
@@ -1118,7 +1187,8 @@ struct Stepper {
         if (lv.n_blocks)
             hipLaunchKernelGGL((k_mr_stream<S, LT, COLLIDE, KEEP>), dim3(lv.n_blocks), dim3(kBV), 0, st,
                                (const T*)lv.fout, (T*)lv.fin, lv.d_state, lv.d_links, (uint64_t)lv.slots(),
-                               lv.d_conn, lv.d_origins, (const float*)lv.d_ss, up(l), COLLIDE ? omega(l) : 0.0);
+                               lv.d_conn, lv.d_origins, (const float*)lv.d_ss, up(l),
+                               COLLIDE ? relax(l) : Relax{0.0, 0.0, 0.0});
     }
 
     // n coarse steps.  A level's stream and its next collide touch no other
