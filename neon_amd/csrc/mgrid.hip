@@ -387,18 +387,29 @@ __global__ void __launch_bounds__(kBV)
 
 // store.h:98-163 as a gather: entry e adds its fine sources, in order, to
 // the coarse accumulator target[e].
-template <int S>
-__global__ void __launch_bounds__(256)
-    k_mr_store(const typename MS<S>::T* __restrict__ fine, typename MS<S>::T* __restrict__ coarse,
-               const uint64_t* __restrict__ target, const uint32_t* __restrict__ first,
-               const uint64_t* __restrict__ src, uint32_t n)
+struct StoreArgs {
+    void* coarse;
+    const uint64_t* target;
+    const uint32_t* first;
+    const uint64_t* src;
+    uint32_t n;
+    uint32_t groups;  // workgroups of kBV entries that carry it, a multiple of the 8 XCDs
+};
+
+template <typename T>
+__device__ __forceinline__ void store_entry(const T* __restrict__ fine, const StoreArgs& s, uint32_t e)
 {
-    using T = typename MS<S>::T;
-    const uint32_t e = blockIdx.x * 256 + threadIdx.x;
-    if (e >= n) return;
-    T acc = coarse[target[e]];
-    for (uint32_t k = first[e]; k < first[e + 1]; k++) acc += fine[src[k]];
-    coarse[target[e]] = acc;
+    if (e >= s.n) return;
+    T* coarse = (T*)s.coarse;
+    T acc = coarse[s.target[e]];
+    for (uint32_t k = s.first[e]; k < s.first[e + 1]; k++) acc += fine[s.src[k]];
+    coarse[s.target[e]] = acc;
+}
+
+template <int S>
+__global__ void __launch_bounds__(kBV) k_mr_store(const typename MS<S>::T* __restrict__ fine, StoreArgs s)
+{
+    store_entry(fine, s, blockIdx.x * kBV + threadIdx.x);
 }
 
 struct UpLevel {  // the next coarser level, seen from this one (explosion)
@@ -407,15 +418,73 @@ struct UpLevel {  // the next coarser level, seen from this one (explosion)
     int32_t nb[3];
 };
 
+// Byte offsets of the 27 neighbour blocks' populations (scalar registers; an
+// absent neighbour gives the own block, whose value no link uses) and of the
+// upstream voxel of a velocity (cx, cy, cz) among them.  O: 32 bits where the
+// level's populations fit 4 GiB -- a third of the address instructions of the
+// 64-bit form, and most of this pass's instructions outside the collision.
+template <typename O>
+struct Rows {
+    O c[27];
+    template <typename T, int NQ>
+    static __device__ __forceinline__ Rows load(const uint32_t* __restrict__ conn, uint32_t b)
+    {
+        Rows r;
+#pragma unroll
+        for (int d = 0; d < 27; d++) {
+            const uint32_t t = conn[(uint64_t)b * 27 + d];
+            r.c[d] = (O)(t != kInvalidBlock ? t : b) * (O)(NQ * kBV * sizeof(T));
+        }
+        return r;
+    }
+    // (by value: an entry read inside an arm would make the table an array in memory)
+    static __device__ __forceinline__ O pick(bool c, O a, O b) { return c ? a : b; }
+    template <typename T, int s0, int s1, int s2>
+    __device__ __forceinline__ O at(int x, int y, int z) const
+    {
+        const bool c0 = s0 != 0 && x == (s0 < 0 ? 0 : 7);
+        const bool c1 = s1 != 0 && y == (s1 < 0 ? 0 : 7);
+        const bool c2 = s2 != 0 && z == (s2 < 0 ? 0 : 7);
+        O t = c[13];
+        if constexpr (s0 != 0) t = pick(c0, c[13 + s0], t);
+        if constexpr (s1 != 0) t = pick(c1, c[13 + 3 * s1], t);
+        if constexpr (s2 != 0) t = pick(c2, c[13 + 9 * s2], t);
+        if constexpr (s0 != 0 && s1 != 0) t = pick(c0 && c1, c[13 + s0 + 3 * s1], t);
+        if constexpr (s0 != 0 && s2 != 0) t = pick(c0 && c2, c[13 + s0 + 9 * s2], t);
+        if constexpr (s1 != 0 && s2 != 0) t = pick(c1 && c2, c[13 + 3 * s1 + 9 * s2], t);
+        if constexpr (s0 != 0 && s1 != 0 && s2 != 0) t = pick(c0 && c1 && c2, c[13 + s0 + 3 * s1 + 9 * s2], t);
+        return t + (O)((((x + s0) & 7) + 8 * ((y + s1) & 7) + 64 * ((z + s2) & 7)) * (int)sizeof(T));
+    }
+};
+
+// k_mr_stream's shape per lattice and type, by what it measured (coarse step
+// of the 128^3 three-level lid): the wavefronts per SIMD its registers must
+// allow (workgroups are 2 per SIMD each), how many links one batch of fix-up
+// loads covers, and whether the neighbour offsets are formed again for the
+// fix-ups (fewer registers) or kept.  KBC binary32 keeps them (414 us against
+// 438 formed again; batches of 1, 3, 9: 470, 414, 431 us; the 64-bit offsets
+// would spill); BGK binary32 forms
+// them again (219 against 246 us, 46-74 against 85-108 registers).
+template <int S, class LT>
+struct StreamShape {
+    static constexpr bool wide = LT::Q == 27, f64 = S == NX_F64;
+    static constexpr int waves = wide || f64 ? 4 : 6;
+    static constexpr int batch = wide ? 3 : f64 ? 5 : 10;
+    static constexpr bool again = f64 || !wide;
+};
+
 // stream.h:170-225 (stream fused with coalescence and explosion), pull, for
 // the bulk leaf voxels of one level.  The plain pull of all populations is
-// issued first (upstream voxel through the connectivity row in scalar
-// registers); voxels with another link state then fix those links up:
-// bounce-back (own opposite + the wall's opposite), explosion (the coarse
-// post-collision population of the uncle, the next level's voxel holding
-// the upstream position), coalescence (the refined upstream voxel's
-// accumulated fine populations times its weight); links in state "none"
-// keep the value in `out`.
+// issued with the state and link words, before either is known (one memory
+// round trip; a slot that is no bulk leaf reads values it does not use); then
+// voxels with another link state fix those links up: bounce-back (own
+// opposite + the wall's opposite), explosion (the coarse post-collision
+// population of the uncle, the next level's voxel holding the upstream
+// position), coalescence (the refined upstream voxel's accumulated fine
+// populations times its weight); links in state "none" keep the value in
+// `out`.  The fix-ups' loads go out in batches of populations: on
+// refined grids most wavefronts hold a wall or an interface, and a wait per
+// link made the fix-ups the longest part of the pass.
 // COLLIDE: the pulled populations are collided at once with omega and the
 // result written to `out`, and refined voxels reset their accumulator in
 // `out` -- stream followed by the next collide of the same level
@@ -423,101 +492,142 @@ struct UpLevel {  // the next coarser level, seen from this one (explosion)
 // sequence, bit for bit.  KEEP = false: the level has no link in state
 // "none" (checked on the host), every population is stored.  `links` holds
 // LT::W words per voxel slot, word k at k * n_slots.
-template <int S, class LT, bool COLLIDE, bool KEEP>
-__global__ void __launch_bounds__(kBV)
+// The first st.groups workgroups carry the level's fine-to-coarse store (a
+// launch of its own costs more than its work): it reads this level's
+// post-collision field as the stream does and adds to refined voxels of the
+// next level, which the explosion never reads (checked on the host).
+// Measured (MI355X, coarse step of the 128^3 three-level lid; before with the
+// present collision): KBC f32 414 us (457), f64 680 (737), BGK f32 219 (246),
+// f64 371 (393); of the 48^3 lid 105 (144) and 67 us (90) in binary32.
+template <int S, class LT, bool COLLIDE, bool KEEP, typename O>
+__global__ void __launch_bounds__(kBV, (StreamShape<S, LT>::waves))
     k_mr_stream(const typename MS<S>::T* __restrict__ fout, typename MS<S>::T* __restrict__ out,
                 const uint32_t* __restrict__ state, const uint64_t* __restrict__ links, uint64_t n_slots,
                 const uint32_t* __restrict__ conn, const int32_t* __restrict__ origins,
-                const float* __restrict__ ss, UpLevel up, Relax om)
+                const float* __restrict__ ss, UpLevel up, Relax om, StoreArgs sa)
 {
     using T = typename MS<S>::T;
     constexpr int NQ = LT::Q;
-    const uint32_t b = xcd_remap(blockIdx.x, gridDim.x), v = threadIdx.x;  // neighbour blocks share an XCD's L2
-    const Conn cb = load_conn(conn, b);
-    const uint32_t st = state[(uint64_t)b * kBV + v];
-    if ((st & kActive) && (st & kRefined) && cls_bits(st) == NX_CELL_BULK) {
+    if (blockIdx.x < sa.groups) {
+        store_entry(fout, sa, blockIdx.x * kBV + threadIdx.x);
+        return;
+    }
+    // neighbour blocks share an XCD's L2
+    const uint32_t b = xcd_remap(blockIdx.x - sa.groups, gridDim.x - sa.groups), v = threadIdx.x;
+    const Rows<O> rows = Rows<O>::template load<T, NQ>(conn, b);
+    const int x = (int)(v & 7u), y = (int)((v >> 3) & 7u), z = (int)(v >> 6);
+    const O own = rows.c[13] + (O)(v * sizeof(T));
+    auto ld = [](const void* p, O at) __attribute__((always_inline)) { return *(const T*)((const char*)p + at); };
+    auto st = [](void* p, O at, T val) __attribute__((always_inline)) {
+        __builtin_nontemporal_store(val, (T*)((char*)p + at));
+    };
+    uint32_t sv = state[(uint64_t)b * kBV + v];
+    uint64_t lk[LT::W];
+#pragma unroll
+    for (int k = 0; k < LT::W; k++) lk[k] = links[(uint64_t)k * n_slots + (uint64_t)b * kBV + v];
+    T f[NQ];
+    for_q(std::make_integer_sequence<int, NQ>{}, [&](auto qc) __attribute__((always_inline)) {
+        constexpr int q = decltype(qc)::value;
+        f[q] = ld(fout + q * kBV, rows.template at<T, -LT::cx(q), -LT::cy(q), -LT::cz(q)>(x, y, z));
+    });
+#pragma unroll
+    for (int q = 0; q < NQ; q++) nx_pin(f[q]);
+    nx_pin(sv);
+#pragma unroll
+    for (int k = 0; k < LT::W; k++) nx_pin(lk[k]);
+    if ((sv & kActive) && (sv & kRefined) && cls_bits(sv) == NX_CELL_BULK) {
         // a refined voxel: with COLLIDE the collide's reset of its
         // accumulator (collide.h:131-141); otherwise its fin, which the
         // reference never writes after the set-up's 0, back to 0 (a fused
         // pass earlier in the call left an accumulator in this buffer)
-        const uint64_t own = (uint64_t)b * (NQ * kBV) + v;
 #pragma unroll
-        for (int q = 0; q < NQ; q++) __builtin_nontemporal_store(T(0), &out[own + (uint64_t)q * kBV]);
+        for (int q = 0; q < NQ; q++) st(out + q * kBV, own, T(0));
         return;
     }
-    if (!bulk_leaf(st)) return;
-    uint64_t lk[LT::W];
-#pragma unroll
-    for (int k = 0; k < LT::W; k++) lk[k] = links[(uint64_t)k * n_slots + (uint64_t)b * kBV + v];
-    const int x = (int)(v & 7u), y = (int)((v >> 3) & 7u), z = (int)(v >> 6);
-    const uint64_t own = (uint64_t)b * (NQ * kBV) + v;
-    T f[NQ];
-    for_q(std::make_integer_sequence<int, NQ>{}, [&](auto qc) {
-        constexpr int q = decltype(qc)::value;
-        if constexpr (q == LT::REST) {
-            f[q] = fout[own + (uint64_t)q * kBV];
-        } else {
-            uint32_t t, nv;
-            upstream_off<-LT::cx(q), -LT::cy(q), -LT::cz(q)>(b, cb, x, y, z, t, nv);
-            f[q] = fout[t != kInvalidBlock ? ((uint64_t)t * NQ + q) * kBV + nv : own + (uint64_t)q * kBV];
-        }
-    });
-#pragma unroll
-    for (int q = 0; q < NQ; q++) nx_pin(f[q]);
+    if (!bulk_leaf(sv)) return;
     uint32_t keep = 0;  // links whose value stays as it is in `out`
-    bool any = false;
+    // (opaque copies: the neighbour offsets are formed again where a link
+    // needs them instead of staying in registers across the pass)
+    int xl = x, yl = y, zl = z;
+    if constexpr (StreamShape<S, LT>::again || sizeof(O) == 8) {
+        nx_pin(xl);
+        nx_pin(yl);
+        nx_pin(zl);
+    }
+    constexpr int kBatch = StreamShape<S, LT>::batch;
+    for_q(std::make_integer_sequence<int, (NQ + kBatch - 1) / kBatch>{}, [&](auto gc) __attribute__((always_inline)) {
+        constexpr int q0 = decltype(gc)::value * kBatch, q1 = q0 + kBatch < NQ ? q0 + kBatch : NQ;
+        using Batch = std::make_integer_sequence<int, q1 - q0>;
+        uint32_t kind[kBatch];
+        uint32_t any = 0;
+        bool expl = false;
+        for_q(Batch{}, [&](auto ic) __attribute__((always_inline)) {
+            constexpr int i = decltype(ic)::value, q = q0 + i;
+            kind[i] = (uint32_t)((lk[q / kLinksPerWord] >> (3 * (q % kLinksPerWord))) & 7u);
+            any |= kind[i];
+            expl |= kind[i] == (uint32_t)kExpl;
+        });
+        if (!__any(any != 0)) return;
+        uint32_t tb[kBatch], slot[kBatch];
 #pragma unroll
-    for (int k = 0; k < LT::W; k++) any |= lk[k] != 0;
-    if (any) {
-        for_q(std::make_integer_sequence<int, NQ>{}, [&](auto qc) {
-            constexpr int q = decltype(qc)::value;
-            if constexpr (q != LT::REST) {
-                const uint64_t kind = (lk[q / kLinksPerWord] >> (3 * (q % kLinksPerWord))) & 7u;
-                if (kind == kPlain) return;
-                uint32_t t, nv;
-                upstream_off<-LT::cx(q), -LT::cy(q), -LT::cz(q)>(b, cb, x, y, z, t, nv);
-                bool ok = true;
-                if (kind == kWall) {
-                    constexpr int o = LT::opp(q);
-                    ok = t != kInvalidBlock;
-                    if (ok) f[q] = fout[own + (uint64_t)o * kBV] + fout[((uint64_t)t * NQ + o) * kBV + nv];
-                } else if (kind == kExpl) {
-                    const int ux = (origins[3 * (uint64_t)b] + x - LT::cx(q)) >> 1;
-                    const int uy = (origins[3 * (uint64_t)b + 1] + y - LT::cy(q)) >> 1;
-                    const int uz = (origins[3 * (uint64_t)b + 2] + z - LT::cz(q)) >> 1;
-                    const int bx = ux >> 3, by = uy >> 3, bz = uz >> 3;
-                    ok = up.table && !(bx < 0 || by < 0 || bz < 0 || bx >= up.nb[0] || by >= up.nb[1] ||
-                                       bz >= up.nb[2]);
-                    const uint32_t tb = ok ? up.table[((uint64_t)bz * up.nb[1] + by) * up.nb[0] + bx]
-                                           : kInvalidBlock;
-                    ok = tb != kInvalidBlock;
-                    const uint32_t slot = (uint32_t)((ux & 7) + 8 * (uy & 7) + 64 * (uz & 7));
-                    if (ok) f[q] = ((const T*)up.fout)[((uint64_t)tb * NQ + q) * kBV + slot];
-                } else if (kind == kCoal) {
-                    ok = t != kInvalidBlock && ss;
-                    if (ok) f[q] = f[q] * (T)ss[((uint64_t)t * NQ + q) * kBV + nv];
-                } else {
-                    ok = false;
-                }
-                if (!ok) {
-                    keep |= 1u << q;
-                    f[q] = out[own + (uint64_t)q * kBV];
-                }
+        for (int i = 0; i < kBatch; i++) tb[i] = kInvalidBlock;
+        if (__any(expl)) {
+            for_q(Batch{}, [&](auto ic) __attribute__((always_inline)) {
+                constexpr int i = decltype(ic)::value, q = q0 + i;
+                if (kind[i] != (uint32_t)kExpl) return;
+                const int ux = (origins[3 * (uint64_t)b] + xl - LT::cx(q)) >> 1;
+                const int uy = (origins[3 * (uint64_t)b + 1] + yl - LT::cy(q)) >> 1;
+                const int uz = (origins[3 * (uint64_t)b + 2] + zl - LT::cz(q)) >> 1;
+                const int bx = ux >> 3, by = uy >> 3, bz = uz >> 3;
+                slot[i] = (uint32_t)((ux & 7) + 8 * (uy & 7) + 64 * (uz & 7));
+                if (up.table && !(bx < 0 || by < 0 || bz < 0 || bx >= up.nb[0] || by >= up.nb[1] || bz >= up.nb[2]))
+                    tb[i] = up.table[((uint64_t)bz * up.nb[1] + by) * up.nb[0] + bx];
+            });
+#pragma unroll
+            for (int i = 0; i < kBatch; i++) nx_pin(tb[i]);
+        }
+        T a[kBatch], w[kBatch];
+        for_q(Batch{}, [&](auto ic) __attribute__((always_inline)) {
+            constexpr int i = decltype(ic)::value, q = q0 + i, o = LT::opp(q);
+            a[i] = w[i] = T(0);
+            if (kind[i] == (uint32_t)kPlain) return;
+            const O nb = rows.template at<T, -LT::cx(q), -LT::cy(q), -LT::cz(q)>(xl, yl, zl);
+            if (kind[i] == (uint32_t)kWall) {
+                a[i] = ld(fout + o * kBV, own);
+                w[i] = ld(fout + o * kBV, nb);
+            } else if (kind[i] == (uint32_t)kCoal) {
+                w[i] = (T)ss[(uint64_t)(nb / (O)sizeof(T)) + q * kBV];
+            } else if (tb[i] != kInvalidBlock) {
+                w[i] = ((const T*)up.fout)[((uint64_t)tb[i] * NQ + q) * kBV + slot[i]];
+            } else {
+                keep |= 1u << q;
+                w[i] = ld(out + q * kBV, own);
             }
         });
-    }
+#pragma unroll
+        for (int i = 0; i < kBatch; i++) {
+            nx_pin(a[i]);
+            nx_pin(w[i]);
+        }
+        for_q(Batch{}, [&](auto ic) __attribute__((always_inline)) {
+            constexpr int i = decltype(ic)::value, q = q0 + i;
+            const T one = kind[i] == (uint32_t)kWall ? a[i] + w[i] : w[i];
+            const T scaled = kind[i] == (uint32_t)kCoal ? f[q] * w[i] : f[q];
+            f[q] = kind[i] == (uint32_t)kPlain || kind[i] == (uint32_t)kCoal ? scaled : one;
+        });
+    });
     if constexpr (COLLIDE) {
         T o[NQ];
         LT::template collide<T>(f, om, o);
 #pragma unroll
-        for (int q = 0; q < NQ; q++) __builtin_nontemporal_store(o[q], &out[own + (uint64_t)q * kBV]);
+        for (int q = 0; q < NQ; q++) st(out + q * kBV, own, o[q]);
     } else if constexpr (KEEP) {
 #pragma unroll
         for (int q = 0; q < NQ; q++)
-            if (!((keep >> q) & 1u)) __builtin_nontemporal_store(f[q], &out[own + (uint64_t)q * kBV]);
+            if (!((keep >> q) & 1u)) st(out + q * kBV, own, f[q]);
     } else {
 #pragma unroll
-        for (int q = 0; q < NQ; q++) __builtin_nontemporal_store(f[q], &out[own + (uint64_t)q * kBV]);
+        for (int q = 0; q < NQ; q++) st(out + q * kBV, own, f[q]);
     }
 }
 
@@ -558,7 +668,8 @@ struct Level {
     float* d_ss = nullptr;  // coalescence weights (levels above 0)
     void* fin = nullptr;
     void* fout = nullptr;
-    bool keep = true;  // the level has links in state "none"
+    bool keep = true;      // the level has links in state "none"
+    bool separate = false; // an explosion link reads a refined voxel: the store needs its own launch
     int nq = 19;       // populations per voxel
     // active voxels as runs (first, one past the last) of the dense order
     std::vector<std::pair<size_t, size_t>> runs;
@@ -848,9 +959,10 @@ bool has_parent(const nx_mgrid_s& g, int l, int x, int y, int z)
 // Link states of every bulk leaf voxel of level l (stream.h:170-225 decided
 // per link), 3 bits per population, W words per voxel slot (word k at
 // k * slots); returns the number of links in state "none".
-uint64_t links_of(const nx_mgrid_s& g, int l, std::vector<uint64_t>& out)
+uint64_t links_of(const nx_mgrid_s& g, int l, std::vector<uint64_t>& out, bool& refined_uncle)
 {
     uint64_t n_skip = 0;
+    refined_uncle = false;
     const Level& lv = g.L[l];
     const HostLat& L = g.lat;
     out.assign((size_t)L.W * lv.slots(), 0);
@@ -875,7 +987,10 @@ uint64_t links_of(const nx_mgrid_s& g, int l, std::vector<uint64_t>& out)
                         const Level& c = g.L[l + 1];
                         const int ux = (x >> 1) + uoff(x, -L.c[q][0]), uy = (y >> 1) + uoff(y, -L.c[q][1]),
                                   uz = (z >> 1) + uoff(z, -L.c[q][2]);
-                        if (c.active(ux, uy, uz)) kind = kExpl;
+                        if (c.active(ux, uy, uz)) {
+                            kind = kExpl;
+                            refined_uncle = refined_uncle || (c.st[c.lin(ux, uy, uz)] & kRefined);
+                        }
                     }
                     lk[q / kLinksPerWord] |= kind << (3 * (q % kLinksPerWord));
                     n_skip += kind == kSkip;
@@ -1030,7 +1145,7 @@ int setup_cells(nx_mgrid g, const uint8_t* const* cls, const double uw[3])
                 lv.runs.back().second = i + 1;
             }
         std::vector<uint64_t> lk;
-        const uint64_t n_skip = links_of(*g, l, lk);
+        const uint64_t n_skip = links_of(*g, l, lk, lv.separate);
         lv.keep = n_skip != 0;
         if (int e = upload((void**)&lv.d_links, lk.data(), lk.size() * 8)) return e;
     }
@@ -1173,22 +1288,34 @@ struct Stepper {
             hipLaunchKernelGGL((k_mr_collide<S, LT>), dim3(lv.n_blocks), dim3(kBV), 0, st, (const T*)lv.fin,
                                (T*)lv.fout, lv.d_state, relax(l));
     }
-    void store(int l) const
+    StoreArgs store_args(int l) const
     {
         const Store& sl = g.store[l];
-        if (l + 1 < g.depth && sl.n)
-            hipLaunchKernelGGL((k_mr_store<S>), dim3((sl.n + 255) / 256), dim3(256), 0, st, (const T*)g.L[l].fout,
-                               (T*)g.L[l + 1].fout, sl.d_target, sl.d_first, sl.d_src, sl.n);
+        if (l + 1 >= g.depth || !sl.n) return StoreArgs{nullptr, nullptr, nullptr, nullptr, 0, 0};
+        return StoreArgs{g.L[l + 1].fout, sl.d_target, sl.d_first, sl.d_src, sl.n, ((sl.n + kBV - 1) / kBV + 7u) & ~7u};
     }
+    void store(int l) const
+    {
+        const StoreArgs a = store_args(l);
+        if (a.n)
+            hipLaunchKernelGGL((k_mr_store<S>), dim3(a.groups), dim3(kBV), 0, st, (const T*)g.L[l].fout, a);
+    }
+    // with_store: the level's store, due since its collide, rides along
     template <bool COLLIDE, bool KEEP>
-    void stream(int l) const
+    void stream(int l, bool with_store) const
     {
         const Level& lv = g.L[l];
-        if (lv.n_blocks)
-            hipLaunchKernelGGL((k_mr_stream<S, LT, COLLIDE, KEEP>), dim3(lv.n_blocks), dim3(kBV), 0, st,
-                               (const T*)lv.fout, (T*)lv.fin, lv.d_state, lv.d_links, (uint64_t)lv.slots(),
+        if (!lv.n_blocks) return;
+        const StoreArgs a = with_store ? store_args(l) : StoreArgs{nullptr, nullptr, nullptr, nullptr, 0, 0};
+        auto go = [&](auto off) {
+            hipLaunchKernelGGL((k_mr_stream<S, LT, COLLIDE, KEEP, decltype(off)>), dim3(lv.n_blocks + a.groups), dim3(kBV),
+                               0, st, (const T*)lv.fout, (T*)lv.fin, lv.d_state, lv.d_links, (uint64_t)lv.slots(),
                                lv.d_conn, lv.d_origins, (const float*)lv.d_ss, up(l),
-                               COLLIDE ? relax(l) : Relax{0.0, 0.0, 0.0});
+                               COLLIDE ? relax(l) : Relax{0.0, 0.0, 0.0}, a);
+        };
+        // byte offsets in 32 bits where the level's populations allow it
+        if ((uint64_t)lv.slots() * LT::Q * sizeof(T) < (1ull << 32)) go(uint32_t{});
+        else go(uint64_t{});
     }
 
     // n coarse steps.  A level's stream and its next collide touch no other
@@ -1199,6 +1326,12 @@ struct Stepper {
     // when its turn comes; the store after it then reads the fused pass's
     // output.  The last stream of each level in the call is not fused, so
     // the fields between calls are those of the unfused sequence.
+    //
+    // The store after a collide runs in the launch of the level's next
+    // stream: between the two only finer levels run, whose streams read
+    // unrefined voxels of this level and whose stores add to its refined
+    // ones, while this store reads its unrefined voxels and adds to the next
+    // level's refined ones, first used by that level's own stream.
     void run(const std::vector<Op>& ops, int n) const
     {
         bool done[kMaxDepth] = {};  // the level's next collide already ran in a fused pass
@@ -1212,15 +1345,15 @@ struct Stepper {
                     else
                         collide(l);
                 } else if (op.kind == 1) {
-                    store(l);
+                    if (lv.separate) store(l);
                 } else if (!lv.keep && !(op.last && k == n - 1)) {
-                    stream<true, false>(l);
+                    stream<true, false>(l, !lv.separate);
                     std::swap(lv.fin, lv.fout);
                     done[l] = true;
                 } else if (lv.keep) {
-                    stream<false, true>(l);
+                    stream<false, true>(l, !lv.separate);
                 } else {
-                    stream<false, false>(l);
+                    stream<false, false>(l, !lv.separate);
                 }
             }
     }
