@@ -74,6 +74,42 @@ __device__ __forceinline__ void upstream(uint32_t b, const Conn& cn, int x, int 
     upstream_off<-CX[q], -CY[q], -CZ[q]>(b, cn, x, y, z, t, nv);
 }
 
+// Byte offsets of the 27 neighbour blocks' populations (scalar registers; an
+// absent neighbour gives the own block, whose value no link uses) and of the
+// upstream voxel of a velocity (cx, cy, cz) among them.  O: 32 bits where the
+// level's populations fit 4 GiB -- a third of the address instructions of the
+// 64-bit form, and most of a pull's instructions outside the collision.
+template <typename O>
+struct Rows {
+    O c[27];
+    template <typename T, int NQ>
+    static __device__ __forceinline__ Rows of(const Conn& cn, uint32_t b)
+    {
+        Rows r;
+#pragma unroll
+        for (int d = 0; d < 27; d++) r.c[d] = (O)(cn.c[d] != kInvalidBlock ? cn.c[d] : b) * (O)(NQ * kBV * sizeof(T));
+        return r;
+    }
+    // (by value: an entry read inside an arm would make the table an array in memory)
+    static __device__ __forceinline__ O pick(bool c, O a, O b) { return c ? a : b; }
+    template <typename T, int s0, int s1, int s2>
+    __device__ __forceinline__ O at(int x, int y, int z) const
+    {
+        const bool c0 = s0 != 0 && x == (s0 < 0 ? 0 : 7);
+        const bool c1 = s1 != 0 && y == (s1 < 0 ? 0 : 7);
+        const bool c2 = s2 != 0 && z == (s2 < 0 ? 0 : 7);
+        O t = c[13];
+        if constexpr (s0 != 0) t = pick(c0, c[13 + s0], t);
+        if constexpr (s1 != 0) t = pick(c1, c[13 + 3 * s1], t);
+        if constexpr (s2 != 0) t = pick(c2, c[13 + 9 * s2], t);
+        if constexpr (s0 != 0 && s1 != 0) t = pick(c0 && c1, c[13 + s0 + 3 * s1], t);
+        if constexpr (s0 != 0 && s2 != 0) t = pick(c0 && c2, c[13 + s0 + 9 * s2], t);
+        if constexpr (s1 != 0 && s2 != 0) t = pick(c1 && c2, c[13 + 3 * s1 + 9 * s2], t);
+        if constexpr (s0 != 0 && s1 != 0 && s2 != 0) t = pick(c0 && c1 && c2, c[13 + s0 + 3 * s1 + 9 * s2], t);
+        return t + (O)((((x + s0) & 7) + 8 * ((y + s1) & 7) + 64 * ((z + s2) & 7)) * (int)sizeof(T));
+    }
+};
+
 template <int q>
 struct QI {
     static constexpr int value = q;

@@ -201,7 +201,7 @@ __device__ __forceinline__ void bulk_voxel(const typename Stor<S>::T* __restrict
 // media: the link contributes the voxel's own opposite population only);
 // no NX_FLAG_OPEN -- every masked link has an upstream voxel; NX_FLAG_MIXED
 // -- per-link validity from the neighbour block's active mask.
-template <int S, int CM, bool FORCE>
+template <int S, int CM, bool FORCE, bool NARROW>
 __global__ void __launch_bounds__(kBV)
     k_step(const typename Stor<S>::T* __restrict__ fin, typename Stor<S>::T* __restrict__ fout,
            const uint32_t* __restrict__ flags, BGeom g, Par p, int remap)
@@ -217,6 +217,8 @@ __global__ void __launch_bounds__(kBV)
         (uint64_t)g.masks[(uint64_t)b * 16 + 2 * (uint32_t)z] |
         ((uint64_t)g.masks[(uint64_t)b * 16 + 2 * (uint32_t)z + 1] << 32);
     const Conn cb = load_conn(g.conn, b);
+    Rows<uint32_t> rows;
+    if constexpr (NARROW) rows = Rows<uint32_t>::of<T, Q>(cb, b);
     const bool active = (plane_bits >> (v & 63u)) & 1u;
     // voxels sharing this voxel's 128-byte line of each population plane
     constexpr uint32_t kLine = 128u / sizeof(T);
@@ -226,16 +228,16 @@ __global__ void __launch_bounds__(kBV)
     T val[Q];
     if (active) {
         fl = flags[(uint64_t)b * kBV + v];
-        for_q(AllQ{}, [&](auto qc) {
+        for_q(AllQ{}, [&](auto qc) __attribute__((always_inline)) {
             constexpr int q = decltype(qc)::value;
-            if constexpr (q == 9) {
+            if constexpr (NARROW) {
+                val[q] = *(const T*)((const char*)(fin + q * kBV) + rows.template at<T, -CX[q], -CY[q], -CZ[q]>(x, y, z));
+            } else if constexpr (q == 9) {
                 val[9] = fin[own + 9 * kBV];
             } else {
                 uint32_t t, nv;
                 upstream<q>(b, cb, x, y, z, t, nv);
-                const uint64_t a =
-                    t != kInvalidBlock ? (uint64_t)t * kBStride + (uint32_t)q * kBV + nv : own;
-                val[q] = fin[a];
+                val[q] = fin[t != kInvalidBlock ? (uint64_t)t * kBStride + (uint32_t)q * kBV + nv : own];
             }
         });
 #pragma unroll
@@ -243,7 +245,15 @@ __global__ void __launch_bounds__(kBV)
         nx_pin(fl);
     }
     if (active && cls_of(fl) == NX_CELL_BULK) {
-        bulk_voxel<S, CM, FORCE>(fin, fout, g, p, b, cb, x, y, z, own, fl, val);
+        int xl = x, yl = y, zl = z;
+        if constexpr (NARROW) {
+            // (opaque copies: the offsets of the loads do not stay in registers
+            // for the few links that want them again)
+            nx_pin(xl);
+            nx_pin(yl);
+            nx_pin(zl);
+        }
+        bulk_voxel<S, CM, FORCE>(fin, fout, g, p, b, cb, xl, yl, zl, own, fl, val);
     } else if (!active && line_any) {
         // inactive voxel in a line that also holds active voxels: write the
         // inactive value so the line is written whole
@@ -950,12 +960,22 @@ extern "C" int nx_d3q19_step_block(const nx_block_desc* d, const void* fin, void
                     return;
                 }
             }
-            if (force)
-                hipLaunchKernelGGL((k_step<S, CM, true>), dim3(g.n_blocks), dim3(kBV), 0, st,
-                                   (const T*)fin, (T*)fout, flags, g, par, g_block_remap);
-            else
-                hipLaunchKernelGGL((k_step<S, CM, false>), dim3(g.n_blocks), dim3(kBV), 0, st,
-                                   (const T*)fin, (T*)fout, flags, g, par, g_block_remap);
+            auto go = [&](auto fc, auto nc) {
+                hipLaunchKernelGGL((k_step<S, CM, decltype(fc)::value, decltype(nc)::value>), dim3(g.n_blocks), dim3(kBV),
+                                   0, st, (const T*)fin, (T*)fout, flags, g, par, g_block_remap);
+            };
+            // 32-bit byte offsets for 2-byte storage where the populations fit
+            // 4 GiB: that step is bound by its instructions (320^3 porous, 597
+            // -> 540 us); the wider ones, bound by HBM, ran 1-2% slower so
+            if constexpr (sizeof(T) == 2) {
+                if ((uint64_t)g.n_blocks * kBStride * sizeof(T) < (1ull << 32)) {
+                    if (force) go(std::true_type{}, std::true_type{});
+                    else go(std::false_type{}, std::true_type{});
+                    return;
+                }
+            }
+            if (force) go(std::true_type{}, std::false_type{});
+            else go(std::false_type{}, std::false_type{});
         }))
         return e;
     NX_CHECK_LAUNCH("k_step(block)");

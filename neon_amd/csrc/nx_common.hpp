@@ -276,6 +276,21 @@ __device__ __forceinline__ void zouhe_bgk(R f[Q], int face, bool velocity, R val
 // acceleration g, force density rho*g:
 //   u = sum c f / rho + g/2 ;  out = (1-omega) f + omega feq(rho,u)
 //       + (1-omega/2) w rho [3 (c-u).g + 9 (c.u)(c.g)]
+// The 19 evaluations share what is equal: c.u and c.g of the opposite
+// direction are exactly the negatives, and terms times a zero component of c
+// (+-0) are left out, which halves the instructions of the collision (it
+// bounds the 2-byte block step).
+template <typename R>
+__device__ __forceinline__ R dot_c(int q, R a0, R a1, R a2)
+{
+    R s = R(0);
+    bool first = true;
+    if (CX[q]) s = CX[q] > 0 ? a0 : -a0, first = false;
+    if (CY[q]) s = first ? (CY[q] > 0 ? a1 : -a1) : (CY[q] > 0 ? s + a1 : s - a1), first = false;
+    if (CZ[q]) s = first ? (CZ[q] > 0 ? a2 : -a2) : (CZ[q] > 0 ? s + a2 : s - a2);
+    return s;
+}
+
 template <typename R>
 __device__ __forceinline__ void bgk_forced(const R f[Q], R omega, R g0, R g1, R g2, R out[Q])
 {
@@ -288,14 +303,17 @@ __device__ __forceinline__ void bgk_forced(const R f[Q], R omega, R g0, R g1, R 
     const R ug = u0 * g0 + u1 * g1 + u2 * g2;
     const R fpre = R(1) - R(0.5) * omega;
 #pragma unroll
-    for (int q = 0; q < Q; q++) {
-        const R w = R(wq(q));
-        const R cu = R(CX[q]) * u0 + R(CY[q]) * u1 + R(CZ[q]) * u2;
-        const R cg = R(CX[q]) * g0 + R(CY[q]) * g1 + R(CZ[q]) * g2;
-        const R eq = rho * w * (R(1) + R(3) * cu + R(4.5) * cu * cu - usqr);
-        const R src = fpre * w * rho * (R(3) * (cg - ug) + R(9) * cu * cg);
-        out[q] = (R(1) - omega) * f[q] + omega * eq + src;
+    for (int i = 0; i < 9; i++) {
+        const R w = R(wq(i + 10)), rw = rho * w, fw = fpre * w * rho;
+        const R cu = dot_c<R>(i + 10, u0, u1, u2), cg = dot_c<R>(i + 10, g0, g1, g2);
+        const R cu3 = R(3) * cu, sq = R(4.5) * cu * cu, cross = R(9) * cu * cg;
+        const R eqp = rw * (R(1) + cu3 + sq - usqr), eqm = rw * (R(1) - cu3 + sq - usqr);
+        const R srcp = fw * (R(3) * (cg - ug) + cross), srcm = fw * (R(3) * (-cg - ug) + cross);
+        out[i] = (R(1) - omega) * f[i] + omega * eqm + srcm;
+        out[i + 10] = (R(1) - omega) * f[i + 10] + omega * eqp + srcp;
     }
+    const R w = R(wq(9));
+    out[9] = (R(1) - omega) * f[9] + omega * (rho * w * (R(1) - usqr)) + fpre * w * rho * (R(3) * -ug);
 }
 
 // Deviation form (project-defined): d = f - w_q.  rho = 1 + sum d,
@@ -364,15 +382,18 @@ __device__ __forceinline__ void bgk_forced_dev(const R d[Q], R omega, R g0, R g1
     const R ug = u0 * g0 + u1 * g1 + u2 * g2;
     const R fpre = R(1) - R(0.5) * omega;
 #pragma unroll
-    for (int q = 0; q < Q; q++) {
-        const R w = R(wq(q));
-        const R cu = R(CX[q]) * u0 + R(CY[q]) * u1 + R(CZ[q]) * u2;
-        const R cg = R(CX[q]) * g0 + R(CY[q]) * g1 + R(CZ[q]) * g2;
-        const R poly = fmaR(cu, fmaR(R(4.5), cu, R(3.)), -usqr);
-        const R deq = fmaR(rho * w, poly, w * drho);
-        const R src = fpre * w * rho * (R(3) * (cg - ug) + R(9) * cu * cg);
-        out[q] = fmaR(omega, deq - d[q], d[q]) + src;
+    for (int i = 0; i < 9; i++) {
+        const R w = R(wq(i + 10)), rw = rho * w, wd = w * drho, fw = fpre * w * rho;
+        const R cu = dot_c<R>(i + 10, u0, u1, u2), cg = dot_c<R>(i + 10, g0, g1, g2);
+        const R cross = R(9) * cu * cg;
+        const R deqp = fmaR(rw, fmaR(cu, fmaR(R(4.5), cu, R(3.)), -usqr), wd);
+        const R deqm = fmaR(rw, fmaR(-cu, fmaR(R(4.5), -cu, R(3.)), -usqr), wd);
+        const R srcp = fw * (R(3) * (cg - ug) + cross), srcm = fw * (R(3) * (-cg - ug) + cross);
+        out[i] = fmaR(omega, deqm - d[i], d[i]) + srcm;
+        out[i + 10] = fmaR(omega, deqp - d[i + 10], d[i + 10]) + srcp;
     }
+    const R w = R(wq(9));
+    out[9] = fmaR(omega, fmaR(rho * w, -usqr, w * drho) - d[9], d[9]) + fpre * w * rho * (R(3) * -ug);
 }
 
 template <int S, int CM, bool FORCE>
