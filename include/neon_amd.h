@@ -317,7 +317,8 @@ int nx_d3q19_wall_mask_block(const nx_block_desc* d, const uint32_t* flags_in,
 int nx_d3q19_step_block(const nx_block_desc* d, const void* fin, void* fout,
                         const uint32_t* flags, const nx_lbm_params* p, nx_stream s);
 /* Block-to-XCD assignment of nx_d3q19_step_block (1: each XCD walks one
- * contiguous range of blocks, the default; 0: hardware round-robin).  No
+ * contiguous range of blocks, or runs of neighbouring blocks where the fields
+ * leave the last-level cache, the default; 0: hardware round-robin).  No
  * counterpart in the reference. */
 int nx_d3q19_set_block_remap(int on);
 /* Lanes of nx_d3q19_step_block at 2-byte storage (NX_F16DEV): 1 -- two

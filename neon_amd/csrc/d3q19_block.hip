@@ -207,7 +207,7 @@ __global__ void __launch_bounds__(kBV)
            const uint32_t* __restrict__ flags, BGeom g, Par p, int remap)
 {
     using T = typename Stor<S>::T;
-    const uint32_t b = remap ? xcd_remap(blockIdx.x, gridDim.x) : blockIdx.x;
+    const uint32_t b = remap ? xcd_order<4, 2 * kBStride * sizeof(T)>(blockIdx.x, gridDim.x) : blockIdx.x;
     const uint32_t v = threadIdx.x;
     const int x = (int)(v & 7u), y = (int)((v >> 3) & 7u), z = (int)(v >> 6);
     const uint64_t own = (uint64_t)b * kBStride + v;
@@ -854,7 +854,10 @@ int check(const nx_block_desc* d)
 template <int V>
 using IC = std::integral_constant<int, V>;
 
-// 1: contiguous range of blocks per XCD (nx_d3q19_set_block_remap)
+// 1: one contiguous range of blocks per XCD, or, in the per-block step beyond
+// the last-level cache, runs of 4 blocks (320^3 sphere pack, binary32 711 us,
+// binary64 1374; ranges 747 and 1422, one by one 760 and 1414; 64^3 binary32
+// the other way, 10.6 against 9.9) (nx_d3q19_set_block_remap)
 int g_block_remap = 1;
 // 1: 2-byte storage steps two voxels per lane (nx_d3q19_set_block_pairs)
 int g_block_pairs = 0;

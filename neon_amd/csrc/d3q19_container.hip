@@ -53,7 +53,8 @@ struct nx_container_s {
     // graph of 2 * kPairSteps steps alternating this container and `pair_with`
     hipGraphExec_t pair_graph = nullptr;
     const nx_container_s* pair_with = nullptr;
-    nx_tuning pair_tuning[2] = {};
+    nx_tuning pair_tuning = {};
+    int pair_order = 0;
 };
 
 namespace nx {
@@ -170,6 +171,17 @@ __global__ void __launch_bounds__(kCWG)
     if (bad) *mismatch = 1u;
 }
 
+// Order of the workgroups over the XCDs: 0 as launched, 1 one contiguous slab
+// per XCD, 2 in runs of 16 bytes of each lane's populations.
+template <int BYTES>
+__device__ __forceinline__ uint32_t order_of(int order)
+{
+    constexpr uint32_t C = 16 / BYTES;
+    return order == 0   ? blockIdx.x
+           : order == 1 ? xcd_remap(blockIdx.x, gridDim.x)
+                        : xcd_runs<C>(blockIdx.x, gridDim.x);
+}
+
 // WG threads, CPT cells per thread (cells base + c*WG), LP = load policy
 // (1: non-temporal), copy_walls as above.
 template <int S, int CM, bool FORCE, bool PER, int WG, int CPT, int LP>
@@ -181,7 +193,7 @@ __global__ void __launch_bounds__(WG)
     using T = typename Stor<S>::T;
     using P = typename Stor<S>::P;
     using R = typename Real<S, CM>::R;
-    const uint32_t wg = remap ? xcd_remap(blockIdx.x, gridDim.x) : blockIdx.x;
+    const uint32_t wg = order_of<sizeof(typename Stor<S>::T)>(remap);
     const uint32_t base = wg * (uint32_t)(WG * CPT) + threadIdx.x;
     uint32_t word[CPT];
     T v[CPT][Q];
@@ -258,7 +270,7 @@ __global__ void __launch_bounds__(WG)
     typedef T VL __attribute__((ext_vector_type(VX), aligned(sizeof(T))));  // dword-aligned load
     typedef T VS __attribute__((ext_vector_type(VX)));                      // aligned store
     static_assert(VX * sizeof(T) == 16 && sizeof(T) >= 4, "16-byte lanes of dword elements");
-    const uint32_t wg = remap ? xcd_remap(blockIdx.x, gridDim.x) : blockIdx.x;
+    const uint32_t wg = order_of<sizeof(typename Stor<S>::T)>(remap);
     const uint32_t i0 = (wg * (uint32_t)WG + threadIdx.x) * (uint32_t)VX;
     if (i0 >= g.n) return;
     const uint32_t word = bits[i0 >> 5];
@@ -359,7 +371,7 @@ __global__ void __launch_bounds__(WG)
     using T = typename Stor<S>::T;
     using P = typename Stor<S>::P;
     using R = typename Real<S, CM>::R;
-    const uint32_t wg = remap ? xcd_remap(blockIdx.x, gridDim.x) : blockIdx.x;
+    const uint32_t wg = order_of<sizeof(typename Stor<S>::T)>(remap);
     const uint32_t i = wg * (uint32_t)WG + threadIdx.x;
     const uint32_t ic = min(i, g.n - 1u);
     uint32_t fl = BITMAP ? bits[ic >> 5] : flags[ic];
@@ -444,7 +456,7 @@ __global__ void __launch_bounds__(WG)
     // masks of the populations with c_x = +1 and c_x = -1
     constexpr uint32_t MP = (1u << 10) | (1u << 13) | (1u << 14) | (1u << 15) | (1u << 16);
     constexpr uint32_t MM = (1u << 0) | (1u << 3) | (1u << 4) | (1u << 5) | (1u << 6);
-    const uint32_t wg = remap ? xcd_remap(blockIdx.x, gridDim.x) : blockIdx.x;
+    const uint32_t wg = order_of<sizeof(typename Stor<S>::T)>(remap);
     const uint32_t i = wg * (uint32_t)WG + threadIdx.x;
     const uint32_t ic = min(i, g.n - 1u);
     int x, y, z;
@@ -545,12 +557,52 @@ __global__ void __launch_bounds__(WG)
 // binary16 (65.6k with uniform x-end walls, vs 51.9k for the bitmap +
 // full-pull kernel); 4- and 8-byte storage keep the bitmap kernels, whose
 // lower register count matters more there (FP32: 35.2k either way).
+constexpr nx_tuning kDefault[4] = {
+    {256, 1, 0, 0, 1, 1}, {256, 1, 0, 0, 1, 2}, {256, 1, 0, 0, 1, 1}, {256, 1, 0, 0, 1, 3}};
 nx_tuning g_tuning[4][3] = {
-    {{256, 1, 0, 0, 1, 1}, {256, 1, 0, 0, 1, 1}, {256, 1, 0, 0, 1, 1}},
-    {{256, 1, 0, 0, 1, 2}, {256, 1, 0, 0, 1, 2}, {256, 1, 0, 0, 1, 2}},
-    {{256, 1, 0, 0, 1, 1}, {256, 1, 0, 0, 1, 1}, {256, 1, 0, 0, 1, 1}},
-    {{256, 1, 0, 0, 1, 3}, {256, 1, 0, 0, 1, 3}, {256, 1, 0, 0, 1, 3}},
+    {kDefault[0], kDefault[0], kDefault[0]},
+    {kDefault[1], kDefault[1], kDefault[1]},
+    {kDefault[2], kDefault[2], kDefault[2]},
+    {kDefault[3], kDefault[3], kDefault[3]},
 };
+
+bool g_tuned[4][3] = {};  // set by the caller or the autotuner
+
+// Launch of one container: the tuned one, or, by the size of its two fields,
+//  * up to 48 MB, a little more than the eight L2s hold: one slab per XCD, so
+//    that a step finds in its L2 what the last one wrote there, and the flag
+//    word directly (48^3 binary32 7.6 -> 6.0 us, binary64 9.5 -> 8.6, binary16
+//    7.7 -> 6.9; 63 x 65 x 61 binary32 10.2 -> 8.9; larger ones lose, 63 x 65 x
+//    61 binary64, 76 MB, 19.6 -> 20.7);
+//  * beyond the 256 MB last-level cache with rows that are no whole lines (128
+//    bytes; half lines do for binary32, 176^3 158 -> 162 us in runs), where
+//    every wavefront's stores end in lines it shares: workgroups in runs, and
+//    for binary32 the edge-speculating kernel, which writes whole wavefronts
+//    (255^3 binary32 744 -> 689 us, binary16 439 -> 404; 250 x 131 x 175
+//    binary32 250 -> 235; binary64 is even and stays);
+//  * otherwise as launched (256^3, in runs of 4: binary32 463 -> 466 us,
+//    binary16 254 -> 256; 129 x 127 x 131 binary16 in slabs 54 -> 56).
+struct Launch {
+    nx_tuning t;
+    int order;
+};
+
+Launch launch_of(const nx_dense_desc& d)
+{
+    Launch l{g_tuning[d.storage][d.compute], 0};
+    l.order = l.t.xcd_remap;
+    if (g_tuned[d.storage][d.compute]) return l;
+    const uint64_t es = d.storage == NX_F64 ? 8 : d.storage == NX_F16DEV ? 2 : 4;
+    const uint64_t both = 2ull * 19 * es * (uint64_t)d.dim[0] * (uint64_t)d.dim[1] * (uint64_t)d.dim[2];
+    if (both <= (48ull << 20)) {
+        l.t.xcd_remap = l.order = 1;
+        if (es == 4) l.t.boundary = 1;
+    } else if (both > (256ull << 20) && es < 8 && (uint64_t)d.dim[0] * es % (es == 2 ? 128 : 64)) {
+        l.order = 2;
+        if (es == 4 && d.compute == NX_COMPUTE_F32 && !d.periodic) l.t.boundary = 3;
+    }
+    return l;
+}
 
 template <int S, int CM>
 constexpr bool tunable()
@@ -572,7 +624,7 @@ bool valid_tuning(const nx_tuning& t, int storage)
 }
 
 template <int S, int CM, bool FORCE, bool PER>
-void launch_fused(const nx_tuning& t, const nx_container_s& c, hipStream_t s)
+void launch_fused(const nx_tuning& t, int remap, const nx_container_s& c, hipStream_t s)
 {
     using T = typename Stor<S>::T;
     auto go = [&](auto wgc, auto cptc, auto lpc) {
@@ -581,7 +633,7 @@ void launch_fused(const nx_tuning& t, const nx_container_s& c, hipStream_t s)
         const uint32_t nb = (c.g.n + WG * CPT - 1) / (WG * CPT);
         hipLaunchKernelGGL((k_fused<S, CM, FORCE, PER, WG, CPT, LP>), dim3(nb), dim3(WG), 0, s,
                            (const T*)c.fin, (T*)c.fout, c.flags, c.interior, c.g, c.p,
-                           t.xcd_remap, c.copy_walls);
+                           remap, c.copy_walls);
     };
     if (t.boundary >= 1 && t.boundary <= 3) {
         auto go_fix = [&](auto wgc, auto lpc) {
@@ -590,15 +642,15 @@ void launch_fused(const nx_tuning& t, const nx_container_s& c, hipStream_t s)
             if (t.boundary == 3)
                 hipLaunchKernelGGL((k_fused_edge<S, CM, FORCE, PER, WG, LP>), dim3(nb), dim3(WG), 0, s,
                                    (const T*)c.fin, (T*)c.fout, c.flags, c.interior, c.g, c.p,
-                                   t.xcd_remap, c.copy_walls, c.xwall_uniform, c.xwall);
+                                   remap, c.copy_walls, c.xwall_uniform, c.xwall);
             else if (t.boundary == 2)
                 hipLaunchKernelGGL((k_fused_fix<S, CM, FORCE, PER, WG, LP, true>), dim3(nb), dim3(WG), 0, s,
                                    (const T*)c.fin, (T*)c.fout, c.flags, c.interior, c.g, c.p,
-                                   t.xcd_remap, c.copy_walls);
+                                   remap, c.copy_walls);
             else
                 hipLaunchKernelGGL((k_fused_fix<S, CM, FORCE, PER, WG, LP, false>), dim3(nb), dim3(WG), 0, s,
                                    (const T*)c.fin, (T*)c.fout, c.flags, c.interior, c.g, c.p,
-                                   t.xcd_remap, c.copy_walls);
+                                   remap, c.copy_walls);
         };
         if constexpr (tunable<S, CM>() && !FORCE && !PER) {
             auto by_lp = [&](auto wgc) {
@@ -621,7 +673,7 @@ void launch_fused(const nx_tuning& t, const nx_container_s& c, hipStream_t s)
             const uint32_t nb = (lanes + WG - 1) / WG;
             hipLaunchKernelGGL((k_fused_vx<S, CM, FORCE, PER, WG, VX, LP>), dim3(nb), dim3(WG), 0, s,
                                (const T*)c.fin, (T*)c.fout, c.flags, c.interior, c.g, c.p,
-                               t.xcd_remap, c.copy_walls);
+                               remap, c.copy_walls);
         };
         if constexpr (tunable<S, CM>() && !FORCE && !PER) {
             auto by_lp = [&](auto wgc) {
@@ -652,18 +704,18 @@ void launch_fused(const nx_tuning& t, const nx_container_s& c, hipStream_t s)
     }
 }
 
-int run_container(const nx_container_s& c, const nx_tuning& t, hipStream_t s)
+int run_container(const nx_container_s& c, const nx_tuning& t, int remap, hipStream_t s)
 {
     if (int e = by_type(&c.d, [&](auto sc, auto cc) {
             constexpr int S = decltype(sc)::value;
             constexpr int CM = decltype(cc)::value;
             const bool per = c.g.periodic != 0;
             if (c.force) {
-                if (per) launch_fused<S, CM, true, true>(t, c, s);
-                else launch_fused<S, CM, true, false>(t, c, s);
+                if (per) launch_fused<S, CM, true, true>(t, remap, c, s);
+                else launch_fused<S, CM, true, false>(t, remap, c, s);
             } else {
-                if (per) launch_fused<S, CM, false, true>(t, c, s);
-                else launch_fused<S, CM, false, false>(t, c, s);
+                if (per) launch_fused<S, CM, false, true>(t, remap, c, s);
+                else launch_fused<S, CM, false, false>(t, remap, c, s);
             }
         }))
         return e;
@@ -790,7 +842,8 @@ extern "C" int nx_d3q19_iteration_dense(const nx_dense_desc* d, const void* fin,
 extern "C" int nx_container_run(nx_container c, nx_stream s)
 {
     if (!c) return set_error(NX_ERR_INVALID, "null container");
-    return run_container(*c, g_tuning[c->d.storage][c->d.compute], (hipStream_t)s);
+    const Launch l = launch_of(c->d);
+    return run_container(*c, l.t, l.order, (hipStream_t)s);
 }
 
 extern "C" int nx_container_info(nx_container c, uint64_t* n_interior, uint64_t* n_boundary,
@@ -829,11 +882,12 @@ extern "C" int nx_container_run_pair(nx_container a, nx_container b, int32_t n_s
         a->fout != b->fin)
         return set_error(NX_ERR_INVALID, "run_pair: b must step b's input back into a's input");
     const hipStream_t st = (hipStream_t)s;
-    const nx_tuning& t = g_tuning[a->d.storage][a->d.compute];
+    const Launch l = launch_of(a->d);
+    const nx_tuning& t = l.t;
     int32_t done = 0;
     if (st != nullptr && n_steps >= 2 * kPairSteps) {
         const bool same = a->pair_graph && a->pair_with == b &&
-                          !memcmp(&a->pair_tuning[0], &t, sizeof(t));
+                          !memcmp(&a->pair_tuning, &t, sizeof(t)) && a->pair_order == l.order;
         if (!same) {
             if (a->pair_graph) hipGraphExecDestroy(a->pair_graph);
             a->pair_graph = nullptr;
@@ -841,8 +895,8 @@ extern "C" int nx_container_run_pair(nx_container a, nx_container b, int32_t n_s
             NX_CHECK_HIP(hipStreamBeginCapture(st, hipStreamCaptureModeThreadLocal));
             int e = 0;
             for (int k = 0; k < kPairSteps && !e; k++) {
-                e = run_container(*a, t, st);
-                if (!e) e = run_container(*b, t, st);
+                e = run_container(*a, t, l.order, st);
+                if (!e) e = run_container(*b, t, l.order, st);
             }
             const hipError_t ec = hipStreamEndCapture(st, &g);
             if (e) {
@@ -854,13 +908,14 @@ extern "C" int nx_container_run_pair(nx_container a, nx_container b, int32_t n_s
             hipGraphDestroy(g);
             NX_CHECK_HIP(ei);
             a->pair_with = b;
-            a->pair_tuning[0] = t;
+            a->pair_tuning = t;
+            a->pair_order = l.order;
         }
         for (; done + 2 * kPairSteps <= n_steps; done += 2 * kPairSteps)
             NX_CHECK_HIP(hipGraphLaunch(a->pair_graph, st));
     }
     for (; done < n_steps; done++)
-        if (int e = run_container(done % 2 == 0 ? *a : *b, t, st)) return e;
+        if (int e = run_container(done % 2 == 0 ? *a : *b, t, l.order, st)) return e;
     return NX_OK;
 }
 
@@ -881,6 +936,8 @@ extern "C" int nx_d3q19_set_tuning_dense(const nx_dense_desc* d, const nx_tuning
                          "{0,1}, vx = 1 or 16 bytes of cells (2 f64, 4 f32), boundary in {0,1,2,3} "
                          "(1 and 2 need vx = 1)");
     g_tuning[d->storage][d->compute] = *t;
+    // setting the default again gives the choice back to launch_of
+    g_tuned[d->storage][d->compute] = memcmp(t, &kDefault[d->storage], sizeof(*t)) != 0;
     return NX_OK;
 }
 
@@ -907,10 +964,10 @@ extern "C" int nx_container_autotune(nx_container c, nx_stream s, nx_tuning* bes
                     if ((vx > 1 || bd) && cpt == 2) continue;  // one cell (or lane of VX cells) per thread
                     const nx_tuning t{wg, cpt, lp, rm, vx, bd};
                     for (int r = 0; r < 3; r++)
-                        if (int e = run_container(*c, t, (hipStream_t)s)) return e;
+                        if (int e = run_container(*c, t, t.xcd_remap, (hipStream_t)s)) return e;
                     NX_CHECK_HIP(hipEventRecord(e0, (hipStream_t)s));
                     for (int r = 0; r < reps; r++)
-                        if (int e = run_container(*c, t, (hipStream_t)s)) return e;
+                        if (int e = run_container(*c, t, t.xcd_remap, (hipStream_t)s)) return e;
                     NX_CHECK_HIP(hipEventRecord(e1, (hipStream_t)s));
                     NX_CHECK_HIP(hipEventSynchronize(e1));
                     float ms = 0;
@@ -924,6 +981,7 @@ extern "C" int nx_container_autotune(nx_container c, nx_stream s, nx_tuning* bes
     hipEventDestroy(e0);
     hipEventDestroy(e1);
     slot = bt;
+    g_tuned[c->d.storage][c->d.compute] = true;
     if (best) *best = bt;
     if (best_ms) *best_ms = bms;
     return NX_OK;

@@ -5,10 +5,10 @@
 // 256 cells (4 wavefronts) per workgroup over the linear cell index, so every
 // population load and store of a wavefront is one contiguous 64-cell run;
 // the +-1 x shifts of the pull read a neighbouring cache line that the
-// adjacent wavefront of the same workgroup fetches anyway.  Workgroups are
-// remapped so each XCD walks a contiguous slab (L2 keeps the row-boundary
-// lines).  Each population is read once and written once per step:
-// 2*19*sizeof(storage) bytes per cell update.
+// adjacent wavefront of the same workgroup fetches anyway.  Workgroups reach
+// the XCDs in runs or slabs (L2 keeps the row-boundary lines).  Each population
+// is read once and written once per step: 2*19*sizeof(storage) bytes per cell
+// update.
 #include <cmath>
 #include <mutex>
 #include <string>
@@ -19,6 +19,16 @@ namespace nx {
 namespace dense {
 namespace {
 
+// Beyond the last-level cache workgroups reach the XCDs in runs of 16 (512 x
+// 128 x 128 duct, binary32 / binary64: 232 / 463 us; one contiguous slab per
+// XCD 241 / 509, one by one 237 / 470; 301 x 77 x 101 96 / 172 against 101 / 186
+// and 99 / 172; the cavity step of 200^3 binary16 152 -> 127).
+template <int S>
+__device__ __forceinline__ uint32_t order()
+{
+    return xcd_order<16, 2 * Q * kWG * sizeof(typename Stor<S>::T)>(blockIdx.x, gridDim.x);
+}
+
 // Generic step (any boundary mode, including periodic wrap).
 template <int S, int CM, bool FORCE, bool PERIODIC>
 __global__ void __launch_bounds__(kWG)
@@ -26,7 +36,7 @@ __global__ void __launch_bounds__(kWG)
            const uint32_t* __restrict__ flags, DGeom g, Par p)
 {
     using R = typename Real<S, CM>::R;
-    const uint32_t i = xcd_remap(blockIdx.x, gridDim.x) * kWG + threadIdx.x;
+    const uint32_t i = order<S>() * kWG + threadIdx.x;
     if (i >= g.n) return;
     const uint32_t fl = __builtin_nontemporal_load(&flags[i]);
     if (cls_of(fl) != NX_CELL_BULK) return;
@@ -53,7 +63,7 @@ __global__ void __launch_bounds__(kWG)
               const uint32_t* __restrict__ flags, DGeom g, Par p, ZhValues zh)
 {
     using R = typename Real<S, CM>::R;
-    const uint32_t i = xcd_remap(blockIdx.x, gridDim.x) * kWG + threadIdx.x;
+    const uint32_t i = order<S>() * kWG + threadIdx.x;
     if (i >= g.n) return;
     const uint32_t fl = __builtin_nontemporal_load(&flags[i]);
     if (cls_of(fl) != NX_CELL_BULK) return;

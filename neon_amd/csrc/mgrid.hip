@@ -368,7 +368,7 @@ __global__ void __launch_bounds__(kBV)
 {
     using T = typename MS<S>::T;
     constexpr int NQ = LT::Q;
-    const uint32_t b = xcd_remap(blockIdx.x, gridDim.x), v = threadIdx.x;  // neighbour blocks share an XCD's L2
+    const uint32_t b = xcd_runs<4>(blockIdx.x, gridDim.x), v = threadIdx.x;
     const uint32_t st = state[(uint64_t)b * kBV + v];
     if (!(st & kActive) || cls_bits(st) != NX_CELL_BULK) return;
     const uint64_t own = (uint64_t)b * (NQ * kBV) + v;
@@ -473,8 +473,9 @@ __global__ void __launch_bounds__(kBV, (StreamShape<S, LT>::waves))
         store_entry(fout, sa, blockIdx.x * kBV + threadIdx.x);
         return;
     }
-    // neighbour blocks share an XCD's L2
-    const uint32_t b = xcd_remap(blockIdx.x - sa.groups, gridDim.x - sa.groups), v = threadIdx.x;
+    // runs of 4 blocks per XCD (240^3 lid: BGK f32 974 us a coarse step, f64
+    // 1764, KBC f32 1845; one range per XCD 1043, 1830, 1896)
+    const uint32_t b = xcd_runs<4>(blockIdx.x - sa.groups, gridDim.x - sa.groups), v = threadIdx.x;
     const Rows<O> rows = Rows<O>::template of<T, NQ>(load_conn(conn, b), b);
     const int x = (int)(v & 7u), y = (int)((v >> 3) & 7u), z = (int)(v >> 6);
     const O own = rows.c[13] + (O)(v * sizeof(T));
