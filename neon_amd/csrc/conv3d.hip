@@ -2,14 +2,13 @@
 // matrix cores, FP32 accumulation (the learned warm start's network).  No
 // counterpart in the reference.
 //
-// All three are implicit GEMMs.  On grids whose rows hold >= 32 voxels the
-// operands are staged in LDS (the input block with its halo for the forward); smaller grids
-// read their fragments straight from global memory (the 27-fold reuse of
-// every input voxel served by L1/L2):
+// All three are implicit GEMMs:
 //   forward      M = voxels, N = cout, K = taps*cin      (A: 8 channels of one
 //                tap per lane = one 16-byte load; B: 8 weights, 16 bytes);
-//                for rows of >= 32 voxels the input block with its halo is
-//                staged in LDS, 16 channels at a time (k_fwd_tile)
+//                the input block with its halo is staged in LDS (k_fwd_blk, and
+//                k_fwd_y16 for 16 channels); rows of 1 or 2 voxels read their
+//                fragments from global memory (k_fwd), 1^3 kernels need no
+//                halo (k_pw)
 //   bwd-data     the forward on the flipped, transposed weights
 //   bwd-weight   M = cout, N = cin, K = voxels (split over workgroups,
 //                FP32 partials, fixed-order reduction): all 27 taps from one
