@@ -34,12 +34,13 @@ CASES = [  # (shape n,d,h,w), cin, cout, ks
     ((3, 4, 2, 4), 96, 48, 3),
 ]
 
-# rows of >= 32 voxels: the all-taps weight-gradient kernel (k_bwd_w27),
-# including 1, 3 and 4 output-channel tiles and several input-channel blocks
+# rows of >= 32 voxels: the all-taps weight gradient (k_bwd_wr), with 1, 3 and
+# 4 output-channel blocks and several input-channel blocks
 WIDE = [((1, 4, 4, 32), 16, 16, 3), ((2, 2, 4, 64), 48, 16, 3), ((1, 4, 2, 32), 32, 64, 3),
         ((1, 2, 2, 32), 16, 48, 3), ((2, 2, 2, 64), 96, 32, 3)]
-# blocks of 32 x 4 x 4 voxels: the LDS-tiled forward, 16 input channels at a
-# time (k_fwd_tile; also the backward-data pass of these layers)
+# blocks of 32 x 4 x 4 voxels: the staged forward (k_fwd_blk, 32 channels and a
+# last 16 at a time, one or two output-channel blocks) and, for 16 input
+# channels, the march along z (k_fwd_z16); also the backward-data pass
 TILED = [((1, 4, 4, 32), 16, 48, 3), ((2, 4, 4, 32), 32, 64, 3), ((1, 8, 8, 64), 16, 16, 3),
          ((1, 4, 4, 64), 32, 32, 3), ((1, 4, 4, 32), 48, 32, 3), ((2, 4, 4, 64), 48, 16, 3),
          ((1, 4, 8, 32), 96, 32, 3)]

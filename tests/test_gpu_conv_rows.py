@@ -1,6 +1,8 @@
-"""The row-marching convolution kernels at the edges of their tiles, against
-the FP64 oracle: rows of 4 to 64 voxels, fewer rows or planes than a tile, two
-tiles along z, channel counts that end in a 16-channel slice, and infinities.
+"""The staged convolution kernels at the edges of their tiles, against the FP64
+oracle: rows of 4 to 64 voxels, fewer rows or planes than a tile, two tiles
+along z, channel counts that end in a 16-channel slice, and infinities; and
+runs of several rows, planes and chunks that end inside a column, a plane and a
+sample.
 
 Tolerance: as tests/test_gpu_conv.py -- every output sums at most 27 * 256
 products in FP32, so it lies within 1e-5 of the sum of their magnitudes."""
@@ -14,6 +16,12 @@ pytestmark = pytest.mark.gpu
 SHAPES = [((1, 16, 16, 16), 80, 32), ((1, 32, 4, 16), 16, 48), ((1, 1, 1, 16), 32, 32), ((2, 64, 2, 8), 48, 16),
           ((1, 2, 1, 4), 48, 16), ((1, 4, 8, 4), 80, 32), ((1, 16, 4, 32), 48, 16), ((1, 2, 16, 32), 16, 48),
           ((3, 1, 1, 64), 16, 32), ((1, 16, 8, 64), 16, 16), ((2, 8, 2, 32), 112, 16)]
+# Work of one workgroup: k_fwd_z16 3 planes of 8 (640 planes over 256 runs);
+# k_bwd_wr 7 chunks = 3.5 rows of 64 voxels (5,120 chunks, 768 splits) and 7
+# rows of 32 (1,280, 192 splits); k_bwd_wc the partials of a slice, each 3 of 11
+# chunks (768 chunks, 70 splits), on rows of 8 and 4 one of 4
+RUNS = [((5, 8, 64, 64), 16, 16), ((5, 8, 32, 32), 64, 32), ((6, 16, 16, 16), 32, 64), ((8, 16, 8, 8), 64, 32),
+        ((8, 16, 8, 4), 48, 64)]
 
 
 def _bf(rng, shape, scale=1.0):
@@ -21,7 +29,7 @@ def _bf(rng, shape, scale=1.0):
     return bits, U.from_bf16_bits(bits)
 
 
-@pytest.mark.parametrize("shape,cin,cout", SHAPES)
+@pytest.mark.parametrize("shape,cin,cout", SHAPES + RUNS)
 def test_rows_vs_oracle(nx, shape, cin, cout):
     from neon_amd import surrogate as S
     rng = np.random.default_rng(cin + cout)
