@@ -54,7 +54,6 @@ struct nx_container_s {
     hipGraphExec_t pair_graph = nullptr;
     const nx_container_s* pair_with = nullptr;
     nx_tuning pair_tuning = {};
-    int pair_order = 0;
 };
 
 namespace nx {
@@ -172,14 +171,15 @@ __global__ void __launch_bounds__(kCWG)
 }
 
 // Order of the workgroups over the XCDs: 0 as launched, 1 one contiguous slab
-// per XCD, 2 in runs of 16 bytes of each lane's populations.
+// per XCD, 2 (2-byte storage) in runs of 8.  Wider storage has no third way: its
+// three-way choice at the head of the kernel cost the binary32 bitmap kernel up
+// to 3 percent (48 x 234 x 86 34.4 -> 35.4 us), and runs earned 2 there.
 template <int BYTES>
 __device__ __forceinline__ uint32_t order_of(int order)
 {
-    constexpr uint32_t C = 16 / BYTES;
-    return order == 0   ? blockIdx.x
-           : order == 1 ? xcd_remap(blockIdx.x, gridDim.x)
-                        : xcd_runs<C>(blockIdx.x, gridDim.x);
+    if constexpr (BYTES == 2)
+        if (order == 2) return xcd_runs<8>(blockIdx.x, gridDim.x);
+    return order ? xcd_remap(blockIdx.x, gridDim.x) : blockIdx.x;
 }
 
 // WG threads, CPT cells per thread (cells base + c*WG), LP = load policy
@@ -557,51 +557,33 @@ __global__ void __launch_bounds__(WG)
 // binary16 (65.6k with uniform x-end walls, vs 51.9k for the bitmap +
 // full-pull kernel); 4- and 8-byte storage keep the bitmap kernels, whose
 // lower register count matters more there (FP32: 35.2k either way).
-constexpr nx_tuning kDefault[4] = {
-    {256, 1, 0, 0, 1, 1}, {256, 1, 0, 0, 1, 2}, {256, 1, 0, 0, 1, 1}, {256, 1, 0, 0, 1, 3}};
 nx_tuning g_tuning[4][3] = {
-    {kDefault[0], kDefault[0], kDefault[0]},
-    {kDefault[1], kDefault[1], kDefault[1]},
-    {kDefault[2], kDefault[2], kDefault[2]},
-    {kDefault[3], kDefault[3], kDefault[3]},
+    {{256, 1, 0, 0, 1, 1}, {256, 1, 0, 0, 1, 1}, {256, 1, 0, 0, 1, 1}},
+    {{256, 1, 0, 0, 1, 2}, {256, 1, 0, 0, 1, 2}, {256, 1, 0, 0, 1, 2}},
+    {{256, 1, 0, 0, 1, 1}, {256, 1, 0, 0, 1, 1}, {256, 1, 0, 0, 1, 1}},
+    {{256, 1, 0, 0, 1, 3}, {256, 1, 0, 0, 1, 3}, {256, 1, 0, 0, 1, 3}},
 };
 
-bool g_tuned[4][3] = {};  // set by the caller or the autotuner
-
-// Launch of one container: the tuned one, or, by the size of its two fields,
-//  * up to 48 MB, a little more than the eight L2s hold: one slab per XCD, so
-//    that a step finds in its L2 what the last one wrote there, and the flag
-//    word directly (48^3 binary32 7.6 -> 6.0 us, binary64 9.5 -> 8.6, binary16
-//    7.7 -> 6.9; 63 x 65 x 61 binary32 10.2 -> 8.9; larger ones lose, 63 x 65 x
-//    61 binary64, 76 MB, 19.6 -> 20.7);
-//  * beyond the 256 MB last-level cache with rows that are no whole lines (128
-//    bytes; half lines do for binary32, 176^3 158 -> 162 us in runs), where
-//    every wavefront's stores end in lines it shares: workgroups in runs, and
-//    for binary32 the edge-speculating kernel, which writes whole wavefronts
-//    (255^3 binary32 744 -> 689 us, binary16 439 -> 404; 250 x 131 x 175
-//    binary32 250 -> 235; binary64 is even and stays);
-//  * otherwise as launched (256^3, in runs of 4: binary32 463 -> 466 us,
-//    binary16 254 -> 256; 129 x 127 x 131 binary16 in slabs 54 -> 56).
-struct Launch {
-    nx_tuning t;
-    int order;
-};
-
-Launch launch_of(const nx_dense_desc& d)
+// Order of the workgroups (order_of).  Where the tuning asks for no slabs it
+// follows the size of the two fields:
+//  * 4- and 8-byte storage up to 48 MB, a little more than the eight L2s hold:
+//    one slab per XCD, so that a step finds in its L2 what the last one wrote
+//    there (binary32 32^3 5.1 -> 4.6 us, 48^3 7.0 -> 5.7, 50 x 117 x 53, 45 MB,
+//    14.5 -> 11.9; binary64 48^3 9.2 -> 8.2).  Above it slabs win and lose
+//    (112 x 37 x 84, 50 MB, 14.4 -> 15.3 us; 36 x 165 x 80, 69 MB, 20.4 -> 18.8);
+//    with 2-byte storage they do at every size (48^3 8.6 -> 7.8, 25 x 164 x 53,
+//    16 MB, 8.6 -> 10.2, 112 x 37 x 84 10.4 -> 11.6);
+//  * 2-byte storage beyond the 256 MB last-level cache with rows that are no
+//    whole 128-byte lines, where every wavefront's stores end in lines it
+//    shares: runs (255^3 431 -> 395 us, 99 x 131 x 277 89 -> 86);
+//  * otherwise as launched.
+int order_for(const nx_dense_desc& d, const nx_tuning& t)
 {
-    Launch l{g_tuning[d.storage][d.compute], 0};
-    l.order = l.t.xcd_remap;
-    if (g_tuned[d.storage][d.compute]) return l;
+    if (t.xcd_remap) return 1;
     const uint64_t es = d.storage == NX_F64 ? 8 : d.storage == NX_F16DEV ? 2 : 4;
     const uint64_t both = 2ull * 19 * es * (uint64_t)d.dim[0] * (uint64_t)d.dim[1] * (uint64_t)d.dim[2];
-    if (both <= (48ull << 20)) {
-        l.t.xcd_remap = l.order = 1;
-        if (es == 4) l.t.boundary = 1;
-    } else if (both > (256ull << 20) && es < 8 && (uint64_t)d.dim[0] * es % (es == 2 ? 128 : 64)) {
-        l.order = 2;
-        if (es == 4 && d.compute == NX_COMPUTE_F32 && !d.periodic) l.t.boundary = 3;
-    }
-    return l;
+    if (es >= 4) return both <= (48ull << 20) ? 1 : 0;
+    return both > (256ull << 20) && (uint64_t)d.dim[0] * es % 128 ? 2 : 0;
 }
 
 template <int S, int CM>
@@ -624,7 +606,7 @@ bool valid_tuning(const nx_tuning& t, int storage)
 }
 
 template <int S, int CM, bool FORCE, bool PER>
-void launch_fused(const nx_tuning& t, int remap, const nx_container_s& c, hipStream_t s)
+void launch_fused(const nx_tuning& t, int order, const nx_container_s& c, hipStream_t s)
 {
     using T = typename Stor<S>::T;
     auto go = [&](auto wgc, auto cptc, auto lpc) {
@@ -633,7 +615,7 @@ void launch_fused(const nx_tuning& t, int remap, const nx_container_s& c, hipStr
         const uint32_t nb = (c.g.n + WG * CPT - 1) / (WG * CPT);
         hipLaunchKernelGGL((k_fused<S, CM, FORCE, PER, WG, CPT, LP>), dim3(nb), dim3(WG), 0, s,
                            (const T*)c.fin, (T*)c.fout, c.flags, c.interior, c.g, c.p,
-                           remap, c.copy_walls);
+                           order, c.copy_walls);
     };
     if (t.boundary >= 1 && t.boundary <= 3) {
         auto go_fix = [&](auto wgc, auto lpc) {
@@ -642,15 +624,15 @@ void launch_fused(const nx_tuning& t, int remap, const nx_container_s& c, hipStr
             if (t.boundary == 3)
                 hipLaunchKernelGGL((k_fused_edge<S, CM, FORCE, PER, WG, LP>), dim3(nb), dim3(WG), 0, s,
                                    (const T*)c.fin, (T*)c.fout, c.flags, c.interior, c.g, c.p,
-                                   remap, c.copy_walls, c.xwall_uniform, c.xwall);
+                                   order, c.copy_walls, c.xwall_uniform, c.xwall);
             else if (t.boundary == 2)
                 hipLaunchKernelGGL((k_fused_fix<S, CM, FORCE, PER, WG, LP, true>), dim3(nb), dim3(WG), 0, s,
                                    (const T*)c.fin, (T*)c.fout, c.flags, c.interior, c.g, c.p,
-                                   remap, c.copy_walls);
+                                   order, c.copy_walls);
             else
                 hipLaunchKernelGGL((k_fused_fix<S, CM, FORCE, PER, WG, LP, false>), dim3(nb), dim3(WG), 0, s,
                                    (const T*)c.fin, (T*)c.fout, c.flags, c.interior, c.g, c.p,
-                                   remap, c.copy_walls);
+                                   order, c.copy_walls);
         };
         if constexpr (tunable<S, CM>() && !FORCE && !PER) {
             auto by_lp = [&](auto wgc) {
@@ -673,7 +655,7 @@ void launch_fused(const nx_tuning& t, int remap, const nx_container_s& c, hipStr
             const uint32_t nb = (lanes + WG - 1) / WG;
             hipLaunchKernelGGL((k_fused_vx<S, CM, FORCE, PER, WG, VX, LP>), dim3(nb), dim3(WG), 0, s,
                                (const T*)c.fin, (T*)c.fout, c.flags, c.interior, c.g, c.p,
-                               remap, c.copy_walls);
+                               order, c.copy_walls);
         };
         if constexpr (tunable<S, CM>() && !FORCE && !PER) {
             auto by_lp = [&](auto wgc) {
@@ -704,18 +686,19 @@ void launch_fused(const nx_tuning& t, int remap, const nx_container_s& c, hipStr
     }
 }
 
-int run_container(const nx_container_s& c, const nx_tuning& t, int remap, hipStream_t s)
+int run_container(const nx_container_s& c, const nx_tuning& t, hipStream_t s)
 {
+    const int order = order_for(c.d, t);
     if (int e = by_type(&c.d, [&](auto sc, auto cc) {
             constexpr int S = decltype(sc)::value;
             constexpr int CM = decltype(cc)::value;
             const bool per = c.g.periodic != 0;
             if (c.force) {
-                if (per) launch_fused<S, CM, true, true>(t, remap, c, s);
-                else launch_fused<S, CM, true, false>(t, remap, c, s);
+                if (per) launch_fused<S, CM, true, true>(t, order, c, s);
+                else launch_fused<S, CM, true, false>(t, order, c, s);
             } else {
-                if (per) launch_fused<S, CM, false, true>(t, remap, c, s);
-                else launch_fused<S, CM, false, false>(t, remap, c, s);
+                if (per) launch_fused<S, CM, false, true>(t, order, c, s);
+                else launch_fused<S, CM, false, false>(t, order, c, s);
             }
         }))
         return e;
@@ -842,8 +825,7 @@ extern "C" int nx_d3q19_iteration_dense(const nx_dense_desc* d, const void* fin,
 extern "C" int nx_container_run(nx_container c, nx_stream s)
 {
     if (!c) return set_error(NX_ERR_INVALID, "null container");
-    const Launch l = launch_of(c->d);
-    return run_container(*c, l.t, l.order, (hipStream_t)s);
+    return run_container(*c, g_tuning[c->d.storage][c->d.compute], (hipStream_t)s);
 }
 
 extern "C" int nx_container_info(nx_container c, uint64_t* n_interior, uint64_t* n_boundary,
@@ -882,12 +864,11 @@ extern "C" int nx_container_run_pair(nx_container a, nx_container b, int32_t n_s
         a->fout != b->fin)
         return set_error(NX_ERR_INVALID, "run_pair: b must step b's input back into a's input");
     const hipStream_t st = (hipStream_t)s;
-    const Launch l = launch_of(a->d);
-    const nx_tuning& t = l.t;
+    const nx_tuning& t = g_tuning[a->d.storage][a->d.compute];
     int32_t done = 0;
     if (st != nullptr && n_steps >= 2 * kPairSteps) {
         const bool same = a->pair_graph && a->pair_with == b &&
-                          !memcmp(&a->pair_tuning, &t, sizeof(t)) && a->pair_order == l.order;
+                          !memcmp(&a->pair_tuning, &t, sizeof(t));
         if (!same) {
             if (a->pair_graph) hipGraphExecDestroy(a->pair_graph);
             a->pair_graph = nullptr;
@@ -895,8 +876,8 @@ extern "C" int nx_container_run_pair(nx_container a, nx_container b, int32_t n_s
             NX_CHECK_HIP(hipStreamBeginCapture(st, hipStreamCaptureModeThreadLocal));
             int e = 0;
             for (int k = 0; k < kPairSteps && !e; k++) {
-                e = run_container(*a, t, l.order, st);
-                if (!e) e = run_container(*b, t, l.order, st);
+                e = run_container(*a, t, st);
+                if (!e) e = run_container(*b, t, st);
             }
             const hipError_t ec = hipStreamEndCapture(st, &g);
             if (e) {
@@ -909,13 +890,12 @@ extern "C" int nx_container_run_pair(nx_container a, nx_container b, int32_t n_s
             NX_CHECK_HIP(ei);
             a->pair_with = b;
             a->pair_tuning = t;
-            a->pair_order = l.order;
         }
         for (; done + 2 * kPairSteps <= n_steps; done += 2 * kPairSteps)
             NX_CHECK_HIP(hipGraphLaunch(a->pair_graph, st));
     }
     for (; done < n_steps; done++)
-        if (int e = run_container(done % 2 == 0 ? *a : *b, t, l.order, st)) return e;
+        if (int e = run_container(done % 2 == 0 ? *a : *b, t, st)) return e;
     return NX_OK;
 }
 
@@ -936,8 +916,6 @@ extern "C" int nx_d3q19_set_tuning_dense(const nx_dense_desc* d, const nx_tuning
                          "{0,1}, vx = 1 or 16 bytes of cells (2 f64, 4 f32), boundary in {0,1,2,3} "
                          "(1 and 2 need vx = 1)");
     g_tuning[d->storage][d->compute] = *t;
-    // setting the default again gives the choice back to launch_of
-    g_tuned[d->storage][d->compute] = memcmp(t, &kDefault[d->storage], sizeof(*t)) != 0;
     return NX_OK;
 }
 
@@ -964,10 +942,10 @@ extern "C" int nx_container_autotune(nx_container c, nx_stream s, nx_tuning* bes
                     if ((vx > 1 || bd) && cpt == 2) continue;  // one cell (or lane of VX cells) per thread
                     const nx_tuning t{wg, cpt, lp, rm, vx, bd};
                     for (int r = 0; r < 3; r++)
-                        if (int e = run_container(*c, t, t.xcd_remap, (hipStream_t)s)) return e;
+                        if (int e = run_container(*c, t, (hipStream_t)s)) return e;
                     NX_CHECK_HIP(hipEventRecord(e0, (hipStream_t)s));
                     for (int r = 0; r < reps; r++)
-                        if (int e = run_container(*c, t, t.xcd_remap, (hipStream_t)s)) return e;
+                        if (int e = run_container(*c, t, (hipStream_t)s)) return e;
                     NX_CHECK_HIP(hipEventRecord(e1, (hipStream_t)s));
                     NX_CHECK_HIP(hipEventSynchronize(e1));
                     float ms = 0;
@@ -981,7 +959,6 @@ extern "C" int nx_container_autotune(nx_container c, nx_stream s, nx_tuning* bes
     hipEventDestroy(e0);
     hipEventDestroy(e1);
     slot = bt;
-    g_tuned[c->d.storage][c->d.compute] = true;
     if (best) *best = bt;
     if (best_ms) *best_ms = bms;
     return NX_OK;

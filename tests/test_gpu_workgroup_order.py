@@ -1,7 +1,7 @@
-"""The order in which a step deals workgroups to the XCDs, beyond the size of
-the last-level cache (runs of workgroups with an incomplete last round) and
-with rows of odd length, against the CPU oracle, bit for bit: every cell is
-stepped exactly once."""
+"""The order in which a step deals workgroups to the XCDs -- slabs, as launched,
+runs of workgroups with an incomplete last round -- on both sides of the field
+sizes where it changes and with rows of odd length, against the CPU oracle, bit
+for bit: every cell is stepped exactly once."""
 import numpy as np
 import pytest
 
@@ -27,14 +27,37 @@ def test_container_odd_rows_beyond_cache(nx, orc, dim, st, sto, periodic):
     _same(g, o)
 
 
-def test_zouhe_beyond_cache(nx, orc):
-    X, Y, Z = dim = (131, 127, 109)
+@pytest.mark.parametrize("force", [(0.0, 0.0, 0.0), (1e-5, 0.0, 2e-6)])
+@pytest.mark.parametrize("dim,st,sto", [((80, 72, 64), "f32", 1), ((45, 53, 40), "f32", 1), ((56, 72, 45), "f32dev", 2),
+                                        ((83, 42, 43), "f64", 0), ((64, 50, 96), "f16dev", 3)])
+def test_container_at_the_sizes_between(nx, orc, dim, st, sto, force):
+    """Fields on both sides of the 48 MB up to which a step takes one slab per
+    XCD (binary32: the interior-bitmap kernel either way), with obstacles."""
+    X, Y, Z = dim
+    rng = np.random.default_rng(X)
+    cls = np.full((Z, Y, X), 2, np.uint32)
+    cls[:, :, [0, -1]] = cls[:, [0, -1]] = cls[[0, -1]] = 0
+    for _ in range(4):
+        z, y, x = (int(rng.integers(2, n - 8)) for n in (Z, Y, X))
+        cls[z:z + 5, y:y + 6, x:x + 7] = 0
+    cm = 0 if st == "f64" else 1
+    g, o = nx.DenseLattice(dim, st, "f64" if st == "f64" else "f32"), orc.DenseOracle(dim, sto, cm)
+    for lat in (g, o):
+        lat.set_classes(cls.reshape(-1))
+        lat.run(5, 1.6, force=force)
+    _same(g, o)
+
+
+@pytest.mark.parametrize("dim,st,cm,mb", [((131, 127, 109), "f32", 1, 256), ((181, 151, 155), "f64", 0, 1200)])
+def test_zouhe_large(nx, orc, dim, st, cm, mb):
+    X, Y, Z = dim
+    assert 38 * (8 if st == "f64" else 4) * X * Y * Z > mb << 20
     cls = np.full((Z, Y, X), 2, np.uint32)
     cls[:, [0, -1]] = cls[[0, -1]] = 0
     zh = np.zeros(cls.shape, np.uint32)
     zh[:, :, 0], zh[:, :, -1] = 1, 2
     zh[cls != 2] = 0
-    g, o = nx.DenseLattice(dim, "f32", "f32"), orc.DenseOracle(dim, 1, 1)
+    g, o = nx.DenseLattice(dim, st, st), orc.DenseOracle(dim, cm, cm)
     for lat in (g, o):
         lat.set_classes(cls.reshape(-1), zouhe=zh.reshape(-1))
         lat.run_zouhe(3, 1.4, [1.002, 0.998, 0, 0, 0, 0])
