@@ -207,7 +207,9 @@ __global__ void __launch_bounds__(kBV)
            const uint32_t* __restrict__ flags, BGeom g, Par p, int remap)
 {
     using T = typename Stor<S>::T;
-    const uint32_t b = remap ? xcd_order<4, 2 * kBStride * sizeof(T)>(blockIdx.x, gridDim.x) : blockIdx.x;
+    const uint32_t b = !remap ? blockIdx.x
+                       : gridDim.x > (256u << 20) / (uint32_t)(2 * kBStride * sizeof(T)) ? xcd_runs<4>(blockIdx.x, gridDim.x)
+                                                                                       : xcd_remap(blockIdx.x, gridDim.x);
     const uint32_t v = threadIdx.x;
     const int x = (int)(v & 7u), y = (int)((v >> 3) & 7u), z = (int)(v >> 6);
     const uint64_t own = (uint64_t)b * kBStride + v;

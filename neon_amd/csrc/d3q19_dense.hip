@@ -6,7 +6,7 @@
 // population load and store of a wavefront is one contiguous 64-cell run;
 // the +-1 x shifts of the pull read a neighbouring cache line that the
 // adjacent wavefront of the same workgroup fetches anyway.  Workgroups reach
-// the XCDs in runs or slabs (L2 keeps the row-boundary lines).  Each population
+// the XCDs in slabs or runs (L2 keeps the row-boundary lines).  Each population
 // is read once and written once per step: 2*19*sizeof(storage) bytes per cell
 // update.
 #include <cmath>
@@ -19,14 +19,29 @@ namespace nx {
 namespace dense {
 namespace {
 
-// Beyond the last-level cache workgroups reach the XCDs in runs of 16 (512 x
-// 128 x 128 duct, binary32 / binary64: 232 / 463 us; one contiguous slab per
-// XCD 241 / 509, one by one 237 / 470; 301 x 77 x 101 96 / 172 against 101 / 186
-// and 99 / 172; the cavity step of 200^3 binary16 152 -> 127).
-template <int S>
+// Order of the workgroups over the XCDs: one contiguous slab per XCD, except
+// for large fields, whose eight far slabs of 38 population streams each cost
+// more DRAM pages than their locality gives.  Measured (MI355X, slabs against
+// the order taken; both fields):
+//   plain step, 2-byte storage beyond the 256 MB last-level cache, runs of 16:
+//     256 x 200 x 100, 371 MB, 89 -> 76 us; 200^3 152 -> 127; 255^3 501 -> 497
+//   plain step, 4- and 8-byte storage beyond 700 MB, as launched: 256 x 200 x 100
+//     binary32, 742 MB, 181 -> 165; 255^3 807 -> 792; 200^3 binary64 514 -> 486;
+//     below that it wins and loses (131 x 127 x 109, 263 MB, 77 -> 85; 124 x 116 x
+//     145 binary64, 605 MB, 126 -> 138)
+//   Zou-He step beyond 1200 MB, runs of 16: 512 x 128 x 128 binary32 238 -> 235,
+//     binary64 510 -> 464, 350 x 110 x 128 binary64 298 -> 277; below that it wins
+//     and loses (286 x 64 x 116 binary64, 616 MB, 118 -> 127; 301 x 77 x 101 binary64,
+//     679 MB, 188 -> 172; 512 x 64 x 120 binary64, 1140 MB, 230 -> 233)
+template <int S, bool ZOUHE>
 __device__ __forceinline__ uint32_t order()
 {
-    return xcd_order<16, 2 * Q * kWG * sizeof(typename Stor<S>::T)>(blockIdx.x, gridDim.x);
+    constexpr uint32_t kBytes = 2 * Q * kWG * sizeof(typename Stor<S>::T);  // both fields, per workgroup
+    constexpr uint32_t kMB = ZOUHE ? 1200 : sizeof(typename Stor<S>::T) == 2 ? 256 : 700;
+    const uint32_t b = blockIdx.x, n = gridDim.x;
+    if (n <= (kMB << 20) / kBytes) return xcd_remap(b, n);
+    if constexpr (ZOUHE || sizeof(typename Stor<S>::T) == 2) return xcd_runs<16>(b, n);
+    return b;
 }
 
 // Generic step (any boundary mode, including periodic wrap).
@@ -36,7 +51,7 @@ __global__ void __launch_bounds__(kWG)
            const uint32_t* __restrict__ flags, DGeom g, Par p)
 {
     using R = typename Real<S, CM>::R;
-    const uint32_t i = order<S>() * kWG + threadIdx.x;
+    const uint32_t i = order<S, false>() * kWG + threadIdx.x;
     if (i >= g.n) return;
     const uint32_t fl = __builtin_nontemporal_load(&flags[i]);
     if (cls_of(fl) != NX_CELL_BULK) return;
@@ -63,7 +78,7 @@ __global__ void __launch_bounds__(kWG)
               const uint32_t* __restrict__ flags, DGeom g, Par p, ZhValues zh)
 {
     using R = typename Real<S, CM>::R;
-    const uint32_t i = order<S>() * kWG + threadIdx.x;
+    const uint32_t i = order<S, true>() * kWG + threadIdx.x;
     if (i >= g.n) return;
     const uint32_t fl = __builtin_nontemporal_load(&flags[i]);
     if (cls_of(fl) != NX_CELL_BULK) return;

@@ -469,17 +469,6 @@ __device__ __forceinline__ uint32_t xcd_runs(uint32_t b, uint32_t n)
     return s + S > n ? b : s + (r & 7u) * C + (r >> 3);
 }
 
-// The order by the size of both fields, BYTES of them per workgroup: beyond the
-// 256 MB last-level cache eight far slabs of 38 population streams each cost
-// more DRAM pages than their locality gives, so runs; within it slabs (Zou-He
-// duct binary32, 128 x 64 x 64: slabs 19.8 us, runs 20.8; 301 x 77 x 101: 102.7
-// and 96.6).
-template <uint32_t C, uint32_t BYTES>
-__device__ __forceinline__ uint32_t xcd_order(uint32_t b, uint32_t n)
-{
-    return n > (256u << 20) / BYTES ? xcd_runs<C>(b, n) : xcd_remap(b, n);
-}
-
 // ---- wave64 reductions with DPP ---------------------------------------------
 template <int CTRL, int ROW_MASK = 0xF>
 __device__ __forceinline__ double dpp_f64(double v)
