@@ -700,8 +700,9 @@ struct nx_mgrid_s {
     nx::mres::Level L[nx::mres::kMaxDepth];
     nx::mres::Store store[nx::mres::kMaxDepth];
     bool ready = false;
+    int device = 0;  // the grid's memory
     // read-back: worker w's pinned and device chunk and its stream, made at the
-    // first read-back and given back with the grid
+    // first large read-back and given back with the grid
     std::mutex read_mu;
     struct Reader {
         void* host = nullptr;
@@ -988,7 +989,10 @@ extern "C" int nx_mgrid_create_levels(const int32_t dim[3], int32_t depth, const
         return set_error(NX_ERR_UNSUPPORTED, "nx_mgrid_create: storage NX_F64 or NX_F32 (the reference's types)");
     if (lattice != NX_MGRID_BGK19 && lattice != NX_MGRID_KBC27)
         return set_error(NX_ERR_INVALID, "nx_mgrid_create_levels: lattice NX_MGRID_BGK19 or NX_MGRID_KBC27");
+    int device = 0;
+    NX_CHECK_HIP(hipGetDevice(&device));
     auto* g = new nx_mgrid_s;
+    g->device = device;
     g->storage = storage;
     g->lattice = lattice;
     g->lat = lattice == NX_MGRID_KBC27 ? host_lat_of<L27>() : host_lat_of<L19>();
@@ -1358,14 +1362,24 @@ namespace {
 // active voxels copied to the caller's array (the others keep what they hold
 // there).  128^3, 27 populations, float: one host copy per voxel took 155 ms,
 // this about 6 ms with 8 workers (bound by the page faults of a fresh array).
-constexpr size_t kReadBytes = 4u << 20;
+// Levels up to kPlainBytes, and any level where the chunks' memory cannot be
+// had, take the host copies: the first chunked read of a grid pays 0.2 to 0.3 ms
+// for that memory and a stream (17 x 13 x 9, 19 populations, float: 312 us, with
+// host copies 146; 24^3, 1 MB: 313 and 522).
+constexpr size_t kReadBytes = 4u << 20, kPlainBytes = 256u << 10;
+
+bool make_reader(nx_mgrid_s::Reader& r)
+{
+    const bool ok = (r.st || hipStreamCreateWithFlags(&r.st, hipStreamNonBlocking) == hipSuccess) &&
+                    (r.dev || hipMalloc(&r.dev, kReadBytes) == hipSuccess) &&
+                    (r.host || hipHostMalloc(&r.host, kReadBytes, hipHostMallocDefault) == hipSuccess);
+    if (!ok) (void)hipGetLastError();
+    return ok;
+}
 
 template <typename T>
 int read_chunk(const nx_mgrid_s& g, const Level& lv, int which, size_t e0, size_t e1, nx_mgrid_s::Reader& r, void* dense)
 {
-    if (!r.st) NX_CHECK_HIP(hipStreamCreateWithFlags(&r.st, hipStreamNonBlocking));
-    if (!r.dev) NX_CHECK_HIP(hipMalloc(&r.dev, kReadBytes));
-    if (!r.host) NX_CHECK_HIP(hipHostMalloc(&r.host, kReadBytes, hipHostMallocDefault));
     const uint32_t n = (uint32_t)(e1 - e0);
     hipLaunchKernelGGL(k_mr_dense<T>, dim3((n + 255) / 256), dim3(256), 0, r.st, (const T*)(which ? lv.fout : lv.fin),
                        lv.d_state, lv.d_table, lv.dim[0], lv.dim[1], (uint64_t)lv.nvox(), lv.nb[0], lv.nb[1], lv.nq,
@@ -1386,6 +1400,61 @@ int read_chunk(const nx_mgrid_s& g, const Level& lv, int which, size_t e0, size_
     return NX_OK;
 }
 
+int read_plain(const Level& lv, int which, size_t es, void* dense)
+{
+    std::vector<uint8_t> buf((size_t)lv.nq * kBV * lv.n_blocks * es);
+    if (!buf.empty()) NX_CHECK_HIP(hipMemcpy(buf.data(), which ? lv.fout : lv.fin, buf.size(), hipMemcpyDeviceToHost));
+    for (int z = 0; z < lv.dim[2]; z++)
+        for (int y = 0; y < lv.dim[1]; y++)
+            for (int x = 0; x < lv.dim[0]; x++) {
+                const int64_t s = lv.slot(x, y, z);
+                if (s < 0) continue;
+                for (int q = 0; q < lv.nq; q++)
+                    std::memcpy((uint8_t*)dense + ((size_t)q * lv.nvox() + lv.lin(x, y, z)) * es, buf.data() + lv.elem(s, q) * es,
+                                es);
+            }
+    return NX_OK;
+}
+
+int read_chunks(nx_mgrid_s& g, const Level& lv, int which, size_t total, size_t es, void* dense)
+{
+    const size_t chunk = kReadBytes / es, chunks = (total + chunk - 1) / chunk;
+    std::atomic<size_t> next{0};
+    std::atomic<int> code{NX_OK};
+    std::mutex err_mu;
+    std::string err;
+    auto work = [&](size_t w) {
+        int e = NX_OK;
+        try {
+            // (a worker that cannot have its chunk leaves the work to the others)
+            if (w > 0 && (hipSetDevice(g.device) != hipSuccess || !make_reader(g.reader[w]))) return;
+            for (size_t c; e == NX_OK && code == NX_OK && (c = next++) < chunks;) {
+                const size_t e0 = c * chunk, e1 = std::min(total, e0 + chunk);
+                e = es == 8 ? read_chunk<double>(g, lv, which, e0, e1, g.reader[w], dense)
+                            : read_chunk<float>(g, lv, which, e0, e1, g.reader[w], dense);
+            }
+            if (e != NX_OK) {
+                std::lock_guard<std::mutex> el(err_mu);
+                if (code == NX_OK) err = nx_last_error();  // (per thread)
+                code = e;
+            }
+        } catch (...) {
+            code = NX_ERR_HIP;  // no memory for a message
+        }
+    };
+    // one worker per 2 chunks, the calling thread among them
+    const size_t workers = std::min<size_t>(8, (chunks + 1) / 2);
+    std::vector<std::thread> th;
+    try {
+        for (size_t w = 1; w < workers; w++) th.emplace_back(work, w);
+    } catch (...) {
+        // fewer threads than wished for: the others take the chunks
+    }
+    work(0);
+    for (auto& x : th) x.join();
+    return code == NX_OK ? NX_OK : set_error(code, err);
+}
+
 }  // namespace
 
 extern "C" int nx_mgrid_fields(nx_mgrid g, int32_t level, int32_t which, void* dense)
@@ -1397,36 +1466,17 @@ extern "C" int nx_mgrid_fields(nx_mgrid g, int32_t level, int32_t which, void* d
     const Level& lv = g->L[level];
     const size_t total = lv.nvox() * (size_t)lv.nq, es = g->storage == NX_F64 ? 8 : 4;
     if (lv.runs.empty()) return NX_OK;
+    if (total * es <= kPlainBytes) return read_plain(lv, which, es, dense);
     std::lock_guard<std::mutex> lk(g->read_mu);
     int dev = 0;
     NX_CHECK_HIP(hipGetDevice(&dev));
-    const size_t chunk = kReadBytes / es, chunks = (total + chunk - 1) / chunk;
-    std::atomic<size_t> next{0};
-    std::atomic<int> code{NX_OK};
-    std::mutex err_mu;
-    std::string err;
-    auto work = [&](nx_mgrid_s::Reader& r) {
-        int e = hipSetDevice(dev) == hipSuccess ? NX_OK : set_error(NX_ERR_HIP, "nx_mgrid_fields: hipSetDevice");
-        for (size_t c; e == NX_OK && code == NX_OK && (c = next++) < chunks;)
-            e = g->storage == NX_F64 ? read_chunk<double>(*g, lv, which, c * chunk, std::min(total, (c + 1) * chunk), r, dense)
-                                     : read_chunk<float>(*g, lv, which, c * chunk, std::min(total, (c + 1) * chunk), r, dense);
-        if (e != NX_OK) {
-            std::lock_guard<std::mutex> el(err_mu);
-            if (code == NX_OK) err = nx_last_error();  // (per thread)
-            code = e;
-        }
-    };
-    // one worker per 2 chunks, the calling thread among them
-    const size_t workers = std::min<size_t>(8, (chunks + 1) / 2);
-    std::vector<std::thread> th;
-    try {
-        for (size_t w = 1; w < workers; w++) th.emplace_back(work, std::ref(g->reader[w]));
-    } catch (...) {
-        // fewer threads than wished for: the others take the chunks
+    if (dev != g->device) {
+        NX_CHECK_HIP(hipSetDevice(g->device));
+        NX_CHECK_HIP(hipDeviceSynchronize());
     }
-    work(g->reader[0]);
-    for (auto& x : th) x.join();
-    return code == NX_OK ? NX_OK : set_error(code, err);
+    const int e = make_reader(g->reader[0]) ? read_chunks(*g, lv, which, total, es, dense) : read_plain(lv, which, es, dense);
+    if (dev != g->device) NX_CHECK_HIP(hipSetDevice(dev));
+    return e;
 }
 
 extern "C" int nx_mgrid_destroy(nx_mgrid g)

@@ -1,6 +1,7 @@
 """Read-back of a refined level (nx_mgrid_fields): only active voxels of the
 caller's array are written, also where a level has partial blocks, inactive
-interiors and more values than one read-back chunk."""
+interiors and more values than one read-back chunk, or so few that it is copied
+without the chunks."""
 import ctypes as C
 
 import numpy as np
@@ -10,7 +11,8 @@ pytestmark = pytest.mark.gpu
 
 
 @pytest.mark.parametrize("dim,lattice,storage", [((40, 36, 28), "bgk19", "f32"), ((64, 48, 72), "kbc27", "f64"),
-                                                 ((17, 13, 9), "bgk19", "f64")])
+                                                 ((17, 13, 9), "bgk19", "f64"), ((17, 13, 9), "bgk19", "f32"),
+                                                 ((24, 24, 24), "kbc27", "f32")])
 def test_inactive_voxels_keep_the_callers_values(nx, dim, lattice, storage):
     from neon_amd import mgrid as mg
     g = mg.MGrid(dim, list(mg.cavity_lambdas(dim, (0.0, -0.4, -1.0))), storage, lattice=lattice)
