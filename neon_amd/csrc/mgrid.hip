@@ -631,7 +631,8 @@ struct Level {
     void* fin = nullptr;
     void* fout = nullptr;
     bool keep = true;      // the level has links in state "none"
-    bool separate = false; // an explosion link reads a refined voxel: the store needs its own launch
+    bool separate = false; // an explosion link reads a refined voxel or a store adds to a leaf: the store
+                           // needs its own launch
     int nq = 19;       // populations per voxel
     // active voxels as runs (first, one past the last) of the dense order
     std::vector<std::pair<size_t, size_t>> runs;
@@ -1141,6 +1142,9 @@ int setup_cells(nx_mgrid g, const uint8_t* const* cls, const double uw[3])
                         if (cs < 0) continue;
                         cnt[c.elem(cs, q)] += 1.f;
                         if (!leaf || !f.active(x + sx, y + sy, z + sz)) continue;
+                        // a target that is a leaf: the streams of both levels read it
+                        if (!(c.st[c.lin(px + sx, py + sy, pz + sz)] & kRefined))
+                            g->L[l].separate = g->L[l + 1].separate = true;
                         tl.emplace_back(c.elem(cs, q), f.elem(f.slot(x, y, z), q));
                     }
                 }
