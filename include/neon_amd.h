@@ -329,6 +329,11 @@ int nx_d3q19_set_block_remap(int on);
  * 0 -- one voxel per lane.  Same results bit for bit.  No counterpart in
  * the reference. */
 int nx_d3q19_set_block_pairs(int on);
+/* Byte offsets of nx_d3q19_step_block (2-byte storage) and of the refinement
+ * path's stream: 0 -- 32 bits where the populations of the field or level fit
+ * 4 GiB (the default); 1 -- 64 bits everywhere, as larger ones take.  Same
+ * results bit for bit; for comparisons.  No counterpart in the reference. */
+int nx_d3q19_set_wide_offsets(int on);
 /* The same step with the block neighbourhood staged in LDS (the reference
  * reads neighbour blocks through bPartition::getNghData,
  * bPartition_imp.h:218-309): one workgroup per tile

@@ -122,4 +122,7 @@ __device__ __forceinline__ void for_q(std::integer_sequence<int, qs...>, F&& f)
 }
 using AllQ = std::make_integer_sequence<int, Q>;
 
+// 64-bit offsets asked for everywhere (nx_d3q19_set_wide_offsets)
+bool wide_offsets();
+
 }  // namespace nx

@@ -863,6 +863,8 @@ using IC = std::integral_constant<int, V>;
 int g_block_remap = 1;
 // 1: 2-byte storage steps two voxels per lane (nx_d3q19_set_block_pairs)
 int g_block_pairs = 0;
+// 1: 64-bit offsets everywhere (nx_d3q19_set_wide_offsets)
+int g_wide_offsets = 0;
 
 template <typename F>
 int by_type(const nx_block_desc* d, F&& f)
@@ -881,6 +883,9 @@ int by_type(const nx_block_desc* d, F&& f)
 }
 
 }  // namespace
+
+bool wide_offsets() { return g_wide_offsets != 0; }
+
 }  // namespace nx
 
 using namespace nx;
@@ -973,7 +978,7 @@ extern "C" int nx_d3q19_step_block(const nx_block_desc* d, const void* fin, void
             // 4 GiB: that step is bound by its instructions (320^3 porous, 597
             // -> 540 us); the wider ones, bound by HBM, ran 1-2% slower so
             if constexpr (sizeof(T) == 2) {
-                if ((uint64_t)g.n_blocks * kBStride * sizeof(T) < (1ull << 32)) {
+                if (!g_wide_offsets && (uint64_t)g.n_blocks * kBStride * sizeof(T) < (1ull << 32)) {
                     if (force) go(std::true_type{}, std::true_type{});
                     else go(std::false_type{}, std::true_type{});
                     return;
@@ -1163,5 +1168,11 @@ extern "C" int nx_d3q19_set_block_remap(int on)
 extern "C" int nx_d3q19_set_block_pairs(int on)
 {
     g_block_pairs = on ? 1 : 0;
+    return NX_OK;
+}
+
+extern "C" int nx_d3q19_set_wide_offsets(int on)
+{
+    g_wide_offsets = on ? 1 : 0;
     return NX_OK;
 }

@@ -1284,7 +1284,7 @@ struct Stepper {
                                COLLIDE ? relax(l) : Relax{0.0, 0.0, 0.0}, a);
         };
         // byte offsets in 32 bits where the level's populations allow it
-        if ((uint64_t)lv.slots() * LT::Q * sizeof(T) < (1ull << 32)) go(uint32_t{});
+        if (!wide_offsets() && (uint64_t)lv.slots() * LT::Q * sizeof(T) < (1ull << 32)) go(uint32_t{});
         else go(uint64_t{});
     }
 
