@@ -19,6 +19,9 @@ with the textbook forced step of tests/textbook.py (Guo, Zheng & Shi 2002,
 written from the formulas in float64) over 10 steps in a periodic box, and
 with the closed-form momentum gain rho*g per step, in both binary32 and
 binary16 deviation storage.
+
+or_residual_dense and or_mass_block: numpy sums over the oracle's moments and
+decoded populations.
 """
 import numpy as np
 import pytest
@@ -151,3 +154,66 @@ def test_forced_deviation_matches_textbook_and_momentum(orc, storage, tol, mom_r
     want = 10 * f0.sum() * np.array(g)
     assert np.abs(gain - want).max() < mom_rtol * np.abs(want).max(), (gain, want)
     assert abs(got.sum() - f0.sum()) < 50 * tol * N ** 3
+
+
+# ---- the reductions that decide convergence and conservation -------------------
+
+
+@pytest.mark.parametrize("storage,compute", [(0, 0), (1, 1), (2, 1), (3, 1)])
+def test_residual_from_moments(orc, storage, compute):
+    """or_residual_dense: the sums and the kept velocity from two snapshots of
+    the oracle's moments, by numpy; obstacles, so that not every cell counts."""
+    dim = (13, 11, 9)
+    X, Y, Z = dim
+    cls = np.full((Z, Y, X), 2, np.uint32)
+    cls[:, :, [0, -1]] = cls[:, [0, -1]] = cls[[0, -1]] = 0
+    cls[:, -1] = 1
+    cls[3:6, 4:7, 5:9] = 0
+    bulk = (cls == 2).reshape(-1)
+    o = orc.DenseOracle(dim, storage, compute)
+    o.set_classes(cls.reshape(-1), ulb=0.05)
+    o.run(7, 1.5)
+    kept = np.full(3 * o.n, 7.0, np.float32)              # no bulk cell ever read holds it
+    kept.reshape(3, -1)[:, bulk] = 0.0
+    first = o.residual(kept)
+    u1 = o.moments()[1].reshape(3, -1).astype(np.float32)
+    assert first[0] == first[1] > 0                       # from u_prev = 0
+    assert np.array_equal(kept.reshape(3, -1)[:, bulk], u1[:, bulk]) and np.all(kept.reshape(3, -1)[:, ~bulk] == 7.0)
+    again = o.residual(kept)
+    assert again[0] == 0.0 and again[1] == first[1]       # an unchanged field
+    o.run(4, 1.5)
+    num, den = o.residual(kept)
+    u2 = o.moments()[1].reshape(3, -1).astype(np.float32)
+    a, b = (v[:, bulk].astype(np.float64) for v in (u1, u2))
+    assert np.isclose(num, np.square(b - a).sum(), rtol=1e-13, atol=0) and num > 0
+    assert np.isclose(den, np.square(b).sum(), rtol=1e-13, atol=0) and abs(den / first[1] - 1) > 1e-3
+    assert np.array_equal(kept.reshape(3, -1)[:, bulk], u2[:, bulk])
+
+
+@pytest.mark.parametrize("storage,compute", [(0, 0), (1, 1), (2, 1), (3, 1)])
+def test_block_mass_from_populations(orc, storage, compute):
+    """or_mass_block: the decoded populations of the active bulk slots, summed by
+    numpy; inactive slots and wall cells, filled with fives, stay out."""
+    dim = (20, 17, 12)
+    act = np.ones(dim[::-1], np.uint8)
+    act[:8, :8, :8] = 0
+    act[9:12, 10:14, 9:15] = 0
+    o = orc.BlockOracle(dim, act.reshape(-1), storage, compute)
+    keep = o.active_slots()
+    cls = np.where(keep, 2, 3).astype(np.uint32)
+    x, y, z = o.slot_coords().T
+    cls[keep & (y == dim[1] - 1)] = 1
+    o.set_classes(cls, ulb=0.05)
+    o.run(5, 1.4)
+    bulk = cls == 2
+    raw = o.fin.view({0: np.float64, 1: np.float32, 2: np.float32, 3: np.float16}[storage]).reshape(-1, 19, 512)
+    raw.transpose(1, 0, 2)[:, ~bulk.reshape(-1, 512)] = 5.0
+    f = raw.astype(np.float64).transpose(1, 0, 2).reshape(19, -1)
+    c = np.array([[-1, 0, 0], [0, -1, 0], [0, 0, -1], [-1, -1, 0], [-1, 1, 0], [-1, 0, -1], [-1, 0, 1], [0, -1, -1], [0, -1, 1],
+                  [0, 0, 0], [1, 0, 0], [0, 1, 0], [0, 0, 1], [1, 1, 0], [1, -1, 0], [1, 0, 1], [1, 0, -1], [0, 1, 1], [0, 1, -1]])
+    w = np.where(np.abs(c).sum(1) == 0, 1 / 3, np.where(np.abs(c).sum(1) == 1, 1 / 18, 1 / 36))
+    if storage >= 2:
+        f = f + w.astype(np.float32).astype(np.float64)[:, None]  # deviations from binary32 w
+    total = f[:, bulk].sum()
+    assert np.isclose(o.mass(), total, rtol=1e-12, atol=0) and abs(total / bulk.sum() - 1) < 0.2
+    assert not np.isclose(total, f[:, keep].sum(), rtol=1e-9)
