@@ -990,10 +990,7 @@ extern "C" int nx_mgrid_create_levels(const int32_t dim[3], int32_t depth, const
         return set_error(NX_ERR_UNSUPPORTED, "nx_mgrid_create: storage NX_F64 or NX_F32 (the reference's types)");
     if (lattice != NX_MGRID_BGK19 && lattice != NX_MGRID_KBC27)
         return set_error(NX_ERR_INVALID, "nx_mgrid_create_levels: lattice NX_MGRID_BGK19 or NX_MGRID_KBC27");
-    int device = 0;
-    NX_CHECK_HIP(hipGetDevice(&device));
     auto* g = new nx_mgrid_s;
-    g->device = device;
     g->storage = storage;
     g->lattice = lattice;
     g->lat = lattice == NX_MGRID_KBC27 ? host_lat_of<L27>() : host_lat_of<L19>();
@@ -1079,6 +1076,7 @@ namespace {
 
 int setup_cells(nx_mgrid g, const uint8_t* const* cls, const double uw[3])
 {
+    NX_CHECK_HIP(hipGetDevice(&g->device));
     const int D = g->depth;
     const size_t es = g->storage == NX_F64 ? 8 : 4;
     // populations
