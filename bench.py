@@ -270,7 +270,7 @@ def copy_calibration(nx):
 def shifted_copy_calibration(nx, N=256, reps=20):
     """The dense step's access pattern without arithmetic (nx_shifted_copy:
     19 planes read at the upstream cells, 19 written) on an N^3 grid for 2-,
-    4- and 8-byte elements: the ceiling of the pull-streaming step on SoA
+    4- and 8-byte elements: a yardstick for the pull-streaming step on SoA
     planes, beside the plain 1 GiB copy."""
     import ctypes as C
     from neon_amd import abi
@@ -700,7 +700,7 @@ def main():
                          "reference for scaling FETCH_SIZE / WRITE_SIZE counters")
     ap.add_argument("--shifted", action="store_true",
                     help="with --copy-calibration: time the step's 19-plane shifted copy (no arithmetic) "
-                         "at 256^3 for 2/4/8-byte elements, the ceiling of the pull-streaming step")
+                         "at 256^3 for 2/4/8-byte elements, a yardstick for the pull-streaming step")
     a = ap.parse_args()
     if a.gpus != 1:
         print(f"bench.py: this benchmark runs on one GPU; --gpus {a.gpus} is not supported "
