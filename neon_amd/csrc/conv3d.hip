@@ -11,8 +11,9 @@
 //   bwd-data     the forward on the flipped, transposed weights
 //   bwd-weight   M = cout, N = cin, K = voxels (split over workgroups, FP32
 //                partials, fixed-order reduction): all 27 taps at once on rows
-//                of >= 32 voxels (k_bwd_wr, k_bwd_w27), else one tap per
-//                workgroup (k_bwd_w)
+//                of >= 32 voxels (k_bwd_wr, k_bwd_w27), the 9 of a z shift on
+//                rows of 4 to 16 (k_bwd_wc), else one tap per workgroup
+//                (k_bwd_w)
 // MFMA 16x16x32 bf16 operand layout: lane l holds row (A) / column (B) l%16
 // and the 8 K values of group l/16; D register r of lane l is row 4*(l/16)+r,
 // column l%16.
@@ -747,7 +748,8 @@ __global__ void __launch_bounds__(256)
 }
 
 // Weight gradient of one tap for a (16*NM) x (16*NN) block of (co, ci): the
-// 1^3 kernel, and 3^3 on rows of 1 or 2 voxels and planes of less than 32.
+// 1^3 kernel, and 3^3 on rows of 1 or 2 voxels, planes of less than 32 and
+// the least work (plan_w).
 // grid.x = T * splits (tap fastest), grid.y = channel blocks.  Each wave
 // takes every 4th 32-voxel chunk of its split and writes its own partial:
 // part[(split*4 + wave)][tap][co][ci].
@@ -1132,11 +1134,12 @@ __global__ void __launch_bounds__(64)
 // ci), rows of W = 4, 8 or 16 voxels, planes of at least 32.  Partial
 // 4 s + v of k_bwd_w is the sum over every 4th chunk (32 voxels: 32 / W rows of
 // a plane) from chunk v of split s; one wavefront adds the partials v, v + 4,
-// .. of a slice in registers (the first of k_reduce_w's sums, in its order):
-// written out one by one the partials' way through memory takes most of the
-// time.  Per chunk it stages the rows of x that the taps reach and the chunk of
-// dy in LDS, a chunk ahead, two more in registers on their way; fragments as in
-// k_bwd_wr.  part[4 slice + v][tap][co][ci].
+// .. of a slice of S in registers (the first of k_reduce_w's sums, in its order):
+// written out one by one the partials' way through memory can take most of the
+// time.  With S = 4 a wavefront has one partial (plan_w).  Per chunk it stages
+// the rows of x that the taps reach and the chunk of dy in LDS, a chunk ahead,
+// two more in registers on their way; fragments as in k_bwd_wr.
+// part[4 slice + v][tap][co][ci].
 // Measured (MI355X, whole call): 16^3 x 8, 64 -> 64 55 us; 16^3 x 16, 256 -> 128
 // 353 us; 8^3 x 8, 64 -> 64 26 us (k_bwd_w: 88, 600 and 43 us).
 template <int W>
@@ -1658,7 +1661,7 @@ struct WPlan {
     bool all_taps;
     uint32_t chunks, per, splits, part_splits;
     uint32_t partials, slices, S;   // partials per output element, added slice by slice (S each)
-    bool classes;                   // k_bwd_wc adds every 4th partial of a slice itself
+    bool staged, classes;           // k_bwd_wc; it adds every 4th partial of a slice itself
 };
 
 WPlan plan_w(const Shape& s)
@@ -1684,7 +1687,16 @@ WPlan plan_w(const Shape& s)
     const uint32_t G = std::max(1u, std::min(64u, p.partials / 32));
     p.S = (p.partials + G - 1) / G;
     p.slices = (p.partials + p.S - 1) / p.S;
-    p.classes = s.ks == 3 && s.w >= 4 && s.w < 32 && s.w * s.h >= 32;
+    // k_bwd_wc, except where there is little to do (chunks x channel blocks: its
+    // start costs 3 us; 16 -> 16 at 8^3 x 3 16.7 against 12.5 us, 64 -> 64 at 4 x 8 x 4
+    // 13.6 and 11.9, from 256 on even or faster).  A wavefront per class of partials
+    // has chunks / (4 slices) chunks to take one after another, one per partial
+    // writes nm nn x 8.4 MB; even at 8 chunks per nm nn (16 -> 16 at 16^3 x 3, 10
+    // chunks: 18.5 and 16.5 us; 32 -> 32 x 8, 28: 31.3 and 30.0; 128 -> 128 x 8, 128:
+    // 109.8 and 110.0; 112 -> 16 x 8, 256: 139 and 28; 64 -> 64 x 8, 28: 46 and 65).
+    p.staged = s.ks == 3 && s.w >= 4 && s.w < 32 && s.w * s.h >= 32 &&
+               (uint64_t)p.chunks * (uint32_t)(s.cout / 16) * (uint32_t)(s.cin / 16) > 256;
+    p.classes = p.staged && p.chunks <= 32u * p.slices * (uint32_t)(p.nm * p.nn);
     return p;
 }
 
@@ -1738,8 +1750,7 @@ size_t bwd_weight_ws(const Shape& s)
     const WPlan p = plan_w(s);
     const size_t nw = (size_t)p.T * s.cout * s.cin, cols = (size_t)kColBlocks * s.cout;
     if (p.all_taps) return (size_t)p.part_splits * (nw + s.cout) * sizeof(float);
-    const size_t parts = 4 * (p.classes ? std::max(1u, std::min(64u, p.part_splits / 8)) : p.part_splits);
-    return std::max(parts * nw, cols) * sizeof(float);
+    return std::max(4 * p.part_splits * nw, cols) * sizeof(float);
 }
 
 int bwd_weight(const Shape& s, const uint16_t* x, const uint16_t* dy, float* dw, float* db, void* ws,
@@ -1773,11 +1784,11 @@ int bwd_weight(const Shape& s, const uint16_t* x, const uint16_t* dy, float* dw,
             default: go27(std::integral_constant<int, 1>{}); break;
         }
         NX_CHECK_LAUNCH("k_bwd_w27");
-    } else if (p.classes) {
+    } else if (p.staged) {
         const uint32_t pairs = (uint32_t)((s.cout / 16) * (s.cin / 16));
         auto go = [&](auto W) {
-            hipLaunchKernelGGL((k_bwd_wc<decltype(W)::value>), dim3(12 * p.slices * pairs), dim3(64), 0, st, x, dy, part, g,
-                               s.cin, s.cout, p.per, p.partials, p.S, pairs);
+            hipLaunchKernelGGL((k_bwd_wc<decltype(W)::value>), dim3(12 * (p.classes ? p.slices : p.splits) * pairs), dim3(64),
+                               0, st, x, dy, part, g, s.cin, s.cout, p.per, p.partials, p.classes ? p.S : 4u, pairs);
         };
         switch (s.w) {
             case 16: go(std::integral_constant<int, 16>{}); break;

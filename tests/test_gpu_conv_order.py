@@ -25,6 +25,7 @@ SHAPES = [((5, 8, 64, 64), 16, 16, 3), ((3, 16, 32, 32), 64, 64, 3), ((2, 8, 16,
           ((8, 16, 8, 8), 64, 32, 3), ((2, 4, 4, 8), 176, 16, 3), ((3, 8, 4, 8), 16, 64, 3),
           ((8, 16, 8, 4), 48, 64, 3), ((2, 4, 4, 4), 256, 32, 3), ((2, 2, 16, 4), 64, 16, 3),
           ((3, 8, 8, 2), 48, 32, 3), ((2, 4, 4, 1), 16, 16, 3), ((3, 1, 1, 64), 32, 16, 3),
+          ((3, 16, 16, 16), 112, 16, 3), ((8, 8, 8, 8), 16, 112, 3), ((16, 8, 8, 4), 112, 16, 3),
           ((3, 16, 16, 16), 48, 16, 1), ((2, 8, 8, 8), 32, 80, 1), ((1, 1, 2, 4), 64, 64, 1)]
 NETS = [(32, (16, 32, 64), 3), (64, (16, 32), 2)]
 

@@ -19,9 +19,10 @@ SHAPES = [((1, 16, 16, 16), 80, 32), ((1, 32, 4, 16), 16, 48), ((1, 1, 1, 16), 3
 # Work of one workgroup: k_fwd_z16 3 planes of 8 (640 planes over 256 runs);
 # k_bwd_wr 7 chunks = 3.5 rows of 64 voxels (5,120 chunks, 768 splits) and 7
 # rows of 32 (1,280, 192 splits); k_bwd_wc the partials of a slice, each 3 of 11
-# chunks (768 chunks, 70 splits), on rows of 8 and 4 one of 4
+# chunks (768 chunks, 70 splits), on rows of 8 and 4 one of 4, and one partial
+# of 9 of 35 chunks (112 -> 16)
 RUNS = [((5, 8, 64, 64), 16, 16), ((5, 8, 32, 32), 64, 32), ((6, 16, 16, 16), 32, 64), ((8, 16, 8, 8), 64, 32),
-        ((8, 16, 8, 4), 48, 64)]
+        ((8, 16, 8, 4), 48, 64), ((3, 16, 16, 16), 112, 16)]
 
 
 def _bf(rng, shape, scale=1.0):
