@@ -1445,7 +1445,9 @@ __global__ void __launch_bounds__(256)
 // adds every rows-th voxel from the j-th, then the threads of a channel are
 // added in order.  The range goes through LDS, 16 bytes a lane and 16 voxels a
 // thread at a time, the next ones on their way: read 2 bytes a lane and one
-// voxel after another it was bound by the latency of its loads.
+// voxel after another it was bound by the latency of its loads.  Ranges of one
+// or two voxels a thread are read directly, without the barriers (8^3, 64
+// channels 2.8 us, through LDS 3.5; 12 voxels a thread 6.2 against 3.7).
 // Measured (MI355X, 64^3, batch 8, with the sum of the partials): 16 channels 22
 // us, 48 channels 56 us (before 73 and 240 us).
 __global__ void __launch_bounds__(256)
@@ -1468,20 +1470,26 @@ __global__ void __launch_bounds__(256)
         }
     };
     float s = 0.f;
-    fetch(v0);
-    for (uint32_t v = v0; v < v1; v += step) {
-        __syncthreads();                                      // the last turn's reads are done
-#pragma unroll
-        for (int k = 0; k < 2; k++)
-            if (threadIdx.x + 256u * k < pieces) *reinterpret_cast<uint4*>(tile + 8u * (threadIdx.x + 256u * k)) = q[k];
-        __syncthreads();
-        fetch(v + step);
+    if (per_block <= 2u * (uint32_t)rows) {
         if (j < rows)
+            for (uint32_t v = v0 + (uint32_t)j; v < v1; v += (uint32_t)rows)
+                s += __builtin_bit_cast(float, (uint32_t)dy[(size_t)v * C + c] << 16);
+    } else {
+        fetch(v0);
+        for (uint32_t v = v0; v < v1; v += step) {
+            __syncthreads();                                  // the last turn's reads are done
 #pragma unroll
-            for (int i = 0; i < 16; i++) {
-                const int at = j + i * rows;
-                if (v + (uint32_t)at < v1) s += __builtin_bit_cast(float, (uint32_t)tile[at * C + c] << 16);
-            }
+            for (int k = 0; k < 2; k++)
+                if (threadIdx.x + 256u * k < pieces) *reinterpret_cast<uint4*>(tile + 8u * (threadIdx.x + 256u * k)) = q[k];
+            __syncthreads();
+            fetch(v + step);
+            if (j < rows)
+#pragma unroll
+                for (int i = 0; i < 16; i++) {
+                    const int at = j + i * rows;
+                    if (v + (uint32_t)at < v1) s += __builtin_bit_cast(float, (uint32_t)tile[at * C + c] << 16);
+                }
+        }
     }
     lds[threadIdx.x] = s;
     __syncthreads();
